@@ -70,9 +70,21 @@ struct Ws32 {
 
 // ----------------------------------------------------------------------------------------------- phase 1
 //
-// One workgroup of 4 waves per item. LDS (byte offsets; D x 4-byte rows for the token rows, 256-byte rows for
-// the 64 x 64 matrices): the chunk's q, k (L2-normalised in place when asked) and v rows, A (then R), T, P and
-// the per-token factors.
+// One item (chunk x value head) at a time per workgroup of 16 waves, one workgroup per CU (148,736 bytes of LDS
+// at D = 128: the chunk's q, k (L2-normalised when asked) and v rows, A (then R), T, P and the per-token
+// factors); a workgroup walks the items item, item + grid, .. and loads the next item's rows into registers
+// while it computes. Bound by the fp32 matrix rate: 2,060 products of 32 cycles at D = 128 are 6.9 us an item on
+// a CU's four SIMDs, so the item is split to keep all four busy and the serial inverse out of the way:
+//   1  rows -> LDS (their norm on the way, 16 lanes a row), the per-token factors (wave 15)
+//   2  the 10 tiles of A (diagonal ones stored transposed) and 6 of P's
+//   3  waves 0-3 (one a SIMD) invert A's diagonal blocks in registers
+//   4  wave d < 4 the rest of block column d of T, its blocks passed on in registers; waves 4-7 P's last 4 tiles
+//   5  R (waves 0-3), Ub, Ub', Ob (NK waves, a value tile each) and W', K^T (the others)
+//   6  Q' (all waves)
+// and the item's stores (164 KB) and the next one's loads (98 KB) in different stretches of it. The 1,024 items of
+// T = 4096 at 16 heads take 83 us, of which 52 us are what their 268 MB take at the rate of a large copy; the 16
+// items of T = 256, 4 heads, D = 64, one a workgroup, 13.7 us. With four waves an item, no loads ahead and the
+// inverse's four levels behind each other: 111-114 and 18 us.
 template <int D>
 struct Lds32 {
   static constexpr int RB = D * 4;
@@ -82,321 +94,518 @@ struct Lds32 {
   static constexpr int BYTES = F + 1280;
 };
 
+constexpr int P32_WAVES = 16;
+
 // Lower-triangle tile t (0..9) of a 4 x 4 block grid -> (row block, column block), row-major order.
 __device__ __forceinline__ void tri_tile(int t, int& rb, int& cb) {
   rb = t < 1 ? 0 : (t < 3 ? 1 : (t < 6 ? 2 : 3));
   cb = t - rb * (rb + 1) / 2;
 }
 
-// 16 consecutive bytes of a q / k / v row as floats (4 fp32 or 8 bf16 elements).
-__device__ __forceinline__ void load_vec(const float* p, float* out) {
-  const f32x4 v = *reinterpret_cast<const f32x4*>(p);
-  out[0] = v[0];
-  out[1] = v[1];
-  out[2] = v[2];
-  out[3] = v[3];
-}
-__device__ __forceinline__ void load_vec(const bf16* p, float* out) {
-  const uint4 w = *reinterpret_cast<const uint4*>(p);
-  const uint32_t u[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    out[2 * j] = __uint_as_float(u[j] << 16);
-    out[2 * j + 1] = __uint_as_float(u[j] & 0xffff0000u);
+// Four consecutive elements of a q / k / v row as loaded through a buffer resource (zeros past its range), and
+// as floats.
+template <typename T>
+struct Row4;
+template <>
+struct Row4<float> {
+  f32x4 v;
+  __device__ __forceinline__ void load(Rsrc r, uint32_t off) {
+    v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
   }
-}
+  __device__ __forceinline__ f32x4 get() const { return v; }
+};
+template <>
+struct Row4<bf16> {
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  u32x2 v;
+  __device__ __forceinline__ void load(Rsrc r, uint32_t off) {
+    v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+  }
+  __device__ __forceinline__ f32x4 get() const {
+    return f32x4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
+                 __uint_as_float(v.y & 0xffff0000u)};
+  }
+};
 
-// acc += X[16 xr .., 16 xc ..] . Y[16 yr .., 16 yc ..] for 16 x 16 blocks of two 64 x 64 LDS matrices.
-__device__ __forceinline__ f32x4 blk_mm(const uint8_t* lb, int xm, int xr, int xc, int ym, int yr, int yc, f32x4 acc) {
-  const int l = threadIdx.x & 63, m = l & 15, g = l >> 4;
-  const f32x4 a = ld4(lb, xm + swz<256>(16 * xr + m, 16 * xc + 4 * g));
-#pragma unroll
-  for (int i = 0; i < 4; ++i) acc = mma(a[i], ld1(lb, ym + swz<256>(16 * yr + 4 * g + i, 16 * yc + m)), acc);
-  return acc;
-}
-// acc += X[16 xr .., 16 xc ..] . Y for a block Y held as a D tile.
-__device__ __forceinline__ f32x4 blk_mm_d(const uint8_t* lb, int xm, int xr, int xc, f32x4 y, f32x4 acc) {
-  const int l = threadIdx.x & 63, m = l & 15, g = l >> 4;
+// acc += X[16 xr .., 16 xc ..] . Y for a 16 x 16 block of a 64 x 64 LDS matrix X and a block Y held as a D tile.
+__device__ __forceinline__ f32x4 blk_mm_d(const uint8_t* lb, int m, int g, int xm, int xr, int xc, f32x4 y, f32x4 acc) {
   const f32x4 a = ld4(lb, xm + swz<256>(16 * xr + m, 16 * xc + 4 * g));
 #pragma unroll
   for (int i = 0; i < 4; ++i) acc = mma(a[i], y[i], acc);
   return acc;
 }
-// Stores a D tile as block (br, bc) of a 64 x 64 LDS matrix.
-__device__ __forceinline__ void blk_put(uint8_t* lb, int mat, int br, int bc, f32x4 d) {
-  const int l = threadIdx.x & 63, m = l & 15, g = l >> 4;
+// Stores a D tile as block (br, bc) of a 64 x 64 LDS matrix; blk_put_t stores its transpose (one 16-byte write).
+__device__ __forceinline__ void blk_put(uint8_t* lb, int m, int g, int mat, int br, int bc, f32x4 d) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) st1(lb, mat + swz<256>(16 * br + 4 * g + i, 16 * bc + m), d[i]);
 }
+__device__ __forceinline__ void blk_put_t(uint8_t* lb, int m, int g, int mat, int br, int bc, f32x4 d) {
+  st4(lb, mat + swz<256>(16 * br + m, 16 * bc + 4 * g), d);
+}
 
-__device__ __forceinline__ void bar() { __syncthreads(); }
+// Workgroup barrier over LDS traffic only: global loads and stores stay in flight across it.
+__device__ __forceinline__ void bar() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// A gate input as loaded through a buffer resource, and as a float.
+template <typename T>
+struct GateReg;
+template <>
+struct GateReg<float> {
+  float v;
+  __device__ __forceinline__ void load(Rsrc r, uint32_t off) {
+    v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+  }
+  __device__ __forceinline__ float get() const { return v; }
+};
+template <>
+struct GateReg<bf16> {
+  uint16_t v;
+  __device__ __forceinline__ void load(Rsrc r, uint32_t off) { v = __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0); }
+  __device__ __forceinline__ float get() const { return bf16_to_f32(v); }
+};
+
+// An item's rows (four elements of D / 64 column groups of row tid / 16 of each of q, k, v) and gate inputs.
+template <typename TIn, typename TG, int D>
+struct Rows32 {
+  Row4<TIn> q[D / 64], k[D / 64], v[D / 64];
+  GateReg<TG> g, beta;
+  // waits for the loads (an empty asm that takes their registers)
+  __device__ __forceinline__ void arrive() {
+#pragma unroll
+    for (int j = 0; j < D / 64; ++j) asm volatile("" : "+v"(q[j].v), "+v"(k[j].v), "+v"(v[j].v));
+    asm volatile("" : "+v"(g.v), "+v"(beta.v));
+  }
+};
+
+template <typename TIn, typename TG, int D>
+__device__ __forceinline__ void load_item(Rows32<TIn, TG, D>& x, int item, const TIn* q, const TIn* k, const TIn* v,
+                                          const TG* g, const TG* beta, const int32_t* cu, const int32_t* chunk_idx,
+                                          int n_seqs, int T, int Hk, int Hv, const RowStrides& rs) {
+  const int c = item / Hv, h = item % Hv, hk = h / (Hv / Hk);
+  const ChunkRange cr = chunk_range(c, cu, chunk_idx, T, n_seqs);
+  constexpr uint32_t E = sizeof(TIn);
+  const uint32_t r = threadIdx.x >> 4, c0 = (threadIdx.x & 15) * 4 * E;
+  auto rows = [&](const TIn* p, long ld, int col, Row4<TIn>* out) {
+    const Rsrc w = raw_rsrc(p + (size_t)cr.t0 * ld + col, (uint32_t)cr.len * (uint32_t)ld * E);
+#pragma unroll
+    for (int j = 0; j < D / 64; ++j) out[j].load(w, r * (uint32_t)ld * E + c0 + 64 * E * j);
+  };
+  rows(q, rs.q, hk * D, x.q);
+  rows(k, rs.k, hk * D, x.k);
+  rows(v, rs.v, h * D, x.v);
+  // the gate inputs of token `lane` (zeros past the chunk end)
+  const uint32_t gbytes = (uint32_t)cr.len * (uint32_t)rs.gb * (uint32_t)sizeof(TG);
+  const uint32_t goff = (threadIdx.x & 63) * (uint32_t)rs.gb * (uint32_t)sizeof(TG);
+  const size_t t = (size_t)cr.t0 * rs.gb + h;
+  x.g.load(raw_rsrc(g + t, gbytes), goff);
+  x.beta.load(raw_rsrc(beta + t, gbytes), goff);
+}
 
 template <typename TIn, typename TG, int D, bool GATE>
-__global__ __launch_bounds__(256) void chunk32_prep_kernel(
+__global__ __launch_bounds__(64 * P32_WAVES) void chunk32_prep_kernel(
     const TIn* __restrict__ q, const TIn* __restrict__ k, const TIn* __restrict__ v, const TG* __restrict__ g,
     const TG* __restrict__ beta, const float* __restrict__ A_log, const float* __restrict__ dt_bias,
-    const int32_t* __restrict__ cu, const int32_t* __restrict__ chunk_idx, int n_seqs, int T, int Hk, int Hv,
-    float scale, int qk_l2norm, const RowStrides rs, uint8_t* __restrict__ ws) {
+    const int32_t* __restrict__ cu, const int32_t* __restrict__ chunk_idx, int n_seqs, int n_items, int T, int Hk,
+    int Hv, float scale, int qk_l2norm, const RowStrides rs, uint8_t* __restrict__ ws) {
   using L = Lds32<D>;
   using WS = Ws32<D>;
-  constexpr int RB = L::RB, NK = WS::NK, NKW = NK / 4;
+  constexpr int RB = L::RB, NK = WS::NK;
   extern __shared__ f32x4 lds32[];
   uint8_t* lb = reinterpret_cast<uint8_t*>(lds32);
-  const int tid = threadIdx.x, wave = wave_id(), l = tid & 63, m = l & 15, gq = l >> 4;
-  const int item = blockIdx.x, c = item / Hv, h = item % Hv, hk = h / (Hv / Hk);
-  const ChunkRange cr = chunk_range(c, cu, chunk_idx, T, n_seqs);
-  uint8_t* out = ws + (size_t)item * WS::ITEM;
+  const f32x4 z4 = {0.f, 0.f, 0.f, 0.f};
+  Rows32<TIn, TG, D> R;
+  if ((int)blockIdx.x >= n_items) return;
+  load_item<TIn, TG, D>(R, blockIdx.x, q, k, v, g, beta, cu, chunk_idx, n_seqs, T, Hk, Hv, rs);
 
-  // ---- rows of q, k (key head hk) and v (value head h) into LDS as fp32; zeros past the chunk end
-  constexpr int VE = 16 / (int)sizeof(TIn), VPR = D / VE;
-  for (int e = tid; e < 64 * VPR; e += 256) {
-    const int r = e / VPR, c0 = (e % VPR) * VE;
-    float xq[VE], xk[VE], xv[VE];
-    if (r < cr.len) {
-      const size_t t = (size_t)(cr.t0 + r);
-      load_vec(q + t * rs.q + (size_t)hk * D + c0, xq);
-      load_vec(k + t * rs.k + (size_t)hk * D + c0, xk);
-      load_vec(v + t * rs.v + (size_t)h * D + c0, xv);
-    } else {
+  for (int item = blockIdx.x; item < n_items; item += gridDim.x) {
+    // the lane's and wave's indexes pass through an empty asm per item: the addresses derived from them are then
+    // formed inside the item instead of being hoisted out of the loop, where they would not fit the registers
+    int tid = threadIdx.x, wave = wave_id();
+    asm volatile("" : "+v"(tid));
+    asm volatile("" : "+s"(wave));
+    const int l = tid & 63, m = l & 15, gq = l >> 4;
+    const int c = item / Hv, h = item % Hv;
+    const int len = chunk_range(c, cu, chunk_idx, T, n_seqs).len;
+    uint8_t* out = ws + (size_t)item * WS::ITEM;
+
+    // ---- 1. rows of q, k (key head hk) and v (value head h) into LDS as fp32 (zeros past the chunk end), q and k
+    // L2-normalised when asked: x * rsqrt(sum x^2 + 1e-6)
+    {
+      const int r = tid >> 4, c0 = (tid & 15) * 4;
+      f32x4 xq[D / 64], xk[D / 64];
+      float sq = 0.f, sk = 0.f;
 #pragma unroll
-      for (int j = 0; j < VE; ++j) xq[j] = xk[j] = xv[j] = 0.f;
-    }
+      for (int j = 0; j < D / 64; ++j) {
+        xq[j] = R.q[j].get();
+        xk[j] = R.k[j].get();
 #pragma unroll
-    for (int j = 0; j < VE; j += 4) {
-      st4(lb, L::Q + swz<RB>(r, c0 + j), f32x4{xq[j], xq[j + 1], xq[j + 2], xq[j + 3]});
-      st4(lb, L::K + swz<RB>(r, c0 + j), f32x4{xk[j], xk[j + 1], xk[j + 2], xk[j + 3]});
-      st4(lb, L::V + swz<RB>(r, c0 + j), f32x4{xv[j], xv[j + 1], xv[j + 2], xv[j + 3]});
-    }
-  }
-  // ---- per-token factors (wave 0, lane = token): g (the in-kernel gate when asked), beta, G = inclusive scan
-  if (wave == 0) {
-    float gt = 0.f, bt = 0.f;
-    if (l < cr.len) {
-      const size_t t = (size_t)(cr.t0 + l) * rs.gb + h;
-      const float gr = io<TG>::load(g + t), br = io<TG>::load(beta + t);
-      gt = GATE ? -expf(A_log[h]) * softplus_exact(gr + dt_bias[h]) : gr;
-      bt = rs.beta_sigmoid ? 1.f / (1.f + expf(-br)) : br;
-    }
-    float G = gt;
+        for (int e = 0; e < 4; ++e) {
+          sq = fmaf(xq[j][e], xq[j][e], sq);
+          sk = fmaf(xk[j][e], xk[j][e], sk);
+        }
+      }
+      float rq = 1.f, rk = 1.f;
+      if (qk_l2norm) {
+        rq = 1.f / sqrtf(group_sum<16>(sq) + 1e-6f);
+        rk = 1.f / sqrtf(group_sum<16>(sk) + 1e-6f);
+      }
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const float o = __shfl_up(G, d, 64);
-      if (l >= d) G += o;
-    }
-    const float GL = __shfl(G, 63, 64);
-    const float eg = expf(G);
-    st1(lb, L::FG + 4 * l, G);
-    st1(lb, L::FB + 4 * l, bt);
-    st1(lb, L::FEG + 4 * l, eg);
-    st1(lb, L::FFK + 4 * l, expf(GL - G));
-    st1(lb, L::FBW + 4 * l, bt * eg);
-    if (l == 0) *reinterpret_cast<float*>(out + WS::G) = GL;
-  }
-  bar();
-  // ---- q, k L2 norm in place: x * rsqrt(sum x^2 + 1e-6), 4 threads a row
-  if (qk_l2norm) {
-    const int r = tid >> 2, c0 = (tid & 3) * (D / 4);
-    f32x4 xq[D / 16], xk[D / 16];
-    float sq = 0.f, sk = 0.f;
-#pragma unroll
-    for (int j = 0; j < D / 16; ++j) {
-      xq[j] = ld4(lb, L::Q + swz<RB>(r, c0 + 4 * j));
-      xk[j] = ld4(lb, L::K + swz<RB>(r, c0 + 4 * j));
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        sq = fmaf(xq[j][e], xq[j][e], sq);
-        sk = fmaf(xk[j][e], xk[j][e], sk);
+      for (int j = 0; j < D / 64; ++j) {
+        st4(lb, L::Q + swz<RB>(r, c0 + 64 * j), xq[j] * rq);
+        st4(lb, L::K + swz<RB>(r, c0 + 64 * j), xk[j] * rk);
+        st4(lb, L::V + swz<RB>(r, c0 + 64 * j), R.v[j].get());
       }
     }
-    sq = group_sum<4>(sq);
-    sk = group_sum<4>(sk);
-    const float rq = 1.f / sqrtf(sq + 1e-6f), rk = 1.f / sqrtf(sk + 1e-6f);
+    // per-token factors (wave 15, lane = token): g (the in-kernel gate when asked), beta, G = inclusive scan
+    if (wave == P32_WAVES - 1) {
+      float gt = 0.f, bt = 0.f;
+      if (l < len) {
+        const float gr = R.g.get(), br = R.beta.get();
+        gt = GATE ? -expf(A_log[h]) * softplus_exact(gr + dt_bias[h]) : gr;
+        bt = rs.beta_sigmoid ? 1.f / (1.f + expf(-br)) : br;
+      }
+      float G = gt;
 #pragma unroll
-    for (int j = 0; j < D / 16; ++j) {
-      st4(lb, L::Q + swz<RB>(r, c0 + 4 * j), xq[j] * rq);
-      st4(lb, L::K + swz<RB>(r, c0 + 4 * j), xk[j] * rk);
+      for (int d = 1; d < 64; d <<= 1) {
+        const float o = __shfl_up(G, d, 64);
+        if (l >= d) G += o;
+      }
+      const float GL = __shfl(G, 63, 64);
+      const float eg = expf(G);
+      st1(lb, L::FG + 4 * l, G);
+      st1(lb, L::FB + 4 * l, bt);
+      st1(lb, L::FEG + 4 * l, eg);
+      st1(lb, L::FFK + 4 * l, expf(GL - G));
+      st1(lb, L::FBW + 4 * l, bt * eg);
+      if (l == 0) *reinterpret_cast<float*>(out + WS::G) = GL;
     }
     bar();
-  }
 
-  // ---- A = strictly-lower(beta_i e^{G_i - G_j} k_i.k_j), P = s lower-incl(e^{G_i - G_j} q_i.k_j): 20 tiles
-  for (int u = wave; u < 20; u += 4) {
-    const bool isP = u >= 10;
-    int I, J;
-    tri_tile(isP ? u - 10 : u, I, J);
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    // ---- A = strictly-lower(beta_i e^{G_i - G_j} k_i.k_j) (tiles u = 0 .. 9), P = s lower-incl(e^{G_i - G_j}
+    // q_i.k_j) (u = 10 .. 19)
+    auto ap_tile = [&](int u) {
+      const bool isP = u >= 10;
+      int I, J;
+      tri_tile(isP ? u - 10 : u, I, J);
+      f32x4 a0 = z4, a1 = z4;
 #pragma unroll
-    for (int n = 0; n < NK; ++n) {
-      const f32x4 a = ld4(lb, (isP ? L::Q : L::K) + swz<RB>(16 * I + m, 16 * n + 4 * gq));
-      const f32x4 b = ld4(lb, L::K + swz<RB>(16 * J + m, 16 * n + 4 * gq));
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc = mma(a[i], b[i], acc);
-    }
-    const int cc = 16 * J + m;
-    const float Gc = ld1(lb, L::FG + 4 * cc);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = 16 * I + 4 * gq + i;
-      const float f = isP ? scale : ld1(lb, L::FB + 4 * r);
-      const bool keep = isP ? r >= cc : r > cc;
-      acc[i] = keep ? f * expf(ld1(lb, L::FG + 4 * r) - Gc) * acc[i] : 0.f;
-    }
-    blk_put(lb, isP ? L::P : L::A, I, J, acc);
-  }
-  bar();
-
-  // ---- T = (I + A)^-1: diagonal blocks by substitution (wave d inverts block d; lane m holds column m)
-  {
-    const int d = wave;
-    float x[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) x[r] = r == m ? 1.f : 0.f;
-#pragma unroll
-    for (int j = 0; j < 16; ++j)
-#pragma unroll
-      for (int r = j + 1; r < 16; ++r) x[r] = fmaf(-ld1(lb, L::A + swz<256>(16 * d + r, 16 * d + j)), x[j], x[r]);
-    if (gq == 0) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) st1(lb, L::T + swz<256>(16 * d + r, 16 * d + m), x[r]);
-    }
-  }
-  bar();
-  // off-diagonal blocks, one level at a time: T_ij = -T_ii sum_{j <= m < i} A_im T_mj
-  const f32x4 z4 = {0.f, 0.f, 0.f, 0.f};
-  if (wave < 3) {
-    const int d = wave;
-    const f32x4 y = blk_mm(lb, L::A, d + 1, d, L::T, d, d, z4);
-    blk_put(lb, L::T, d + 1, d, -blk_mm_d(lb, L::T, d + 1, d + 1, y, z4));
-  }
-  bar();
-  if (wave < 2) {
-    const int d = wave;
-    f32x4 y = blk_mm(lb, L::A, d + 2, d, L::T, d, d, z4);
-    y = blk_mm(lb, L::A, d + 2, d + 1, L::T, d + 1, d, y);
-    blk_put(lb, L::T, d + 2, d, -blk_mm_d(lb, L::T, d + 2, d + 2, y, z4));
-  }
-  bar();
-  if (wave == 0) {
-    f32x4 y = blk_mm(lb, L::A, 3, 0, L::T, 0, 0, z4);
-    y = blk_mm(lb, L::A, 3, 1, L::T, 1, 0, y);
-    y = blk_mm(lb, L::A, 3, 2, L::T, 2, 0, y);
-    blk_put(lb, L::T, 3, 0, -blk_mm_d(lb, L::T, 3, 3, y, z4));
-  }
-  bar();
-
-  // ---- R = P T diag(beta e^G) into A's place (tiles round-robin over the waves)
-  for (int u = wave; u < 10; u += 4) {
-    int I, J;
-    tri_tile(u, I, J);
-    f32x4 acc = z4;
-    for (int M = J; M <= I; ++M) acc = blk_mm(lb, L::P, I, M, L::T, M, J, acc);
-    acc *= ld1(lb, L::FBW + 4 * (16 * J + m));
-    blk_put(lb, L::A, I, J, acc);
-  }
-  bar();
-
-  // ---- W'^T and Q'^T (key tiles of this wave), with K^T: W'^T = K^T (diag(Fk) T diag(beta e^G))^T,
-  //      Q'^T = s Q^T diag(e^G) - K^T R^T; each D tile is the phase-2 A operand block (tt = I, n)
-#pragma unroll
-  for (int j = 0; j < NKW; ++j) {
-    const int n = wave * NKW + j;
-#pragma unroll
-    for (int I = 0; I < 4; ++I) {
-      const int tr = 16 * I + m;
-      const float fk = ld1(lb, L::FFK + 4 * tr);
-      f32x4 aw = z4;
-      f32x4 aq = ld4(lb, L::Q + swz<RB>(tr, 16 * n + 4 * gq)) * (scale * ld1(lb, L::FEG + 4 * tr));
-      for (int J = 0; J <= I; ++J) {
-        const f32x4 t4 = ld4(lb, L::T + swz<256>(tr, 16 * J + 4 * gq));
-        const f32x4 r4 = ld4(lb, L::A + swz<256>(tr, 16 * J + 4 * gq));
-        const f32x4 bw = ld4(lb, L::FBW + 4 * (16 * J + 4 * gq));
-        f32x4 kv;
+      for (int n = 0; n < NK; n += 2) {
+        const f32x4 xa = ld4(lb, (isP ? L::Q : L::K) + swz<RB>(16 * I + m, 16 * n + 4 * gq));
+        const f32x4 xb = ld4(lb, L::K + swz<RB>(16 * J + m, 16 * n + 4 * gq));
+        const f32x4 ya = ld4(lb, (isP ? L::Q : L::K) + swz<RB>(16 * I + m, 16 * n + 16 + 4 * gq));
+        const f32x4 yb = ld4(lb, L::K + swz<RB>(16 * J + m, 16 * n + 16 + 4 * gq));
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          kv[i] = ld1(lb, L::K + swz<RB>(16 * J + 4 * gq + i, 16 * n + m));
-          aw = mma(kv[i], t4[i] * bw[i] * fk, aw);
-          aq = mma(kv[i], -r4[i], aq);
+          a0 = mma(xa[i], xb[i], a0);
+          a1 = mma(ya[i], yb[i], a1);
         }
-        if (I == 3) st4(out, (int)(WS::K + ((size_t)(n * 4 + J) * 64 + l) * 16), kv);
       }
-      st4(out, (int)(WS::W + ((size_t)(I * NK + n) * 64 + l) * 16), aw);
+      f32x4 acc = a0 + a1;
+      const int cc = 16 * J + m, r0 = 16 * I + 4 * gq;
+      const float Gc = ld1(lb, L::FG + 4 * cc);
+      const f32x4 Gr = ld4(lb, L::FG + 4 * r0), br = ld4(lb, L::FB + 4 * r0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const bool keep = isP ? r0 + i >= cc : r0 + i > cc;
+        acc[i] = keep ? (isP ? scale : br[i]) * expf(Gr[i] - Gc) * acc[i] : 0.f;
+      }
+      if (isP || I != J)
+        blk_put(lb, m, gq, isP ? L::P : L::A, I, J, acc);
+      else
+        blk_put_t(lb, m, gq, L::A, I, I, acc);
+    };
+    // ---- 2. A and P's first 6 tiles
+    ap_tile(wave);
+    bar();
+    // the next item's rows (the last item's again past it), in flight over steps 3 and 4: by now the stores of the
+    // item before are through, behind which these loads would hold up the waves that issue them
+    load_item<TIn, TG, D>(R, min(item + (int)gridDim.x, n_items - 1), q, k, v, g, beta, cu, chunk_idx, n_seqs, T, Hk,
+                          Hv, rs);
+
+    // ---- 3. T = (I + A)^-1, the diagonal blocks: wave d < 4 by right-looking substitution on block d held as a D
+    // tile (lane: rows 4 gq + i of column m). Step j subtracts column j of the block (row j of its transpose,
+    // read ahead) times row j of the result, which the lanes of group j / 4 hand to the others by lane swaps.
+    f32x4 td[4];  // wave d < 4: column d of T as D tiles, td[i] = T_(d + i, d)
+    if (wave < 4) {
+      constexpr int AHEAD = 4;  // reads ahead (all 15 would not fit the registers beside the next item's rows)
+      f32x4 a[AHEAD];
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j) a[j] = ld4(lb, L::A + swz<256>(16 * wave + j, 16 * wave + 4 * gq));
+      f32x4 x;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i] = 4 * gq + i == m ? 1.f : 0.f;
+#pragma unroll
+      for (int j = 0; j < 15; ++j) {
+        const uint32_t own = __float_as_uint(x[j & 3]);
+        auto p = __builtin_amdgcn_permlane32_swap(own, own, false, false);
+        const uint32_t hw = p[j >> 3];  // groups (0, 1) or (2, 3) in both halves
+        p = __builtin_amdgcn_permlane16_swap(hw, hw, false, false);
+        const float t = __uint_as_float(p[(j >> 2) & 1]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = fmaf(-a[j % AHEAD][i], t, x[i]);
+        if (j + AHEAD < 15) a[j % AHEAD] = ld4(lb, L::A + swz<256>(16 * wave + j + AHEAD, 16 * wave + 4 * gq));
+      }
+      td[0] = x;
+      blk_put(lb, m, gq, L::T, wave, wave, x);
+    }
+    bar();
+    // ---- 4. wave d < 4: the rest of column d, T_id = -T_ii sum_{d <= m < i} A_im T_md, its blocks taken on as D
+    // tiles (no other column's off-diagonal block enters); waves 4-7 form P's last 4 tiles
+    if (wave < 4) {
+#pragma unroll
+      for (int i = 1; i < 4; ++i) {
+        td[i] = z4;
+        if (wave + i < 4) {  // (wave-uniform)
+          f32x4 y = z4;
+#pragma unroll
+          for (int e = 0; e < i; ++e) y = blk_mm_d(lb, m, gq, L::A, wave + i, wave + e, td[e], y);
+          td[i] = -blk_mm_d(lb, m, gq, L::T, wave + i, wave + i, y, z4);
+          blk_put(lb, m, gq, L::T, wave + i, wave, td[i]);
+        }
+      }
+    } else if (wave < 8) {
+      ap_tile(12 + wave);
+    }
+    bar();
+
+    // the next item's rows are waited for here, ahead of this item's stores: a wait behind them would cover the
+    // stores too (one counter), i.e. every workgroup's burst of writes
+    R.arrive();
+    // ---- 5. beside each other (all of them need T and P alone):
+    if (wave < 4) {
+      // R = P T diag(beta e^G) into A's place: wave d column d, from its D tiles
+      const float bw = ld1(lb, L::FBW + 4 * (16 * wave + m));
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (wave + i < 4) {
+          f32x4 acc = z4;
+#pragma unroll
+          for (int e = 0; e <= i; ++e) acc = blk_mm_d(lb, m, gq, L::P, wave + i, wave + e, td[e], acc);
+          blk_put(lb, m, gq, L::A, wave + i, wave, acc * bw);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+    } else if (wave < 4 + NK) {
+      // Ub = T diag(beta) V and Ob = P Ub (value tile vb); Ub' = diag(Fk) Ub
+      const int vb = wave - 4;
+      f32x4 ub[4];
+#pragma unroll
+      for (int I = 0; I < 4; ++I) ub[I] = z4;
+#pragma unroll
+      for (int J = 0; J < 4; ++J) {
+        const f32x4 b4 = ld4(lb, L::FB + 4 * (16 * J + 4 * gq));
+        f32x4 vv;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vv[i] = b4[i] * ld1(lb, L::V + swz<RB>(16 * J + 4 * gq + i, 16 * vb + m));
+#pragma unroll
+        for (int I = J; I < 4; ++I) ub[I] = blk_mm_d(lb, m, gq, L::T, I, J, vv, ub[I]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int I = 0; I < 4; ++I) {
+        f32x4 ob = z4;
+#pragma unroll
+        for (int J = 0; J <= I; ++J) ob = blk_mm_d(lb, m, gq, L::P, I, J, ub[J], ob);
+        const f32x4 fk = ld4(lb, L::FFK + 4 * (16 * I + 4 * gq));
+        st4(out, (int)(WS::U + ((size_t)(vb * 4 + I) * 64 + l) * 16), ub[I] * fk);
+        st4(out, (int)(WS::O + ((size_t)(vb * 4 + I) * 64 + l) * 16), ob);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      // W'^T = K^T (diag(Fk) T diag(beta e^G))^T, with K^T: each D tile is the phase-2 A operand block (tt = I, n)
+      for (int n = wave - 4 - NK; n < NK; n += 12 - NK) {
+        f32x4 aw[4];
+#pragma unroll
+        for (int I = 0; I < 4; ++I) aw[I] = z4;
+#pragma unroll
+        for (int J = 0; J < 4; ++J) {
+          const f32x4 bw = ld4(lb, L::FBW + 4 * (16 * J + 4 * gq));
+          f32x4 kv, kb;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            kv[i] = ld1(lb, L::K + swz<RB>(16 * J + 4 * gq + i, 16 * n + m));
+            kb[i] = kv[i] * bw[i];
+          }
+          st4(out, (int)(WS::K + ((size_t)(n * 4 + J) * 64 + l) * 16), kv);
+#pragma unroll
+          for (int I = J; I < 4; ++I) {
+            const f32x4 t4 = ld4(lb, L::T + swz<256>(16 * I + m, 16 * J + 4 * gq));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) aw[I] = mma(kb[i], t4[i], aw[I]);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int I = 0; I < 4; ++I)
+          st4(out, (int)(WS::W + ((size_t)(I * NK + n) * 64 + l) * 16), aw[I] * ld1(lb, L::FFK + 4 * (16 * I + m)));
+      }
+    }
+    bar();
+
+    // ---- 6. Q'^T = s Q^T diag(e^G) - K^T R^T: (token tile, key tile) jobs, each wave one long and one short one
+    // (D = 128: token tiles {3, 0} or {2, 1} of one key tile; D = 64: one job a wave)
+#pragma unroll
+    for (int half = 0; half < NK / 4; ++half) {
+      const int n = wave % NK, u = wave / NK;
+      const int I = NK == 8 ? (half == 0 ? 3 - u : u) : 3 - u;
+      const int tr = 16 * I + m;
+      f32x4 aq = ld4(lb, L::Q + swz<RB>(tr, 16 * n + 4 * gq)) * (scale * ld1(lb, L::FEG + 4 * tr));
+      for (int J = 0; J <= I; ++J) {
+        const f32x4 r4 = ld4(lb, L::A + swz<256>(tr, 16 * J + 4 * gq));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) aq = mma(ld1(lb, L::K + swz<RB>(16 * J + 4 * gq + i, 16 * n + m)), -r4[i], aq);
+      }
       st4(out, (int)(WS::Q + ((size_t)(I * NK + n) * 64 + l) * 16), aq);
     }
-  }
-  // ---- Ub = T diag(beta) V and Ob = P Ub (value tiles of this wave); Ub' = diag(Fk) Ub
-#pragma unroll
-  for (int j = 0; j < NKW; ++j) {
-    const int vb = wave * NKW + j;
-    f32x4 ub[4];
-#pragma unroll
-    for (int I = 0; I < 4; ++I) {
-      f32x4 acc = z4;
-      for (int J = 0; J <= I; ++J) {
-        const f32x4 t4 = ld4(lb, L::T + swz<256>(16 * I + m, 16 * J + 4 * gq));
-        const f32x4 b4 = ld4(lb, L::FB + 4 * (16 * J + 4 * gq));
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc = mma(t4[i] * b4[i], ld1(lb, L::V + swz<RB>(16 * J + 4 * gq + i, 16 * vb + m)), acc);
-      }
-      ub[I] = acc;
-    }
-#pragma unroll
-    for (int I = 0; I < 4; ++I) {
-      f32x4 ob = z4;
-#pragma unroll
-      for (int J = 0; J <= I; ++J) ob = blk_mm_d(lb, L::P, I, J, ub[J], ob);
-      const f32x4 fk = ld4(lb, L::FFK + 4 * (16 * I + 4 * gq));
-      st4(out, (int)(WS::U + ((size_t)(vb * 4 + I) * 64 + l) * 16), ub[I] * fk);
-      st4(out, (int)(WS::O + ((size_t)(vb * 4 + I) * 64 + l) * 16), ob);
-    }
+    bar();  // the next item's rows overwrite the LDS
   }
 }
 
 // ----------------------------------------------------------------------------------------------- phase 2
 //
-// One workgroup of 4 waves per (sequence, value head, 16 value rows vb); wave w holds the state rows' key tiles
-// n = w NK/4 .. as D tiles of S^T (lane: S[16 vb + m][16 n + 4 g + i]), which are the B operands of W' S^T and
-// Q' S^T as they stand. Per chunk every wave forms its keys' part of W' S^T and Q' S^T for all 64 tokens and
-// puts it in LDS; after one barrier each wave sums the four parts in wave order into U' = Ub' - W' S^T (all 64
-// tokens: the B operands of its update), and wave w the outputs of token tile w. LDS buffers alternate by
-// chunk, so one barrier a chunk suffices. The next chunk's operands are loaded while the current one computes.
+// One workgroup of 8 waves per (sequence, value head, 16 value rows vb). Wave n < NK holds key tile n of the
+// state rows as a D tile of S^T (lane: S[16 vb + m][16 n + 4 g + i]), which is the B operand of W' S^T and Q' S^T
+// as it stands. Per chunk: the tiles go to LDS; wave tt < 4 forms U' = Ub' - W' S^T of token tile tt over all keys
+// and puts it in LDS, wave 4 + tt the outputs O = Ob + Q' S^T of token tile tt; then every wave n < NK takes all
+// of U' into its tile, S^T <- e^{G_L} S^T + K^T U'. Each SIMD runs one wave of either kind, so its matrix unit
+// (96 products of 32 cycles a chunk at D = 128, 1.28 us, the pass's bound) has a second wave to work for while
+// one is at a barrier or in LDS; the next chunk's operands are loaded in three groups between the phases, as
+// loads issued in one burst hold up the waves that issue them. T = 4096 at 16 heads, D = 128 (64 chunks): 129 us,
+// 2.0 us a chunk; T = 256, 4 heads, D = 64: 5.5 us. With 4 waves, each doing all three products over its quarter
+// of the keys (partial sums through LDS) and the loads in one burst: 190 and 9.6 us.
 template <int D>
 struct Ops32 {
-  static constexpr int NKW = D / 64;
-  f32x4 W[4][NKW], Q[4][NKW], K[NKW][4], U[4], O;
+  static constexpr int NK = D / 16;
+  f32x4 A[NK];  // W' (waves 0-3) or Q' (4-7) of this wave's token tile
+  f32x4 K[4];   // K^T of this wave's key tile
+  f32x4 X;      // Ub' or Ob of this wave's token tile
   float GL;
 };
 
-template <int D>
-__device__ __forceinline__ void load_ops(Ops32<D>& p, const uint8_t* base, int wave, int vb) {
-  using WS = Ws32<D>;
-  constexpr int NK = WS::NK, NKW = NK / 4;
-  const int l = threadIdx.x & 63;
-  auto at = [&](size_t off) { return *reinterpret_cast<const f32x4*>(base + off + (size_t)l * 16); };
-#pragma unroll
-  for (int j = 0; j < NKW; ++j) {
-    const int n = wave * NKW + j;
-#pragma unroll
-    for (int tt = 0; tt < 4; ++tt) {
-      p.W[tt][j] = at(WS::W + (size_t)(tt * NK + n) * 1024);
-      p.Q[tt][j] = at(WS::Q + (size_t)(tt * NK + n) * 1024);
-      p.K[j][tt] = at(WS::K + (size_t)(n * 4 + tt) * 1024);
-    }
+// Stores a D tile of outputs (rows r0 .. r0 + 3 of column col of the chunk's rows, lanes l and l ^ 1 adjacent
+// columns) through a buffer resource that ends with the chunk's last token: two rows a lane as column pairs.
+template <typename TOut>
+__device__ __forceinline__ void store_tile32(Rsrc w, uint32_t row_bytes, int r0, int col, f32x4 d) {
+  const bool odd = (threadIdx.x & 1) != 0;
+  const float x0 = dpp<DPP_QUAD_XOR1>(odd ? d[0] : d[2]), x1 = dpp<DPP_QUAD_XOR1>(odd ? d[1] : d[3]);
+  const float a0 = odd ? x0 : d[0], b0 = odd ? d[2] : x0, a1 = odd ? x1 : d[1], b1 = odd ? d[3] : x1;
+  const uint32_t off = (uint32_t)(r0 + (odd ? 2 : 0)) * row_bytes + (uint32_t)(col & ~1) * (uint32_t)sizeof(TOut);
+  if constexpr (sizeof(TOut) == 2) {
+    __builtin_amdgcn_raw_buffer_store_b32(pack_bf16x2(a0, b0), w, off, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b32(pack_bf16x2(a1, b1), w, off + row_bytes, 0, 0);
+  } else {
+    typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(a0), __float_as_uint(b0)}, w, off, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(a1), __float_as_uint(b1)}, w, off + row_bytes, 0, 0);
   }
+}
+
+template <int D>
+struct StateShared32 {
+  f32x4 S[D / 16][64];  // the state's D tiles
+  f32x4 U[4][64];       // U' of the 4 token tiles
+};
+
+// The chunk loop of one wave (U: waves 0-3, else the output waves).
+template <bool U, typename TOut, int D>
+__device__ __forceinline__ void state_loop32(StateShared32<D>& sh, f32x4& st, const uint8_t* ws, TOut* o, int c0,
+                                             int nc, int bos, int len, int Hv, int h, int vb, int wave) {
+  using WS = Ws32<D>;
+  constexpr int NK = WS::NK;
+  const int l = threadIdx.x & 63, m = l & 15, gq = l >> 4;
+  const int tt = wave & 3;
+  const bool upd = wave < NK;  // this wave holds a state tile (all 8 at D = 128, the U waves at 64)
+  const uint32_t offA = (uint32_t)((U ? WS::W : WS::Q) + (size_t)tt * NK * 1024) + 16u * l;
+  const uint32_t offX = (uint32_t)((U ? WS::U : WS::O) + (size_t)(vb * 4 + tt) * 1024) + 16u * l;
+  const uint32_t offK = (uint32_t)(WS::K + (size_t)(wave & (NK - 1)) * 4 * 1024) + 16u * l;
+  auto chunk_ws = [&](int ci) { return raw_rsrc(ws + ((size_t)(c0 + ci) * Hv + h) * WS::ITEM, (uint32_t)WS::ITEM); };
+  auto ld = [](Rsrc w, uint32_t off) {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(w, off, 0, 0));
+  };
+  auto fetch1 = [&](Rsrc w, Ops32<D>& p) {
 #pragma unroll
-  for (int tt = 0; tt < 4; ++tt) p.U[tt] = at(WS::U + (size_t)(vb * 4 + tt) * 1024);
-  p.O = at(WS::O + (size_t)(vb * 4 + wave) * 1024);
-  p.GL = *reinterpret_cast<const float*>(base + WS::G);
+    for (int n = 0; n < NK / 2; ++n) p.A[n] = ld(w, offA + 1024u * n);
+    p.GL = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(w, 0, (int)WS::G, 0));
+  };
+  auto fetch2 = [&](Rsrc w, Ops32<D>& p) {
+#pragma unroll
+    for (int n = NK / 2; n < NK; ++n) p.A[n] = ld(w, offA + 1024u * n);
+    p.X = ld(w, offX);
+  };
+  auto fetch3 = [&](Rsrc w, Ops32<D>& p) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) p.K[t] = ld(w, offK + 1024u * t);
+  };
+  const f32x4 z4 = {0.f, 0.f, 0.f, 0.f};
+  auto process = [&](int ci, const Ops32<D>& cur, int ni, Ops32<D>& nxt) {
+    if (upd) sh.S[wave][l] = st;
+    const Rsrc wn = chunk_ws(ni);
+    fetch1(wn, nxt);
+    bar();
+    f32x4 x0 = z4, x1 = z4;
+#pragma unroll
+    for (int n = 0; n < NK; n += 2) {
+      const f32x4 s0 = sh.S[n][l], s1 = sh.S[n + 1][l];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        x0 = mma(cur.A[n][i], s0[i], x0);
+        x1 = mma(cur.A[n + 1][i], s1[i], x1);
+      }
+    }
+    f32x4 ov = z4;
+    if constexpr (U)
+      sh.U[tt][l] = cur.X - (x0 + x1);
+    else
+      ov = cur.X + (x0 + x1);
+    fetch2(wn, nxt);
+    bar();
+    fetch3(wn, nxt);
+    if (upd) {
+      f32x4 s0 = st * expf(cur.GL), s1 = z4;
+#pragma unroll
+      for (int t = 0; t < 4; t += 2) {
+        const f32x4 u0 = sh.U[t][l], u1 = sh.U[t + 1][l];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          s0 = mma(cur.K[t][i], u0[i], s0);
+          s1 = mma(cur.K[t + 1][i], u1[i], s1);
+        }
+      }
+      st = s0 + s1;
+    }
+    if constexpr (!U) {
+      const uint32_t row = (uint32_t)Hv * D * (uint32_t)sizeof(TOut);
+      const int tl = min(CHUNK_LEN, len - ci * CHUNK_LEN);
+      store_tile32<TOut>(raw_rsrc(o + ((size_t)(bos + ci * CHUNK_LEN) * Hv + h) * D + 16 * vb, (uint32_t)tl * row), row,
+                         16 * tt + 4 * gq, m, ov);
+    }
+  };
+  // two register buffers in turn, filled one chunk ahead (the last chunk is fetched again at the end, so that
+  // every path issues the same loads)
+  const int last = nc - 1;
+  Ops32<D> b0, b1;
+  {
+    const Rsrc w0 = chunk_ws(0);
+    fetch1(w0, b0);
+    fetch2(w0, b0);
+    fetch3(w0, b0);
+  }
+  process(0, b0, min(1, last), b1);
+  int ci = 1;
+  for (; ci + 1 < nc; ci += 2) {
+    process(ci, b1, ci + 1, b0);
+    process(ci + 1, b0, min(ci + 2, last), b1);
+  }
+  if (ci < nc) process(ci, b1, ci, b0);
 }
 
 template <typename TOut, int D>
-__global__ __launch_bounds__(256) void chunk32_state_kernel(const uint8_t* ws, const float* __restrict__ s_in,
+__global__ __launch_bounds__(512) void chunk32_state_kernel(const uint8_t* ws, const float* __restrict__ s_in,
                                                             float* __restrict__ s_out, TOut* __restrict__ o,
                                                             const int32_t* __restrict__ cu, int n_seqs,
                                                             int n_chunks, int T, int Hv) {
-  using WS = Ws32<D>;
-  constexpr int NK = WS::NK, NKW = NK / 4;
-  // partial products of the 4 waves: [buffer][U', O][wave][token tile][lane]
-  __shared__ f32x4 part[2][2][4][4][64];
+  // (ws is not __restrict__: the prefetch loads stay where they are issued, ahead of the barriers)
+  constexpr int NK = Ws32<D>::NK;
+  __shared__ StateShared32<D> sh;
   // the NK workgroups of one (sequence, head) share an id % 8, so they run on one XCD and share its L2 copy of
   // the chunk workspace (the grid is padded to whole groups of 8 NK)
   const int id = blockIdx.x;
@@ -409,70 +618,16 @@ __global__ __launch_bounds__(256) void chunk32_state_kernel(const uint8_t* ws, c
   // chunks past the workspace (a chunk table shorter than the sequences need) are not read
   const int nc = max(0, min((len + CHUNK_LEN - 1) / CHUNK_LEN, n_chunks - c0));
 
-  const size_t srow = ((size_t)pair * D + 16 * vb + m) * D;  // this lane's state row
-  f32x4 st[NKW];
-#pragma unroll
-  for (int j = 0; j < NKW; ++j) {
-    const int col = 16 * (wave * NKW + j) + 4 * gq;
-    st[j] = s_in != nullptr ? *reinterpret_cast<const f32x4*>(s_in + srow + col) : f32x4{0.f, 0.f, 0.f, 0.f};
+  const size_t at = ((size_t)pair * D + 16 * vb + m) * D + 16 * (wave & (NK - 1)) + 4 * gq;  // this lane's entries
+  f32x4 st = {0.f, 0.f, 0.f, 0.f};
+  if (s_in != nullptr) st = *reinterpret_cast<const f32x4*>(s_in + at);
+  if (nc > 0) {
+    if (wave < 4)
+      state_loop32<true, TOut, D>(sh, st, ws, o, c0, nc, bos, len, Hv, h, vb, wave);
+    else
+      state_loop32<false, TOut, D>(sh, st, ws, o, c0, nc, bos, len, Hv, h, vb, wave);
   }
-  const f32x4 z4 = {0.f, 0.f, 0.f, 0.f};
-  Ops32<D> cur;
-  if (nc > 0) load_ops<D>(cur, ws + ((size_t)c0 * Hv + h) * WS::ITEM, wave, vb);
-  for (int ci = 0; ci < nc; ++ci) {
-    Ops32<D> nxt;
-    load_ops<D>(nxt, ws + ((size_t)(c0 + min(ci + 1, nc - 1)) * Hv + h) * WS::ITEM, wave, vb);
-    const int b = ci & 1;
-#pragma unroll
-    for (int tt = 0; tt < 4; ++tt) {
-      f32x4 pu = z4, po = z4;
-#pragma unroll
-      for (int j = 0; j < NKW; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          pu = mma(cur.W[tt][j][i], st[j][i], pu);
-          po = mma(cur.Q[tt][j][i], st[j][i], po);
-        }
-      part[b][0][wave][tt][l] = pu;
-      part[b][1][wave][tt][l] = po;
-    }
-    __syncthreads();
-    f32x4 u[4];
-#pragma unroll
-    for (int tt = 0; tt < 4; ++tt) {
-      u[tt] = cur.U[tt];
-#pragma unroll
-      for (int w = 0; w < 4; ++w) u[tt] -= part[b][0][w][tt][l];
-    }
-    f32x4 ov = cur.O;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) ov += part[b][1][w][wave][l];
-    // outputs of token tile `wave`: rows 16 wave + 4 g + i of column 16 vb + m
-    const int tl = min(CHUNK_LEN, len - ci * CHUNK_LEN);
-    const size_t t0 = (size_t)bos + (size_t)ci * CHUNK_LEN;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = 16 * wave + 4 * gq + i;
-      if (r < tl) io<TOut>::store(o + ((t0 + r) * Hv + h) * D + 16 * vb + m, ov[i]);
-    }
-    // S^T <- e^{G_L} S^T + K^T U'
-    const float gam = expf(cur.GL);
-#pragma unroll
-    for (int j = 0; j < NKW; ++j) {
-      f32x4 acc = st[j] * gam;
-#pragma unroll
-      for (int tt = 0; tt < 4; ++tt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc = mma(cur.K[j][tt][i], u[tt][i], acc);
-      st[j] = acc;
-    }
-    cur = nxt;
-  }
-  if (s_out != nullptr) {
-#pragma unroll
-    for (int j = 0; j < NKW; ++j)
-      *reinterpret_cast<f32x4*>(s_out + srow + 16 * (wave * NKW + j) + 4 * gq) = st[j];
-  }
+  if (s_out != nullptr && wave < NK) *reinterpret_cast<f32x4*>(s_out + at) = st;
 }
 
 // Phase 1's dynamic LDS is above the default 64 KiB at D = 128: raised once per device and kernel (the first
@@ -500,9 +655,13 @@ int launch_prep32(const char* fn, int n_items, const void* q, const void* k, con
   constexpr int bytes = Lds32<D>::BYTES;
   if (bytes > 65536 && !lds_ready(chunk32_prep_kernel<TIn, TG, D, GATE>, bytes, state))
     return fail(ZGDN_EHIP, "%s: the device refused %d bytes of LDS for the fp32 chunk kernel", fn, bytes);
-  hipLaunchKernelGGL((chunk32_prep_kernel<TIn, TG, D, GATE>), dim3(n_items), dim3(256), bytes, s, (const TIn*)q, (const TIn*)k, (const TIn*)v,
-                     (const TG*)g, (const TG*)beta, A_log, dt_bias, cu, chunk_idx, n_seqs, T, Hk, Hv, scale,
-                     qk_l2norm, rs, ws);
+  int dev = 0, n_cu = 256;
+  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    n_cu = 256;
+  hipLaunchKernelGGL((chunk32_prep_kernel<TIn, TG, D, GATE>), dim3(std::min(n_items, std::max(1, n_cu))),
+                     dim3(64 * P32_WAVES), bytes, s, (const TIn*)q, (const TIn*)k, (const TIn*)v, (const TG*)g,
+                     (const TG*)beta, A_log, dt_bias, cu, chunk_idx, n_seqs, n_items, T, Hk, Hv, scale, qk_l2norm,
+                     rs, ws);
   return ZGDN_OK;
 }
 
@@ -530,7 +689,7 @@ int run32(const char* fn, int n_chunks, const void* q, const void* k, const void
   constexpr int NK = D / 16;
   const long pairs = (long)N * Hv;
   const dim3 grid((unsigned)(((pairs + 7) / 8) * 8 * NK));
-  hipLaunchKernelGGL((chunk32_state_kernel<TIn, D>), grid, dim3(256), 0, s, ws, s_in, s_out, (TIn*)o, cu, N, n_chunks, T, Hv);
+  hipLaunchKernelGGL((chunk32_state_kernel<TIn, D>), grid, dim3(512), 0, s, ws, s_in, s_out, (TIn*)o, cu, N, n_chunks, T, Hv);
   return check_launch(fn);
 }
 
