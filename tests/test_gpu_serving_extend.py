@@ -1,0 +1,96 @@
+"""The serving layer's eager prefill / extend with the caches read and written in place (``_extend_in_place``)
+against the general path over the same calls (``_extend``: index lists, two passes, the operator route; taken when
+an operator attribute is rebound): outputs and every cache.
+
+Where a call's runs are all complete chunks, or all open ones, both paths run the same projections over the same
+rows, and everything is equal to the bit. Where a call holds both, the general path projects them in two products of
+other shapes, whose sums may round an occasional bf16 element the other way: one such element of a row (2^-8
+relative) moves that row's outputs and the state by a share of it, measured up to ~2e-3 relative (test_gpu_serving),
+held here to 5e-3 of the largest value."""
+
+from __future__ import annotations
+
+import importlib
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from gdn_testing import announce, rel_err
+
+pytestmark = pytest.mark.gpu
+
+CACHES = ("_live_state", "_recurrent_state", "_live_conv", "_conv_state", "_win_len")
+
+
+def _pair(serving, cuda, hidden, capacity, seed):
+    gen = torch.Generator().manual_seed(seed)
+    bf = torch.bfloat16
+    w = {"in_proj": (0.05 * torch.randn(2056, hidden, generator=gen)).to(bf).to(cuda),
+         "conv": (0.2 * torch.randn(1536, 1, 4, generator=gen)).to(bf).to(cuda),
+         "wo": (0.05 * torch.randn(hidden, 512, generator=gen)).to(bf).to(cuda)}
+    out_weight = (1 + 0.1 * torch.randn(128, generator=gen)).to(bf).to(cuda)
+    A_log, dt_bias = (0.2 * torch.randn(4, generator=gen).to(cuda) for _ in range(2))
+    fla = importlib.import_module("zonos3-mini_amd.fla_ops")
+    layers = []
+    for general in (False, True):
+        batch = SimpleNamespace(is_decode=False, padded_size=0, gdn_prefill=None, reqs=[], padded_reqs=[])
+        layer = serving.OriginalGDN(SimpleNamespace(hidden_size=hidden), 0, batch_source=lambda b=batch: b)
+        for name in w:
+            getattr(layer, name).weight = w[name]
+        layer.out_weight, layer.A_log, layer.dt_bias = out_weight, A_log, dt_bias
+        layer.allocate_cache(capacity, cuda, bf)
+        if general:
+            layer._conv_fwd = lambda **kw: fla.causal_conv1d_fwd(**kw)
+        assert layer._own_operators() is not general
+        layers.append((layer, batch))
+    return layers, gen
+
+
+# (slot -> new rows) calls in order, and whether every call's rows go to one pass of the general path
+@pytest.mark.parametrize("name,calls,exact", [
+    ("complete chunks", [{0: 64, 1: 192}, {1: 128, 0: 64}], True),
+    ("open chunks", [{2: 1, 0: 63, 1: 3}, {0: 0, 1: 2, 2: 40}, {2: 5}], True),
+    ("ragged", [{0: 70, 1: 5, 2: 63, 3: 200}, {3: 1, 0: 58, 2: 1}, {1: 300, 3: 64, 2: 2, 4: 64}, {0: 9}], False),
+    ("many requests", [{s: 7 + 31 * s for s in range(12)}, {s: 90 - 7 * s for s in range(12)}], False),
+])
+def test_in_place_extend_equals_the_general_path(gdn, cuda, name, calls, exact):
+    serving = importlib.import_module("zonos3-mini_amd.serving")
+    announce(f"serving extend in place: {name}")
+    hidden, capacity = 256, 13
+    (a, batch_a), (b, batch_b) = _pair(serving, cuda, hidden, capacity, 5100)[0]
+    gen = torch.Generator().manual_seed(5101)
+    held = {}
+    for layer in (a, b):  # what a slot held before must not matter to a fresh request
+        for cache in ("_live_state", "_recurrent_state"):
+            getattr(layer, cache).fill_(0.5)
+        for cache in ("_live_conv", "_conv_state", "_window"):
+            getattr(layer, cache).fill_(0.25)
+    for rows in calls:
+        rows = {s: n for s, n in rows.items() if n}
+        reqs = [SimpleNamespace(table_idx=s, uid=s, is_cfg_uncond=False, cached_len=held.get(s, 0), extend_len=n)
+                for s, n in rows.items()]
+        x = torch.randn(sum(rows.values()), hidden, generator=gen).to(torch.bfloat16).to(cuda)
+        ys = []
+        for layer, batch in ((a, batch_a), (b, batch_b)):
+            batch.reqs = batch.padded_reqs = reqs
+            ys.append(layer.forward(x))
+        torch.cuda.synchronize()
+        for s, n in rows.items():
+            held[s] = held.get(s, 0) + n
+        used = sorted(held)
+        if exact:
+            assert torch.equal(*ys), rows
+        else:
+            assert rel_err(ys[0].float(), ys[1].float()) < 5e-3, (rows, rel_err(ys[0].float(), ys[1].float()))
+        for cache in CACHES:
+            ta, tb = (getattr(layer, cache)[used].cpu() for layer in (a, b))
+            if exact or cache == "_win_len":
+                assert torch.equal(ta, tb), (rows, cache)
+            else:
+                assert rel_err(ta.float(), tb.float()) < 5e-3, (rows, cache, rel_err(ta.float(), tb.float()))
+        for s in used:
+            fill = held[s] % 64
+            assert torch.equal(a._window[s, :fill], b._window[s, :fill]), (rows, s)
+        others = [s for s in range(capacity) if s not in held]
+        assert bool((a._live_state[others] == 0.5).all()) and bool((a._window[others] == 0.25).all())

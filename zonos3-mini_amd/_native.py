@@ -85,6 +85,18 @@ SIGNATURES: dict[str, tuple] = {
     ),
 }
 
+# Entry points of this package's own host layer, outside the published header: name -> (restype, argtypes).
+INTERNAL: dict[str, tuple] = {
+    "zgdn_serving_gather": (
+        c_int, [_P, _P, c_int, c_int, _P, c_int, c_int, c_int, c_int, c_int, _P, _P]),
+    "zgdn_serving_extend_workspace": (c_size_t, [c_int, c_int, c_int]),
+    "zgdn_serving_extend": (
+        c_int,
+        [_P, c_long, _P, c_int, c_int, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P, _P, _P, _P, _P, _P, _P, _P,
+         _P, _P, _P, c_float, c_float, _P, c_size_t, _P],
+    ),
+}
+
 _lib: ctypes.CDLL | None = None
 
 
@@ -102,7 +114,7 @@ def lib() -> ctypes.CDLL:
             handle = ctypes.CDLL(str(LIB_PATH), mode=ctypes.RTLD_GLOBAL)
         except OSError as exc:
             raise RuntimeError(f"cannot load {LIB_PATH}: {exc}") from exc
-        for name, (res, args) in SIGNATURES.items():
+        for name, (res, args) in (SIGNATURES | INTERNAL).items():
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args

@@ -1200,6 +1200,75 @@ __global__ __launch_bounds__(64 * P2_WAVES) void chunk_state_kernel(
   }
 }
 
+// The state pass of a serving call: run s's states are its slot's, read from the committed cache (zeros for a fresh
+// slot) and written to the live one after the run's last row and to the committed one after its complete chunks
+// (untouched when it has none; zeros for a fresh slot). The open chunk is a second, one-chunk loop, so that the
+// states between are at hand without a test in the chunk loop; otherwise chunk_state_kernel's packed form.
+template <int NV>
+__global__ __launch_bounds__(64 * P2_WAVES) void chunk_serve_state_kernel(const uint8_t* ws, const ServeRuns r,
+                                                                          float* commit, float* __restrict__ live,
+                                                                          bf16* __restrict__ o, int Hv) {
+  __shared__ StateSharedT<NV> sh;
+  constexpr int NG = DV / VB / NV;
+  const int id = blockIdx.x;
+  const int pair = (id / (8 * NG)) * 8 + (id % 8), vb = ((id % (8 * NG)) / 8) * NV;
+  if (pair >= r.n_runs * Hv) return;
+  const int h = pair % Hv, seq = pair / Hv;
+  const int slot = r.slots[seq];
+  if (slot < 0 || slot >= r.n_slots) return;
+  const int l = lane_id(), wave = threadIdx.x >> 6;
+  const int ncol = 16 * wave + (l & 15);
+  StateArgs a;
+  a.ws = ws;
+  a.Hv = Hv;
+  a.h = h;
+  a.vb = vb;
+  a.xs = 1.f;
+  a.flags = nullptr;
+  a.flag_step = 0;
+  a.spin_max = 0;
+  int bos, len;
+  seq_chunks(r.cu, seq, r.rows, a.c0, bos, len);
+  const int nc = max(0, min((len + CH - 1) / CH, r.n_chunks - a.c0));
+  const int whole = min(nc, len / CH);  // complete chunks
+  const bool fresh = r.fresh[seq] != 0;
+  f32x4 S[NV];
+  const size_t base = ((size_t)slot * Hv + h) * DV * DK;
+  auto at = [&](int v, int i4) { return base + ((size_t)(vb + v) * VB + 4 * (l >> 4) + i4) * DK + ncol; };
+#pragma unroll
+  for (int v = 0; v < NV; ++v)
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) S[v][i4] = fresh ? 0.f : commit[at(v, i4)];
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // settle the state loads before the pipelined loop
+  auto loop = [&]() {
+    if (wave < 4)
+      state_loop<true, bf16, false, NV>(sh, a, o, S);
+    else
+      state_loop<false, bf16, false, NV>(sh, a, o, S);
+  };
+  a.bos = bos;
+  a.len = whole * CH;
+  a.nchunks = whole;
+  loop();
+  if (whole > 0 || fresh) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4) commit[at(v, i4)] = S[v][i4];
+  }
+  if (nc > whole) {
+    a.bos = bos + whole * CH;
+    a.len = len - whole * CH;
+    a.c0 += whole;
+    a.nchunks = 1;
+    loop();
+  }
+#pragma unroll
+  for (int v = 0; v < NV; ++v)
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) live[at(v, i4)] = S[v][i4];
+}
+
 // ------------------------------------------------------------------------------- phases 1 and 2 overlapped
 //
 // One launch in which phase 1 and the state pass run side by side. The state pass of a (sequence, head) chain
@@ -2016,4 +2085,88 @@ extern "C" int zgdn_chunk_fwd_noalloc(const void* q, const void* k, const void* 
   return chunk_fwd_impl(fn, q, k, v, qkv_dtype, g, beta, gb_dtype, A_log, dt_bias, qk_l2norm, initial_state,
                         final_state, o, cu_seqlens, chunk_indices, n_seqs, n_chunks, B, T, Hk, Hv, K, V, q_ld,
                         k_ld, v_ld, gb_ld, beta_sigmoid, scale, ptr, bytes, stream);
+}
+
+
+// The serving layer's eager call (see serving.py): the rows-in-place gather, and everything between the two
+// projections.
+static int serve_runs(const char* fn, const int32_t* tables, int n_runs, int n_chunks, int rows, int new_rows,
+                      int n_slots, zgdn::ServeRuns* r) {
+  using namespace zgdn;
+  if (!tables) return fail(ZGDN_EINVAL, "%s: null pointer", fn);
+  if (n_runs < 1 || n_chunks < 1 || rows < 1 || new_rows < 1 || new_rows > rows || n_slots < 1)
+    return fail(ZGDN_EINVAL, "%s: bad sizes n_runs=%d n_chunks=%d rows=%d new_rows=%d n_slots=%d", fn, n_runs, n_chunks,
+                rows, new_rows, n_slots);
+  // cu [n + 1], slots [n], replay [n], xoff [n], fresh [n], pairs [2 n_chunks]
+  const int32_t* p = tables + n_runs + 1;
+  *r = ServeRuns{tables, p + 4 * (size_t)n_runs, p, p + n_runs, p + 2 * (size_t)n_runs, p + 3 * (size_t)n_runs,
+                 n_runs, n_chunks, rows, new_rows, n_slots};
+  return ZGDN_OK;
+}
+
+extern "C" int zgdn_serving_gather(const void* x, const void* window, int hidden, int dtype, const int32_t* tables,
+                                   int n_runs, int n_chunks, int rows, int new_rows, int n_slots, void* out,
+                                   void* stream) {
+  using namespace zgdn;
+  const char* fn = "zgdn_serving_gather";
+  ServeRuns r;
+  if (const int st = serve_runs(fn, tables, n_runs, n_chunks, rows, new_rows, n_slots, &r)) return st;
+  if (!x || !window || !out) return fail(ZGDN_EINVAL, "%s: null pointer", fn);
+  if (dtype != ZGDN_BF16 || hidden < 8 || hidden % 8 || (((uintptr_t)x | (uintptr_t)window | (uintptr_t)out) % 16))
+    return fail(ZGDN_EUNSUPPORTED, "%s: bf16 rows of a multiple of 8 elements from 16-byte aligned bases (dtype %d, "
+                "hidden %d)", fn, dtype, hidden);
+  serve_gather(r, x, window, hidden, out, (hipStream_t)stream);
+  return check_launch(fn);
+}
+
+extern "C" size_t zgdn_serving_extend_workspace(int n_chunks, int rows, int H) {
+  if (n_chunks < 1 || rows < 1 || H < 1) return 0;
+  return (size_t)n_chunks * H * zgdn::WS_CHUNK + (size_t)rows * H * 128 * 2 * 4;
+}
+
+extern "C" int zgdn_serving_extend(const void* mixed, long mixed_ld, const void* x, int hidden, int dtype,
+                                   const int32_t* tables, int n_runs, int n_chunks, int rows, int new_rows, int n_slots,
+                                   int H, const void* conv_weight, const float* A_log, const float* dt_bias,
+                                   const void* norm_weight, void* conv_commit, void* conv_live, float* state_commit,
+                                   float* state_live, void* window, int32_t* win_len, void* gated, float eps,
+                                   float scale, void* workspace, size_t workspace_bytes, void* stream) {
+  using namespace zgdn;
+  const char* fn = "zgdn_serving_extend";
+  ServeRuns r;
+  if (const int st = serve_runs(fn, tables, n_runs, n_chunks, rows, new_rows, n_slots, &r)) return st;
+  if (!mixed || !x || !conv_weight || !A_log || !dt_bias || !norm_weight || !conv_commit || !conv_live ||
+      !state_commit || !state_live || !window || !win_len || !gated || !workspace)
+    return fail(ZGDN_EINVAL, "%s: null pointer", fn);
+  if (dtype != ZGDN_BF16 || (H != 1 && H != 2 && H != 4 && H != 8 && H != 16) || hidden < 8 || hidden % 8)
+    return fail(ZGDN_EUNSUPPORTED, "%s: bf16, 1, 2, 4, 8 or 16 heads, hidden a multiple of 8 (dtype %d, H=%d, hidden=%d)",
+                fn, dtype, H, hidden);
+  const long inner = (long)H * 128;
+  if (mixed_ld < 4 * inner + 2 * H || mixed_ld % 8)
+    return fail(ZGDN_EINVAL, "%s: in_proj rows of %ld elements (need >= %ld, a multiple of 8)", fn, mixed_ld,
+                4 * inner + 2 * H);
+  if (((uintptr_t)mixed | (uintptr_t)x | (uintptr_t)window | (uintptr_t)gated | (uintptr_t)workspace |
+       (uintptr_t)norm_weight | (uintptr_t)conv_commit | (uintptr_t)conv_live) % 16 || (uintptr_t)conv_weight % 8)
+    return fail(ZGDN_EINVAL, "%s: bases must be 16-byte aligned (the conv weight 8)", fn);
+  if (workspace_bytes < zgdn_serving_extend_workspace(n_chunks, rows, H))
+    return fail(ZGDN_EINVAL, "%s: workspace of %zu bytes, need %zu", fn, workspace_bytes,
+                zgdn_serving_extend_workspace(n_chunks, rows, H));
+  hipStream_t s = (hipStream_t)stream;
+  uint8_t* ws = (uint8_t*)workspace;
+  uint16_t* qkv = (uint16_t*)(ws + (size_t)n_chunks * H * WS_CHUNK);
+  uint16_t* o = qkv + (size_t)rows * 3 * inner;
+  const uint16_t* m = (const uint16_t*)mixed;
+  serve_conv(r, mixed, mixed_ld, conv_weight, conv_commit, conv_live, qkv, H, s);
+  const RowStrides rs{3 * inner, 3 * inner, 3 * inner, mixed_ld, 1};
+  launch_prep<bf16>(true, n_chunks, H, H, qkv, qkv + inner, qkv + 2 * inner, m + 4 * inner, m + 4 * inner + H, A_log,
+                    dt_bias, r.cu, r.pairs, n_runs, rows, scale, 0, rs, ws, s);
+  const int nv = state_nv((long)n_runs * H, device_cus());
+  const dim3 grid((unsigned)((((long)n_runs * H + 7) / 8) * 8 * (DV / VB / nv)));
+  if (nv == 2)
+    hipLaunchKernelGGL(chunk_serve_state_kernel<2>, grid, dim3(64 * P2_WAVES), 0, s, ws, r, state_commit, state_live,
+                       (bf16*)o, H);
+  else
+    hipLaunchKernelGGL(chunk_serve_state_kernel<1>, grid, dim3(64 * P2_WAVES), 0, s, ws, r, state_commit, state_live,
+                       (bf16*)o, H);
+  serve_norm(r, o, m + 3 * inner, mixed_ld, norm_weight, eps, gated, x, hidden, window, win_len, H, s);
+  return check_launch(fn);
 }

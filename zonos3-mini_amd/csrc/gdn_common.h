@@ -193,6 +193,25 @@ struct RowStrides {
   int beta_sigmoid;
 };
 
+// The packed runs of a serving call (device tables, int32): run s holds rows cu[s] .. cu[s + 1] - 1 of the pass,
+// the first replay[s] of them from its slot's window, the others rows xoff[s] .. of the call; it starts from
+// its slot's committed states, or from zeros when fresh[s]. pairs: the (run, chunk) table of the 64-row chunks.
+struct ServeRuns {
+  const int32_t *cu, *pairs, *slots, *replay, *xoff, *fresh;
+  int n_runs, n_chunks, rows, new_rows, n_slots;
+};
+// Chunk `c` of the table as (run, its chunk, its rows, its slot); false where the row names no rows or no slot.
+__device__ __forceinline__ bool serve_chunk(const ServeRuns& r, int c, int& run, int& j, int& bos, int& len, int& slot) {
+  run = r.pairs[2 * c];
+  j = r.pairs[2 * c + 1];
+  if (run < 0 || run >= r.n_runs || j < 0) return false;
+  int eos;
+  seq_bounds(r.cu, run, r.rows, bos, eos);
+  len = eos - bos;
+  slot = r.slots[run];
+  return j < (len + CHUNK_LEN - 1) / CHUNK_LEN && slot >= 0 && slot < r.n_slots;
+}
+
 // -------------------------------------------------------------------------------------------------- math
 
 __device__ __forceinline__ float softplus(float x) { return x > 20.f ? x : log1pf(__expf(x)); }
@@ -210,6 +229,14 @@ namespace zgdn {
 // Records a message for zgdn_last_error() and returns `code`.
 int fail(int code, const char* fmt, ...);
 int check_launch(const char* what);
+
+// The row-local parts of a serving call (gdn_rowops.hip): the conv + SiLU of q|k|v with q and k L2-normalised, from
+// and to the slots' conv caches; the gated norm of the new rows in call order, the slots' windows and lengths.
+void serve_conv(const ServeRuns& r, const void* mixed, long mixed_ld, const void* conv_w, void* conv_commit,
+                void* conv_live, void* qkv, int H, hipStream_t s);
+void serve_norm(const ServeRuns& r, const void* o, const void* z, long z_ld, const void* norm_w, float eps, void* gated,
+                const void* x, int hidden, void* window, int32_t* win_len, int H, hipStream_t s);
+void serve_gather(const ServeRuns& r, const void* x, const void* window, int hidden, void* out, hipStream_t s);
 
 // The fp32-arithmetic chunked path (gdn_chunk_f32.hip): workspace bytes per (chunk, value head) item at head
 // size D, and the forward behind zgdn_chunk_fwd for fp32 q/k/v and for 64-wide heads (arguments checked there).

@@ -413,7 +413,201 @@ __global__ __launch_bounds__(256) void gated_rmsnorm_kernel(const T* __restrict_
   if (rstd != nullptr && lane == 0) rstd[row] = r;
 }
 
+// ------------------------------------------------------------------------------- the serving layer's eager call
+//
+// An eager prefill / extend of the serving layer (servers/sgl/src/zonos3_sgl/models/gdn.py:271-327) runs every
+// request's joined run -- its slot's unfinished chunk, then its new rows -- as one packed sequence, reading and
+// writing the slots' caches in place. The kernels below are its row-local parts; each workgroup finds its rows
+// from the run tables (a few dozen integers), so the host lists no rows. Six requests, 1,067 new rows, hidden 1024:
+// 107 us a call, 65 us of it kernels (two GEMMs 25, phase 1 12, state pass 8, conv 6, norm and gather 4.6 each);
+// through index lists of every row, two passes and some 45 launches of index_select / index_copy / index_fill and
+// the operators 1,074-1,127 us, nearly all of it the host.
+
+constexpr int SV_W = 4;     // conv width, and the width of a slot's conv history
+constexpr int SV_ROWS = 8;  // rows per gather workgroup
+
+// rows of the packed pass from the windows (replayed rows) and the call's rows; hidden elements in 16-byte pieces
+__global__ __launch_bounds__(256) void serve_gather_kernel(const ServeRuns r, const uint4* __restrict__ x,
+                                                           const uint4* __restrict__ window, int row16,
+                                                           uint4* __restrict__ out) {
+  constexpr int SPLIT = CHUNK_LEN / SV_ROWS;
+  int run, j, bos, len, slot;
+  if (!serve_chunk(r, blockIdx.x / SPLIT, run, j, bos, len, slot)) return;
+  const int t0 = j * CHUNK_LEN + (blockIdx.x % SPLIT) * SV_ROWS, n = min(SV_ROWS, len - t0);
+  const int replay = min(max(r.replay[run], 0), CHUNK_LEN), xoff = r.xoff[run];
+  for (int e = threadIdx.x; e < n * row16; e += 256) {
+    const int i = e / row16, c = e - i * row16, t = t0 + i;
+    const int xr = min(max(xoff + t - replay, 0), r.new_rows - 1);
+    const uint4* src = t < replay ? window + ((size_t)slot * CHUNK_LEN + t) * row16 : x + (size_t)xr * row16;
+    out[(size_t)(bos + t) * row16 + c] = src[c];
+  }
+}
+
+// The conv + SiLU of CONV_TT rows of a chunk for 512 channels (two a thread, one head of 128 a wave), with the
+// arithmetic and rounding of conv_kernel; q and k (channels below 2 x 128 H) then L2-normalised in the wave with
+// l2norm128_kernel's order of summation (a quad of lanes holds its eight elements), so both are bit-identical to
+// those two kernels. The tile holding a run's start writes the slot's new histories: the last 4 raw rows of the
+// run (live) and of its complete chunks (committed; untouched when it has none, zeros for a fresh slot).
+__global__ __launch_bounds__(256) void serve_conv_kernel(const ServeRuns r, const bf16* __restrict__ mixed, long ld,
+                                                         const bf16* __restrict__ w, bf16* conv_commit,
+                                                         bf16* __restrict__ conv_live, bf16* __restrict__ qkv, int H) {
+  const int C = 3 * H * 128;
+  const int c0 = (blockIdx.y * 256 + threadIdx.x) * 2;
+  if (c0 >= C) return;  // (whole waves: C is a multiple of 128)
+  int run, j, bos, len, slot;
+  if (!serve_chunk(r, blockIdx.x / CONV_SPLIT, run, j, bos, len, slot)) return;
+  const int t0 = j * CONV_CH + (blockIdx.x % CONV_SPLIT) * CONV_TT;
+  if (t0 >= len) return;
+  const int n = min(CONV_TT, len - t0), last = len - 1;
+  const bool fresh = r.fresh[run] != 0;
+  const uint32_t* col = reinterpret_cast<const uint32_t*>(mixed + (size_t)bos * ld + c0);
+  const long ld2 = ld / 2;  // (rows in channel pairs)
+  auto raw = [&](int t) { return col[(size_t)min(max(t, 0), last) * ld2]; };
+  uint32_t xr[CONV_TT], hx[3];
+#pragma unroll
+  for (int i = 0; i < CONV_TT; ++i) xr[i] = raw(t0 + i);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) hx[i] = raw(t0 - 3 + i);
+  const uint2 w0 = *reinterpret_cast<const uint2*>(w + (size_t)c0 * SV_W);
+  const uint2 w1 = *reinterpret_cast<const uint2*>(w + (size_t)(c0 + 1) * SV_W);
+  if (t0 == 0) {
+    // the rows before the run: the slot's committed history [C][4], oldest first; then the new histories
+    bf16* hc = conv_commit + ((size_t)slot * C + c0) * SV_W;
+    uint2 h0 = *reinterpret_cast<const uint2*>(hc), h1 = *reinterpret_cast<const uint2*>(hc + SV_W);
+    if (fresh) h0 = h1 = make_uint2(0, 0);
+    // old[i]: both channels' history column i
+    const uint32_t old[SV_W] = {(h0.x & 0xffffu) | (h1.x << 16), (h0.x >> 16) | (h1.x & 0xffff0000u),
+                                (h0.y & 0xffffu) | (h1.y << 16), (h0.y >> 16) | (h1.y & 0xffff0000u)};
+#pragma unroll
+    for (int i = 0; i < 3; ++i) hx[i] = old[i + 1];
+    auto put = [&](bf16* dst, int end) {  // the last 4 rows of [history | first `end` rows]
+      uint32_t v[SV_W];
+#pragma unroll
+      for (int i = 0; i < SV_W; ++i) {
+        const int t = end - SV_W + i;
+        uint32_t o = old[SV_W - 1];
+#pragma unroll
+        for (int e = 0; e < SV_W - 1; ++e)
+          if (t + SV_W == e) o = old[e];
+        v[i] = t >= 0 ? raw(t) : o;
+      }
+      bf16* d = dst + ((size_t)slot * C + c0) * SV_W;
+      *reinterpret_cast<uint4*>(d) =
+          make_uint4((v[0] & 0xffffu) | (v[1] << 16), (v[2] & 0xffffu) | (v[3] << 16),
+                     (v[0] >> 16) | (v[1] & 0xffff0000u), (v[2] >> 16) | (v[3] & 0xffff0000u));
+    };
+    put(conv_live, len);
+    const int whole = len - len % CONV_CH;
+    if (whole > 0 || fresh) put(conv_commit, whole);
+  }
+  const float k0[4] = {__uint_as_float(w0.x << 16), __uint_as_float(w0.x & 0xffff0000u), __uint_as_float(w0.y << 16),
+                       __uint_as_float(w0.y & 0xffff0000u)};
+  const float k1[4] = {__uint_as_float(w1.x << 16), __uint_as_float(w1.x & 0xffff0000u), __uint_as_float(w1.y << 16),
+                       __uint_as_float(w1.y & 0xffff0000u)};
+  const bool norm = c0 < 2 * H * 128;  // (wave-uniform)
+  uint32_t win[3] = {hx[0], hx[1], hx[2]};
+#pragma unroll
+  for (int i = 0; i < CONV_TT; ++i) {
+    float a = 0.f, b = 0.f;
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      a = fmaf(k0[m], __uint_as_float(win[m] << 16), a);
+      b = fmaf(k1[m], __uint_as_float(win[m] & 0xffff0000u), b);
+    }
+    a = fmaf(k0[3], __uint_as_float(xr[i] << 16), a);
+    b = fmaf(k1[3], __uint_as_float(xr[i] & 0xffff0000u), b);
+    win[0] = win[1];
+    win[1] = win[2];
+    win[2] = xr[i];
+    uint32_t pk = pack_bf16x2(a, b);
+    pk = pack_bf16x2(silu_fast(__uint_as_float(pk << 16)), silu_fast(__uint_as_float(pk & 0xffff0000u)));
+    if (norm) {
+      const float y0 = __uint_as_float(pk << 16), y1 = __uint_as_float(pk & 0xffff0000u);
+      // sum of squares of the quad's 8 elements in order, then over the 16 quads
+      float ss = 0.f;
+      ss = fmaf(dpp<0x00>(y0), dpp<0x00>(y0), ss);  // quad_perm broadcasts of lanes 0 .. 3
+      ss = fmaf(dpp<0x00>(y1), dpp<0x00>(y1), ss);
+      ss = fmaf(dpp<0x55>(y0), dpp<0x55>(y0), ss);
+      ss = fmaf(dpp<0x55>(y1), dpp<0x55>(y1), ss);
+      ss = fmaf(dpp<0xAA>(y0), dpp<0xAA>(y0), ss);
+      ss = fmaf(dpp<0xAA>(y1), dpp<0xAA>(y1), ss);
+      ss = fmaf(dpp<0xFF>(y0), dpp<0xFF>(y0), ss);
+      ss = fmaf(dpp<0xFF>(y1), dpp<0xFF>(y1), ss);
+      ss += dpp<DPP_ROW_HALF_MIRROR>(ss);
+      ss += dpp<DPP_ROW_MIRROR>(ss);
+      auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(ss), __float_as_uint(ss), false, false);
+      ss = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+      p = __builtin_amdgcn_permlane32_swap(__float_as_uint(ss), __float_as_uint(ss), false, false);
+      ss = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+      const float rn = rsqrtf(ss + 1e-6f);
+      pk = pack_bf16x2(y0 * rn, y1 * rn);
+    }
+    if (i < n) *reinterpret_cast<uint32_t*>(qkv + (size_t)(bos + t0 + i) * C + c0) = pk;
+  }
+}
+
+// The gated norm (gated_rmsnorm128_kernel's arithmetic) of a chunk's rows, 16 head rows a workgroup, written in the
+// order of the call's new rows (replayed rows are dropped), so that wo runs on the new rows alone; the open chunk's
+// new rows also go to the slot's window, and the run's first workgroup sets the window's length.
+__global__ __launch_bounds__(256) void serve_norm_kernel(const ServeRuns r, const bf16* __restrict__ o,
+                                                         const bf16* __restrict__ z, long z_ld,
+                                                         const bf16* __restrict__ w, float eps, bf16* __restrict__ gated,
+                                                         const uint4* __restrict__ x, int row16, uint4* window,
+                                                         int32_t* win_len, int H) {
+  const int per = 16 / H;  // tokens a workgroup (H = 1, 2, 4, 8 or 16)
+  const int split = CHUNK_LEN / per;
+  int run, j, bos, len, slot;
+  if (!serve_chunk(r, blockIdx.x / split, run, j, bos, len, slot)) return;
+  const int t0 = j * CHUNK_LEN + (blockIdx.x % split) * per;
+  const int replay = min(max(r.replay[run], 0), CHUNK_LEN), xoff = r.xoff[run];
+  const int fill = len % CHUNK_LEN, whole = len - fill;
+  if (t0 == 0 && threadIdx.x == 0) win_len[slot] = fill;
+  if (t0 >= len) return;
+  if (t0 >= whole) {
+    const int n = min(per, len - t0);
+    for (int e = threadIdx.x; e < n * row16; e += 256) {
+      const int i = e / row16, c = e - i * row16, t = t0 + i, xr = xoff + t - replay;
+      if (t >= replay && xr >= 0 && xr < r.new_rows)
+        window[((size_t)slot * CHUNK_LEN + t - whole) * row16 + c] = x[(size_t)xr * row16 + c];
+    }
+  }
+  const int hr = threadIdx.x >> 4, sub = threadIdx.x & 15, t = t0 + hr / H, h = hr % H;
+  const int dst = xoff + t - replay;
+  if (t >= len || t < replay || dst < 0 || dst >= r.new_rows) return;  // (whole 16-lane groups)
+  const size_t row = (size_t)(bos + t);
+  const oct<bf16>::raw xw = oct<bf16>::load(o + (row * H + h) * 128 + 8 * sub);
+  const oct<bf16>::raw gw = oct<bf16>::load(z + row * z_ld + h * 128 + 8 * sub);
+  const oct<bf16>::raw ww = oct<bf16>::load(w + 8 * sub);
+  float v[8], gv[8], wv[8];
+  oct<bf16>::unpack(xw, v);
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ss = fmaf(v[i], v[i], ss);
+  const float rn = rsqrtf(group_sum<16>(ss) / 128.f + eps);
+  oct<bf16>::unpack(gw, gv);
+  oct<bf16>::unpack(ww, wv);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = rnd<bf16>(v[i] * rn * wv[i]) * silu(gv[i]);
+  oct<bf16>::store(gated + ((size_t)dst * H + h) * 128 + 8 * sub, v);
+}
+
 }  // namespace
+
+void serve_gather(const ServeRuns& r, const void* x, const void* window, int hidden, void* out, hipStream_t s) {
+  hipLaunchKernelGGL(serve_gather_kernel, dim3(r.n_chunks * (CHUNK_LEN / SV_ROWS)), dim3(256), 0, s, r, (const uint4*)x,
+                     (const uint4*)window, hidden / 8, (uint4*)out);
+}
+void serve_conv(const ServeRuns& r, const void* mixed, long mixed_ld, const void* conv_w, void* conv_commit,
+                void* conv_live, void* qkv, int H, hipStream_t s) {
+  hipLaunchKernelGGL(serve_conv_kernel, dim3(r.n_chunks * CONV_SPLIT, (3 * H * 128 + 511) / 512), dim3(256), 0, s, r,
+                     (const bf16*)mixed, mixed_ld, (const bf16*)conv_w, (bf16*)conv_commit, (bf16*)conv_live, (bf16*)qkv, H);
+}
+void serve_norm(const ServeRuns& r, const void* o, const void* z, long z_ld, const void* norm_w, float eps, void* gated,
+                const void* x, int hidden, void* window, int32_t* win_len, int H, hipStream_t s) {
+  hipLaunchKernelGGL(serve_norm_kernel, dim3(r.n_chunks * CHUNK_LEN * H / 16), dim3(256), 0, s, r, (const bf16*)o,
+                     (const bf16*)z, z_ld, (const bf16*)norm_w, eps, (bf16*)gated, (const uint4*)x, hidden / 8,
+                     (uint4*)window, win_len, H);
+}
 }  // namespace zgdn
 
 extern "C" int zgdn_causal_conv1d_fwd(const void* x, const void* weight, const void* bias, int dtype,

@@ -265,6 +265,11 @@ class launch_form:
         return False
 
 
+def two_launches() -> bool:
+    """Whether the chunked path runs as two launches (the default), not as the overlapped one."""
+    return _native.lib().zgdn_chunk_get_launch_form() != 1
+
+
 def chunk_status(clear: bool = True) -> int:
     """Bits of the chunked path's sticky device status word (0 = no error): ``_native.STATUS_WAIT_GAVE_UP``
     when an overlapped launch's bounded wait ran out, leaving that call's outputs undefined. Synchronises the
@@ -746,3 +751,48 @@ def in_proj_conv(x, w, conv_weight, channels, initial_state=None, output_final_s
     _native.call("zgdn_in_proj_conv", x.data_ptr(), x_ld, w.data_ptr(), y.data_ptr(), N, M, N, K,
                  conv_weight.data_ptr(), C, _ptr(initial_state), _ptr(final), BF16, _stream(dev))
     return y, final
+
+
+def serving_extend(x, in_proj, conv_weight, A_log, dt_bias, norm_weight, conv_commit, conv_live, state_commit,
+                   state_live, window, win_len, tables, n_runs, n_chunks, rows, heads, eps, scale):
+    """The mixer between a serving call's rows and ``wo``, in place on the per-slot caches: the packed runs'
+    rows (gathered from the windows and ``x`` when some run replays rows: ``rows`` > x's), ``in_proj``, conv +
+    SiLU + q/k norm, the chunked delta rule and the gated norm of the new rows in x's order. ``tables``: the int32
+    run tables on the device (``serving.run_tables``). x [new rows, hidden], the weights and the conv caches and
+    window bfloat16, the states float32, as ``serving.OriginalGDN`` holds them. Returns [new rows, heads * 128]."""
+    dev, hidden, new = x.device, x.shape[1], x.shape[0]
+    cap = window.shape[0]
+    inner = heads * 128
+    stream = _stream(dev)
+    bf = torch.bfloat16
+    for name, t, dt in (("x", x, bf), ("conv_weight", conv_weight, bf), ("norm_weight", norm_weight, bf),
+                        ("conv_commit", conv_commit, bf), ("conv_live", conv_live, bf), ("window", window, bf),
+                        ("state_commit", state_commit, torch.float32), ("state_live", state_live, torch.float32),
+                        ("win_len", win_len, torch.int32), ("tables", tables, torch.int32),
+                        ("A_log", A_log, torch.float32), ("dt_bias", dt_bias, torch.float32)):
+        if t.dtype != dt or t.device != dev or not t.is_contiguous():
+            raise RuntimeError(f"{name}: expected contiguous {dt} on {dev}, got {t.dtype} on {t.device}")
+    if (window.shape != (cap, CHUNK, hidden) or conv_commit.shape != (cap, 3 * inner, 4)
+            or conv_live.shape != conv_commit.shape or state_commit.shape != (cap, heads, 128, 128)
+            or state_live.shape != state_commit.shape or win_len.shape != (cap,) or conv_weight.numel() != 12 * inner
+            or norm_weight.shape != (128,) or A_log.shape != (heads,) or dt_bias.shape != (heads,)
+            or tables.numel() != 5 * n_runs + 1 + 2 * n_chunks):
+        raise RuntimeError(f"serving_extend: caches, weights or tables do not fit {cap} slots of {heads} heads, "
+                           f"hidden {hidden}, {n_runs} runs of {n_chunks} chunks")
+    # (16-byte accesses: a slice that starts elsewhere is copied)
+    x, conv_weight, norm_weight = (t.clone() if t.data_ptr() % 16 else t for t in (x, conv_weight, norm_weight))
+    packed = x
+    if rows != new:
+        packed = torch.empty(rows, hidden, device=dev, dtype=bf)
+        _native.call("zgdn_serving_gather", x.data_ptr(), window.data_ptr(), hidden, BF16, tables.data_ptr(), n_runs,
+                     n_chunks, rows, new, cap, packed.data_ptr(), stream)
+    mixed = torch.nn.functional.linear(packed, in_proj)
+    ws_bytes = int(_native.lib().zgdn_serving_extend_workspace(n_chunks, rows, heads))
+    workspace = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
+    gated = torch.empty(new, inner, device=dev, dtype=bf)
+    _native.call("zgdn_serving_extend", mixed.data_ptr(), mixed.stride(0), x.data_ptr(), hidden, BF16, tables.data_ptr(),
+                 n_runs, n_chunks, rows, new, cap, heads, conv_weight.data_ptr(), A_log.data_ptr(), dt_bias.data_ptr(),
+                 norm_weight.data_ptr(), conv_commit.data_ptr(), conv_live.data_ptr(), state_commit.data_ptr(),
+                 state_live.data_ptr(), window.data_ptr(), win_len.data_ptr(), gated.data_ptr(), float(eps), float(scale),
+                 workspace.data_ptr(), ws_bytes, stream)
+    return gated

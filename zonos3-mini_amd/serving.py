@@ -11,7 +11,10 @@ request, and the request's unfinished chunk is kept raw in the slot's 64-row win
 replays it in front of its new rows and prefill/extend/decode cuts never move a chunk boundary.
 
 Design of this module.
-- Eager calls are planned on the host first (``plan_extend``): every request's replayed window rows and
+- Eager prefills and extends of a bf16 layer on this package's own operators run each request's joined run (its
+  unfinished chunk, then its new rows) as one packed sequence, the kernels reading and writing the slots' caches in
+  place from a few numbers a request (``_extend_in_place``).
+- Other eager calls (accent adapters, rebound operators, fp32) are planned on the host first (``plan_extend``): every request's replayed window rows and
   new rows form one joined run, cut after its last complete chunk; the complete part goes to a committed
   pass, the rest to an open pass. The plan is a set of index lists (source rows, output rows, window rows)
   uploaded in one pinned copy; the device work is then one gather per pass, the packed pass itself and one
@@ -207,6 +210,16 @@ def plan_extend(reqs: list[Request]) -> tuple[list[int], PackedPass, PackedPass]
     return replayed, committed, open_
 
 
+def run_tables(reqs: list[Request]) -> tuple[list[int], int, int]:
+    """The tables of an eager call's joined runs for ``ops.serving_extend``, as one flat list -- cu [n + 1], slots,
+    replayed rows, first row in x, fresh flags (n each), then the (run, chunk) pairs -- with the numbers of
+    packed rows and of chunks. Per request and chunk; nothing per row."""
+    cu, pairs = _table_lists([r.replay + r.new for r in reqs])
+    first = list(itertools.accumulate((r.new for r in reqs[:-1]), initial=0))
+    flat = cu + [r.slot for r in reqs] + [r.replay for r in reqs] + first + [int(r.cached == 0) for r in reqs] + pairs
+    return flat, cu[-1], len(pairs) // 2
+
+
 class _Weight:
     def __init__(self, shape):
         self.weight = torch.empty(shape)
@@ -331,19 +344,44 @@ class OriginalGDN:
         if mask is not None:  # a request's adapters: the mask row of its first new row
             firsts = list(itertools.accumulate((r.new for r in reqs[:-1]), initial=0))
             mask = mask.index_select(0, device_tensor(firsts, torch.long, mask.device))
-        fresh = [r.slot for r in reqs if r.cached == 0]
+        in_place = not batch.is_decode and mask is None and self._extends_in_place(x)
+        fresh = [] if in_place else [r.slot for r in reqs if r.cached == 0]
         if fresh:
             self._reset_slots(device_tensor(fresh, torch.long, x.device))
-        if batch.is_decode:
+        if in_place:
+            y = self._extend_in_place(x, reqs)
+        elif batch.is_decode:
             y = self._decode_rows(x, device_tensor([r.slot for r in reqs], torch.long, x.device), mask)
         else:
             y = self._extend(x, reqs, mask)
         for r in reqs:
             self._owners[r.slot] = r.owner
             self._lengths[r.slot] = r.end
-        if not batch.is_decode:
+        if not batch.is_decode and not in_place:  # (the in-place launches wait for nothing)
             self._status_arm()
         return y
+
+    def _extends_in_place(self, x) -> bool:
+        """Whether an eager prefill / extend takes ``_extend_in_place``: a bf16 layer on the GPU with this
+        package's own operators and passes, the two-launch chunked form."""
+        bf = torch.bfloat16
+        return (x.is_cuda and x.dtype == bf and self._conv_state.dtype == bf and self.in_proj.weight.dtype == bf
+                and self.conv.weight.dtype == bf and self._hidden % 8 == 0 and self._own_operators()
+                and "_run_packed" not in self.__dict__ and type(self)._run_packed is OriginalGDN._run_packed
+                and ops.two_launches())
+
+    def _extend_in_place(self, x, reqs: list[Request]):
+        """``_extend`` with each request's joined run as one packed sequence (the open chunk goes on from the
+        complete ones' states in the same pass) and the caches read and written by the kernels themselves, so
+        that the host lists a few numbers a request instead of every row. A fresh slot starts from zeros; its
+        window rows past the fill keep what they held."""
+        flat, rows, n_chunks = run_tables(reqs)
+        gated = ops.serving_extend(
+            x.contiguous(), self.in_proj.weight, self.conv.weight, self.A_log.float(), self.dt_bias.float(),
+            self.out_weight.to(x.dtype), self._conv_state, self._live_conv, self._recurrent_state, self._live_state,
+            self._window, self._win_len, device_tensor(flat, torch.int32, x.device), len(reqs), n_chunks, rows, HEADS,
+            NORM_EPS, HEAD_DIM**-0.5)
+        return F.linear(gated, self.wo.weight)
 
     def _admit(self, batch, rows: int) -> list[Request]:
         """The eager batch's requests after every check (a failed check raises RuntimeError before any
