@@ -124,9 +124,15 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_calls: dict = {}  # entry points that have been called, by name
+
+
 def call(name: str, *args) -> None:
     """Call entry point ``name``; a non-zero status raises RuntimeError with the library's message."""
-    status = getattr(lib(), name)(*args)
+    fn = _calls.get(name)
+    if fn is None:
+        fn = _calls[name] = getattr(lib(), name)
+    status = fn(*args)
     if status != OK:
         msg = lib().zgdn_last_error().decode(errors="replace")
         raise RuntimeError(msg or f"{name} failed with status {status}")

@@ -503,10 +503,7 @@ __global__ __launch_bounds__(64 * W) void attnres_reg_kernel(const SourcePtrs sr
 template <typename T>
 void launch_attnres(const SourcePtrs& p, int n_sources, int tokens, int dim, long row_stride, const void* query,
                     float eps, void* out, hipStream_t stream) {
-  int dev = 0, n_cu = 256;  // the device's CUs, for the token mapping (cu_local_token)
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    n_cu = 256;
-  n_cu = std::max(1, n_cu);
+  const int n_cu = device_cus();  // for the token mapping (cu_local_token)
   const int per = tokens >= n_cu ? (tokens + n_cu - 1) / n_cu : 0;  // tokens per CU (0: one per workgroup)
   const int blocks = per > 0 ? n_cu * per : tokens;
   const int nch = (dim + 511) / 512;

@@ -2,6 +2,8 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <algorithm>
+#include <atomic>
 #include <string>
 
 #include "gdn_common.h"
@@ -27,6 +29,22 @@ int check_launch(const char* what) {
   if (err != hipSuccess) return fail(ZGDN_EHIP, "%s: kernel launch failed: %s", what, hipGetErrorString(err));
   g_last_error.clear();
   return ZGDN_OK;
+}
+
+int device_cus() {
+  constexpr int MAX_DEVICES = 64;
+  static std::atomic<int> cus[MAX_DEVICES];
+  int dev = 0, n = 256;
+  if (hipGetDevice(&dev) != hipSuccess) return n;
+  const bool kept = dev >= 0 && dev < MAX_DEVICES;
+  if (kept) {
+    const int v = cus[dev].load(std::memory_order_relaxed);
+    if (v > 0) return v;
+  }
+  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 256;
+  n = std::max(1, n);
+  if (kept) cus[dev].store(n, std::memory_order_relaxed);
+  return n;
 }
 
 }  // namespace zgdn

@@ -1771,14 +1771,7 @@ std::atomic<int> g_never_ready{0};
 // and the 32-sequence packed batch in 548-559 against 624-634 us.) The overlapped state jobs share their CUs
 // with phase-1 workgroups, which slows their chunk steps by a third, and the faster phase 1 leaves less of its
 // time to hide.
-bool overlap_wanted(bool, long, double, long) { return g_launch_form.load(std::memory_order_relaxed) == 1; }
-
-int device_cus() {
-  int dev = 0, n_cu = 256;
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    n_cu = 256;
-  return std::max(1, n_cu);
-}
+bool overlap_wanted() { return g_launch_form.load(std::memory_order_relaxed) == 1; }
 
 // Queues of the overlapped launch: one per XCD (their L2s are not coherent with each other), or 0 when the
 // device's shape does not allow the launch (an XCD count the control block has no room for, or CUs that do
@@ -1801,13 +1794,11 @@ void launch_prep(bool gate, int nchunks, int Hk, int Hv, const void* q, const vo
                  const int32_t* chunk_idx, int n_seqs, int T, float scale, int qk_l2norm, const RowStrides& rs,
                  uint8_t* ws, hipStream_t stream) {
   // P1_WGS_PER_CU resident workgroups per CU (what the LDS footprint allows), each looping over items
-  int dev = 0, n_cu = 256;
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    n_cu = 256;
+  const int n_cu = device_cus();
   const int n_items = nchunks * Hv;
   // at most one item a CU: one workgroup of 16 waves each (the item's latency is the phase's time)
-  const bool wide = n_items <= std::max(1, n_cu);
-  const dim3 grid(wide ? n_items : std::min(n_items, P1_WGS_PER_CU * std::max(1, n_cu)));
+  const bool wide = n_items <= n_cu;
+  const dim3 grid(wide ? n_items : std::min(n_items, P1_WGS_PER_CU * n_cu));
 #define ZGDN_PREP(GT, WV)                                                                                          \
   hipLaunchKernelGGL((chunk_prep_kernel<TG, GT, WV>), grid, dim3(64 * (WV)), 0, stream, (const uint16_t*)q,       \
                      (const uint16_t*)k, (const uint16_t*)v, (const TG*)g, (const TG*)beta, A_log, dt_bias, cu,    \
@@ -1953,13 +1944,13 @@ int chunk_fwd_impl(const char* fn, const void* q, const void* k, const void* v, 
   // phases 1 and 2 in one overlapped launch where it pays (overlap_wanted): unpacked batches of 8 .. 16 long
   // chains (few-chains order) on the plain pass, packed batches of up to 256 sequences and unpacked batches of more
   // chains (many-chains order)
-  const int n_q = overlap_queues(device_cus(), device_xccs());  // one queue per XCD; 0: no overlapped launch
+  // one queue per XCD; 0: no overlapped launch
+  const int n_q = overlap_wanted() ? overlap_queues(device_cus(), device_xccs()) : 0;
   const long n_chains = (long)N * Hv;
   const bool few = cu_seqlens == nullptr && n_chains <= (long)FQ_FEW_CHAINS * n_q;
   const bool fits = n_q > 0 && (few || ((cu_seqlens == nullptr || N <= FQ_MAX_SEQS) &&
                                          (n_chains + n_q - 1) / n_q <= FQ_MAX_QCHAINS));
-  if (!segmented && n_chunks > 0 && n_q > 0 && n_chains >= n_q && fits &&
-      overlap_wanted(few, (long)n_chunks * Hv, (double)n_chunks / std::max(1, N), (n_chains + n_q - 1) / n_q)) {
+  if (!segmented && n_chunks > 0 && n_q > 0 && n_chains >= n_q && fits) {
     const int n_items = n_chunks * Hv;
     int* ctl_base = reinterpret_cast<int*>(ws + (size_t)n_items * WS_CHUNK);
     const FusedCtl ctl{ctl_base, ctl_base + FQ_CLAIMS, ctl_base + FQ_HEADER / 4, n_q, few ? 1 : 0,

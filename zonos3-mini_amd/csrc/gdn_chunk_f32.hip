@@ -655,10 +655,7 @@ int launch_prep32(const char* fn, int n_items, const void* q, const void* k, con
   constexpr int bytes = Lds32<D>::BYTES;
   if (bytes > 65536 && !lds_ready(chunk32_prep_kernel<TIn, TG, D, GATE>, bytes, state))
     return fail(ZGDN_EHIP, "%s: the device refused %d bytes of LDS for the fp32 chunk kernel", fn, bytes);
-  int dev = 0, n_cu = 256;
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    n_cu = 256;
-  hipLaunchKernelGGL((chunk32_prep_kernel<TIn, TG, D, GATE>), dim3(std::min(n_items, std::max(1, n_cu))),
+  hipLaunchKernelGGL((chunk32_prep_kernel<TIn, TG, D, GATE>), dim3(std::min(n_items, device_cus())),
                      dim3(64 * P32_WAVES), bytes, s, (const TIn*)q, (const TIn*)k, (const TIn*)v, (const TG*)g,
                      (const TG*)beta, A_log, dt_bias, cu, chunk_idx, n_seqs, n_items, T, Hk, Hv, scale, qk_l2norm,
                      rs, ws);

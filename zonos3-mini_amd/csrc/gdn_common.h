@@ -229,6 +229,8 @@ namespace zgdn {
 // Records a message for zgdn_last_error() and returns `code`.
 int fail(int code, const char* fmt, ...);
 int check_launch(const char* what);
+// CUs of the current device (256 when it cannot be asked), asked once per device.
+int device_cus();
 
 // The row-local parts of a serving call (gdn_rowops.hip): the conv + SiLU of q|k|v with q and k L2-normalised, from
 // and to the slots' conv caches; the gated norm of the new rows in call order, the slots' windows and lengths.

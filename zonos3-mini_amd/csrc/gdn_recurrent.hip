@@ -14,6 +14,7 @@
 //   S <- alpha S + delta k
 //   o_j = scale (alpha pq + delta (k.q))            (== S_new . q scale)
 #include <algorithm>
+#include <atomic>
 
 #include "gdn_common.h"
 
@@ -337,11 +338,7 @@ bool launch_step(const RecArgs& a, hipStream_t stream) {
   constexpr int RPP = 64 / (K / 8);
   const long long groups = (long long)a.N * a.Hv * ((a.V + RPP - 1) / RPP);
   if (groups > INT32_MAX) return false;
-  int dev = 0, n_cu = 256;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    n_cu = 256;
-  n_cu = std::max(1, n_cu);
+  const int n_cu = device_cus();
   const bool lean = a.s_in != nullptr && a.s_out != nullptr && a.A_log == nullptr && !a.qk_l2norm &&
                     a.V % RPP == 0;
   const long long tiles4 = (long long)a.N * a.Hv * (a.V / (4 * RPP));
@@ -350,11 +347,18 @@ bool launch_step(const RecArgs& a, hipStream_t stream) {
   auto kernel = tiled  ? step_kernel<TIn, TOut, TG, K, true, 4>
                 : lean ? step_kernel<TIn, TOut, TG, K, true, 1>
                        : step_kernel<TIn, TOut, TG, K, false, 1>;
-  int per_cu = STEP_TILE_WGS_PER_CU;
-  if (!tiled && (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64 * STEP_NWAVES, 0) != hipSuccess ||
-                 per_cu < 1))
-    per_cu = 4;
   const long long all = (n_tiles + STEP_NWAVES - 1) / STEP_NWAVES;  // one item per wave
+  int per_cu = STEP_TILE_WGS_PER_CU;
+  if (!tiled && all > 2LL * n_cu) {  // (fewer workgroups are all launched whatever fits)
+    // what fits on a CU is the kernel's own (registers, LDS): asked once per kernel
+    static std::atomic<int> fits[2];
+    per_cu = fits[lean].load(std::memory_order_relaxed);
+    if (per_cu < 1) {
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64 * STEP_NWAVES, 0) != hipSuccess || per_cu < 1)
+        per_cu = 4;
+      fits[lean].store(per_cu, std::memory_order_relaxed);
+    }
+  }
   long long wgs = std::min<long long>(all, (long long)per_cu * n_cu);
   // single groups: up to two per resident wave would leave some waves one behind the others for a whole
   // group's latency; one group per wave (the hardware queues the rest) finishes sooner there (B=16, H=16)

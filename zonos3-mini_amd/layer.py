@@ -88,7 +88,7 @@ def gdn(self, x: torch.Tensor, layer: int, cache) -> torch.Tensor:
         conv, new_hist = ops.causal_conv1d(qkv.unsqueeze(0), conv_w, initial_state=h0, activation="silu",
                                            state_width=kernel - 1)
         conv2d = conv[0]
-    q, k, v = (part.unflatten(-1, (heads, hd)).unsqueeze(0) for part in conv2d.split(inner, -1))
+    q, k, v = (part.view(1, n, heads, hd) for part in conv2d.split(inner, -1))
     s0 = None if state is None else state.reshape(1, heads, hd, hd).float().contiguous()
     kw = dict(initial_state=s0, A_log=A_log, dt_bias=dt_bias, use_qk_l2norm=True)
     if dt in (torch.bfloat16, torch.float32) and hd in (64, 128):
@@ -99,7 +99,7 @@ def gdn(self, x: torch.Tensor, layer: int, cache) -> torch.Tensor:
         o, new_state = ops.recurrent_fwd(q.contiguous(), k.contiguous(), v.contiguous(),
                                          aa.float().reshape(1, n, heads).contiguous(), beta, out_dtype=dt, **kw)
     recurrent = o.reshape(n, heads, hd).to(dt)
-    gated, _ = ops.gated_rmsnorm(recurrent, z.unflatten(-1, (heads, hd)), norm_w, eps=1e-5)
+    gated, _ = ops.gated_rmsnorm(recurrent, z.view(n, heads, hd), norm_w, eps=1e-5)
     gated = gated.reshape(n, inner)
     cache.conv_state[layer] = new_hist.reshape(channels, kernel - 1)
     cache.gdn_state[layer] = new_state.reshape(heads, hd, hd)
