@@ -410,6 +410,62 @@ __global__ __launch_bounds__(GTHREADS) void gemm_strip_kernel(const uint16_t* __
   }
 }
 
+// Few rows (a decode step's batch): workgroups of 16 rows x 16 columns, K split over the 8 waves in slices of 128
+// (256 bytes of a row; 1,024 of K a pass). Such a call is one round trip to the weights and not a loop over them, so
+// each wave issues all its loads at once: its 16 rows of x and of w as 8 direct-to-LDS loads of 1 KiB (4 rows x 256
+// contiguous bytes each; fragments read straight from memory, 16 rows x 64 bytes an instruction, come in at a third
+// of that rate), physical chunk c of row r holding chunk c ^ (r % 16), so that the 16-row fragment reads meet every
+// bank once. A wave's slice is its own: no barrier before the products. The eight partial tiles are added in LDS in
+// slice order. The row tiles of one column tile run on one XCD (ids equal mod 8) and share its L2 copy of the weights.
+constexpr int SK_WAVES = 8, SK_SLICE = 128, SK_TILE = 16;
+constexpr int SK_BYTES = SK_TILE * SK_SLICE * 2;  // one operand's slice: 4 KiB a wave
+
+__global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const uint16_t* X, long x_ld, const uint16_t* W,
+                                                                    uint16_t* __restrict__ Y, long y_ld, int M, int N,
+                                                                    int K, int tiles_m, int tiles_n) {
+  __shared__ uint4 sk[SK_WAVES * 2 * SK_BYTES / 16];
+  typedef __attribute__((address_space(3))) void* lptr;
+  const int grp = blockIdx.x / (8 * tiles_m), in = blockIdx.x % (8 * tiles_m);
+  const int tn = grp * 8 + in % 8, tm = in / 8;
+  if (tn >= tiles_n) return;
+  const int wave = wave_id(), l = threadIdx.x & 63, m = l & 15, g = l >> 4;
+  const int m0 = tm * SK_TILE, n0 = tn * SK_TILE;
+  const Rsrc rx = raw_rsrc(X + (size_t)m0 * x_ld, (uint32_t)(min(SK_TILE, M - m0) * x_ld * 2));
+  const Rsrc rw = raw_rsrc(W + (size_t)n0 * K, (uint32_t)((size_t)min(SK_TILE, N - n0) * K * 2));
+  uint8_t* xs = reinterpret_cast<uint8_t*>(sk) + wave * 2 * SK_BYTES;
+  uint8_t* ws = xs + SK_BYTES;
+  gf32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int k0 = wave * SK_SLICE; k0 < K; k0 += SK_WAVES * SK_SLICE) {  // (wave-uniform; K a multiple of the slice)
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int r = 4 * p + g, c = m ^ r;  // this lane's row of the piece and the chunk its place holds
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lptr)(ws + 1024 * p), 16, (uint32_t)r * (uint32_t)K * 2u + 16u * c,
+                                               (uint32_t)k0 * 2u, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lptr)(xs + 1024 * p), 16, (uint32_t)r * (uint32_t)x_ld * 2u + 16u * c,
+                                               (uint32_t)k0 * 2u, 0, 0);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int s = 0; s < SK_SLICE / 32; ++s) {
+      const int at = m * 256 + (((4 * s + g) ^ m) << 4);
+      acc = gmfma(*reinterpret_cast<const gbf16x8*>(xs + at), *reinterpret_cast<const gbf16x8*>(ws + at), acc);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the next pass overwrites the slices)
+  }
+  __syncthreads();
+  float* part = reinterpret_cast<float*>(sk);  // [wave][lane][4]
+  *reinterpret_cast<gf32x4*>(part + wave * 256 + 4 * l) = acc;
+  __syncthreads();
+  const int t = threadIdx.x;
+  if (t < 256) {
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < SK_WAVES; ++w) v += part[w * 256 + t];
+    const int r = m0 + 4 * (t >> 6) + (t & 3), c = n0 + ((t >> 2) & 15);
+    if (r < M && c < N) Y[(size_t)r * y_ld + c] = f32_to_bf16(v);
+  }
+}
+
 // n bf16 words of zeros (the history of a call without rows or old history).
 __global__ void zero_u16_kernel(uint16_t* p, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -518,4 +574,18 @@ extern "C" int zgdn_in_proj_conv(const void* x, long x_ld, const void* w, void* 
     return check_launch(fn);
   }
   return gemm_launch<true>(fn, x, x_ld, w, y, y_ld, M, N, K, conv_weight, C, hist_in, hist_out, (hipStream_t)stream);
+}
+
+// y = x w^T for the few rows of a decode step (serving.py): the same operands as zgdn_gemm_nt, K split over the
+// waves, so its sums are taken in another order than zgdn_gemm_nt's.
+extern "C" int zgdn_gemm_rows(const void* x, long x_ld, const void* w, void* y, long y_ld, int M, int N, int K,
+                              int dtype, void* stream) {
+  using namespace zgdn;
+  const char* fn = "zgdn_gemm_rows";
+  const int st = gemm_check(fn, x, x_ld, w, y, y_ld, M, N, K, dtype);
+  if (st != ZGDN_OK || M == 0) return st;
+  const int tm = (M + SK_TILE - 1) / SK_TILE, tn = (N + SK_TILE - 1) / SK_TILE;
+  hipLaunchKernelGGL(gemm_skinny_kernel, dim3((tn + 7) / 8 * 8 * tm), dim3(64 * SK_WAVES), 0, (hipStream_t)stream,
+                     (const uint16_t*)x, x_ld, (const uint16_t*)w, (uint16_t*)y, y_ld, M, N, K, tm, tn);
+  return check_launch(fn);
 }

@@ -828,6 +828,18 @@ def gemm_nt(x, w, out=None):
     return out
 
 
+def gemm_rows(x, w):
+    """x . w^T for the few rows of a decode step: ``gemm_nt``'s operands and precision, K split over a workgroup's
+    waves (sums in another order than ``gemm_nt``'s). Returns y [M, N] bfloat16."""
+    dev = x.device if isinstance(x, torch.Tensor) else None
+    x, x_ld = _gemm_operands("x", x, w, dev)
+    M, K = x.shape
+    N = w.shape[0]
+    out = torch.empty(M, N, device=dev, dtype=torch.bfloat16)
+    _native.call("zgdn_gemm_rows", x.data_ptr(), x_ld, w.data_ptr(), out.data_ptr(), N, M, N, K, BF16, _stream(dev))
+    return out
+
+
 def in_proj_conv(x, w, conv_weight, channels, initial_state=None, output_final_state=True):
     """The GDN layer's in_proj with the depthwise causal conv + SiLU of its q|k|v columns fused in, for one
     sequence (lm.py:561-568; C ABI ``zgdn_in_proj_conv``): y[:, :C] = silu(conv(x . w[:C]^T)) with the width-4

@@ -220,6 +220,22 @@ def run_tables(reqs: list[Request]) -> tuple[list[int], int, int]:
     return flat, cu[-1], len(pairs) // 2
 
 
+# The rows up to which a decode step's projections take the package's split-K kernel. Per call in a graph, us, the
+# kernel / torch's F.linear (MI355X, bf16): in_proj (1024 -> 2056) at 1 row 3.1 / 5.8, 32 rows 3.6 / 8.1, 64 rows
+# 4.4 / 8.5, 128 rows 6.3 / 9.1, 192 rows 8.2 / 8.5, 256 rows 10.1 / 8.9; wo (512 -> 1024) 2.3 / 3.6, 2.5 / 4.8,
+# 2.6 / 5.5, 3.0 / 6.5, 4.0 / 4.9, 4.3 / 6.6.
+FEW_ROWS = 128
+
+
+def _few_rows(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """F.linear(x, w) for a decode step's rows."""
+    if (x.is_cuda and x.shape[0] <= FEW_ROWS and x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2
+            and w.is_contiguous() and x.shape[1] == w.shape[1] and w.shape[1] % 128 == 0 and w.shape[0] % 8 == 0
+            and w.data_ptr() % 16 == 0 and w.device == x.device):
+        return ops.gemm_rows(x, w)
+    return F.linear(x, w)
+
+
 class _Weight:
     def __init__(self, shape):
         self.weight = torch.empty(shape)
@@ -471,7 +487,7 @@ class OriginalGDN:
         row goes to the slot's window, and a window that fills commits the live states."""
         bs = slots.shape[0]
         x = x.contiguous()
-        mixed = F.linear(x, self.in_proj.weight)
+        mixed = _few_rows(x, self.in_proj.weight)
         if mask is not None:
             mixed = self._accent.apply_accent(self.in_proj, x, mixed, mask)
         o = ops.serving_decode_step(mixed, x, slots, self.conv.weight, self._live_conv, self._conv_state,
@@ -479,7 +495,7 @@ class OriginalGDN:
                                     self.out_weight.to(x.dtype), self.A_log.float(), self.dt_bias.float(),
                                     eps=NORM_EPS, scale=HEAD_DIM**-0.5, round_qk=True)
         out = o.reshape(bs, HEADS * HEAD_DIM)
-        y = F.linear(out, self.wo.weight)
+        y = _few_rows(out, self.wo.weight)
         if mask is not None:
             y = self._accent.apply_accent(self.wo, out, y, mask)
         return y
