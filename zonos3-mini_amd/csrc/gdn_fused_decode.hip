@@ -69,6 +69,19 @@ struct FusedArgs {
   int qk_round;
 };
 
+// One conv channel's inputs as loaded (the history's last 3 columns, the taps, the new input) and as floats.
+template <typename T, int CW>
+struct ConvIn {
+  T x, h[FD_W - 1], w[FD_W];
+  __device__ __forceinline__ void load(const T* xp, const T* hist, const T* wp) {
+    x = *xp;
+#pragma unroll
+    for (int i = 0; i < FD_W - 1; ++i) h[i] = hist[CW - (FD_W - 1) + i];
+#pragma unroll
+    for (int i = 0; i < FD_W; ++i) w[i] = wp[i];
+  }
+};
+
 // Channel of the group's i-th conv channel: q, k of key head hk, then the v of value heads hk*G ..
 __device__ __forceinline__ int conv_channel(int i, int hk, int Hk, int G) {
   if (i < FD_K) return hk * FD_K + i;
@@ -89,23 +102,33 @@ __global__ __launch_bounds__(64 * FD_WAVES) void fused_decode_kernel(const Fused
 
   const int Hk = p.Hk, Hv = p.Hv;
   const int bs = blockIdx.x / Hk, hk = blockIdx.x % Hk;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   long srow = bs;
+  int dup = 0;
   if constexpr (SERVING) {
     srow = p.slots[bs];
-    if (srow < 0 || srow >= p.n_rows) return;  // a slot outside the caches: nothing is read or written
     // A slot named again later in the batch (padded graph replays repeat one spare slot) is served by its
-    // first stream only: the later ones read and write nothing, so every slot sees exactly Hk arrivals below
-    // and its window-length word keeps only the length.
-    int dup = 0;
-    for (int i = threadIdx.x; i < bs; i += blockDim.x) dup |= p.slots[i] == srow;
-    if (__syncthreads_or(dup)) return;
+    // first stream only: the later ones write nothing, so every slot sees exactly Hk arrivals below and its
+    // window-length word keeps only the length. (Looked up here beside the slot itself, judged below, where the
+    // loads of the step are in flight.)
+    for (int i = tid; i < bs; i += 64 * FD_WAVES) dup |= p.slots[i] == srow;
+    if (srow < 0 || srow >= p.n_rows) return;  // a slot outside the caches: nothing is read or written
   }
   const size_t row = (size_t)srow;
   const int C = 2 * Hk * FD_K + Hv * FD_K;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int sub = lane % FD_LPR, rsub = lane / FD_LPR;
   const int c0 = sub * 4, c1 = FD_K / 2 + sub * 4;
-  // 0. issue the state loads of this lane's rows (row r = pass * 32 + wave * 4 + rsub; head r / 128)
+  // 0. issue the conv's loads, then the state's (row r = pass * 32 + wave * 4 + rsub; head r / 128): loads come back
+  // in order, so the conv, the norms and the gate run while the state is on its way (with the state's first, and the
+  // serving step's slot lookups a round trip of their own ahead: 19.7 against 19.1 us for a decode step of 32
+  // requests, 8.1 against 7.7 us this kernel; at 256 streams the state's bytes bound it either way, 111 us)
+  constexpr int NCI = (NCH + 64 * FD_WAVES - 1) / (64 * FD_WAVES);
+  ConvIn<T, CW> ci[NCI];
+#pragma unroll
+  for (int q = 0; q < NCI; ++q) {
+    const int ch = conv_channel(min(tid + q * 64 * FD_WAVES, NCH - 1), hk, Hk, G);
+    ci[q].load(p.x + bs * p.x_ld + ch, p.conv_cache + (row * C + ch) * CW, p.conv_w + (size_t)ch * FD_W);
+  }
   const size_t group_off = (row * Hv + (size_t)hk * G) * FD_K * FD_K;
   float* sgroup = p.state + group_off;
   float s[PASSES][8];
@@ -117,6 +140,9 @@ __global__ __launch_bounds__(64 * FD_WAVES) void fused_decode_kernel(const Fused
     s[q][0] = u.x; s[q][1] = u.y; s[q][2] = u.z; s[q][3] = u.w;
     s[q][4] = w.x; s[q][5] = w.y; s[q][6] = w.z; s[q][7] = w.w;
   }
+  if constexpr (SERVING) {
+    if (__syncthreads_or(dup)) return;
+  }
   // The slot's window length, advanced in the same launch: workgroup hk of the slot adds 1 << 16 (an arrival
   // count above the length, which stays below 2^16) and takes the length from the low bits of the old value;
   // the last of the slot's Hk arrivals stores the new length (win_len + 1) % window_rows with the count
@@ -127,23 +153,22 @@ __global__ __launch_bounds__(64 * FD_WAVES) void fused_decode_kernel(const Fused
     old_len = __hip_atomic_fetch_add(p.win_len + row, 1 << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
   // 1. conv + SiLU of the group's channels; the history rolls by one (the oldest input drops out)
-  for (int i = tid; i < NCH; i += 64 * FD_WAVES) {
+#pragma unroll
+  for (int q = 0; q < NCI; ++q) {
+    const int i = tid + q * 64 * FD_WAVES;
+    if (i >= NCH) break;
     const int ch = conv_channel(i, hk, Hk, G);
-    const size_t hc = (row * C + ch) * CW;
-    T* hist = p.conv_cache + hc + (CW - (FD_W - 1));  // the taps' history: the last W-1 columns
-    const float xv = io<T>::load(p.x + bs * p.x_ld + ch);
-    const float h0 = io<T>::load(hist), h1 = io<T>::load(hist + 1), h2 = io<T>::load(hist + 2);
-    const T* w = p.conv_w + (size_t)ch * FD_W;
-    float acc = io<T>::load(w) * h0;
-    acc = fmaf(io<T>::load(w + 1), h1, acc);
-    acc = fmaf(io<T>::load(w + 2), h2, acc);
-    acc = fmaf(io<T>::load(w + 3), xv, acc);
+    const ConvIn<T, CW>& in = ci[q];
+    float acc = io<T>::load(&in.w[0]) * io<T>::load(&in.h[0]);
+    acc = fmaf(io<T>::load(&in.w[1]), io<T>::load(&in.h[1]), acc);
+    acc = fmaf(io<T>::load(&in.w[2]), io<T>::load(&in.h[2]), acc);
+    acc = fmaf(io<T>::load(&in.w[3]), io<T>::load(&in.x), acc);
     s_conv[i] = round_to<T>(silu(round_to<T>(acc)));
-    T* dst = p.conv_cache + hc;
-    if constexpr (CW == FD_W) io<T>::store(dst++, h0);  // a full-width history keeps h0 as its oldest input
-    io<T>::store(dst, h1);
-    io<T>::store(dst + 1, h2);
-    io<T>::store(dst + 2, xv);
+    T* dst = p.conv_cache + (row * C + ch) * CW;
+    if constexpr (CW == FD_W) *dst++ = in.h[0];  // a full-width history keeps it as its oldest input
+    dst[0] = in.h[1];
+    dst[1] = in.h[2];
+    dst[2] = in.x;
   }
   if (tid < G) {
     const int h = hk * G + tid;
