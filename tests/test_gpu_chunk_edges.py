@@ -1,0 +1,30 @@
+"""The bf16 chunk kernels at the edges of the state pass's loops (1, 2, 3 and 4 chunks, full and partial last ones) in
+both of its forms -- one value block a workgroup with output waves (few chains), two blocks without (many) -- and
+under decays so strong that a chunk's total decay leaves fp32's range (the outputs' products must not pass through
+factors like exp(G_i - G_L)). Tolerances of the bf16 path: outputs 2e-2 max-abs, states 1e-3 relative."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from gdn_testing import announce, max_abs, rel_err
+from oracle import gdn_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("decay", [1.0, 4.0])
+@pytest.mark.parametrize("H", [2, 16])
+@pytest.mark.parametrize("lengths", [[64, 1, 63], [65, 128, 129], [192, 193, 256, 0, 2]])
+def test_chunk_counts_and_strong_decay(gdn, cuda, lengths, H, decay):
+    announce(f"chunk edges {lengths} H={H} decay x{decay}")
+    cu, _ = O.chunk_tables(lengths)
+    d = O.make_inputs(1, sum(lengths), H, H, 128, 128, seed=900 + H + sum(lengths), dtype=torch.bfloat16,
+                      state_std=0.02, n_states=len(lengths))
+    g = d["g"] * decay  # about -0.8 a token: a chunk's G_L about -52, times 4 about -206 (exp(103) overflows)
+    o, s = gdn.chunk_fwd(*(t.to(cuda) for t in (d["q"], d["k"], d["v"], g, d["beta"])), initial_state=d["s0"].to(cuda),
+                         cu_seqlens=torch.tensor(cu, dtype=torch.int32, device=cuda))
+    torch.cuda.synchronize()
+    o_ref, s_ref = O.gated_delta_recurrence(d["q"], d["k"], d["v"], g, d["beta"], None, d["s0"], cu_seqlens=cu)
+    assert max_abs(o, o_ref) < 2e-2 and rel_err(s, s_ref) < 1e-3, (max_abs(o, o_ref), rel_err(s, s_ref))

@@ -7,18 +7,22 @@
 //   Ub = diag(beta) V + (T - I) diag(beta) V                        [L x V]   (diagonal exact in fp32)
 //   P  = s * lower-incl( exp(G_i - G_j) q_i.k_j )                   [L x L]
 //   U  = Ub - W S0^T                                                (the corrected values)
-//   O  = s diag(exp(G)) Q S0^T + P U  =  Q' S0^T + Ob,   Q' = s diag(exp(G)) Q - P W,   Ob = P Ub
-//   S  = exp(G_L) S0 + U'^T K,   U' = diag(exp(G_L - G)) U = Ub' - W' S0^T  (Ub', W' the rows of Ub, W scaled)
-// Phase 1 (chunk_prep_kernel, one item per chunk x head, all independent) forms W', Q', K^T, Ub', Ob and
-// G_L into a workspace. Phase 2 (chunk_state_kernel, one workgroup per sequence x head x 16 value rows) walks
-// the chunks in order keeping its 16 x 128 slice of the fp32 state in registers: one MFMA pass over [W'; Q']
-// gives U' and the outputs, a second the state update. Only the state pass is sequential, so the workspace is
+//   O  = Q' S0^T + P U,   Q' = s diag(exp(G)) Q
+//   S  = exp(G_L) S0 + U'^T K,   U' = diag(exp(G_L - G)) U
+// Phase 1 (chunk_prep_kernel, one item per chunk x head, all independent) forms W, Q', K^T, Ub, P, the scale of U'
+// and G_L into a workspace. Phase 2 (chunk_state_kernel, one workgroup per
+// sequence x head x 16 value rows) walks the chunks in order keeping its 16 x 128 slice of the fp32 state in
+// registers: one MFMA pass over [W; Q'] gives U and the outputs' state part, a second the state update and P U.
+// (With the outputs' parts that need no state formed ahead, P Ub and P W: 112 more products and two more phases an
+// item, 10 KiB more written and read, for 2 products a chunk less in the state pass. T = 4096 at 16 heads: phase 1
+// 29.7 us against 25.7, the state pass 41.8 against 43.9; 32 packed sequences of 30,526 tokens at 16 heads 217 and 263
+// us against 200 and 254.) Only the state pass is sequential, so the workspace is
 // stored in MFMA fragment order: every phase-2 operand load is one contiguous 1 KiB per wave (rows read
 // straight from row-major matrices cost about 2.3x as much per byte on CDNA), and the next chunk's loads are
 // issued in three groups spread over the current chunk so they overlap its MFMA and LDS work.
 // Numerics: MFMA operands are bf16 with fp32 accumulation; U' enters the state update as a hi + lo bf16 pair
 // (two MFMAs) and the diagonal of T diag(beta) is applied in fp32, which keeps the fp32 state within ~1e-4 of
-// the exact recurrence; the output path (Q', Ob, S in bf16) stays within ~1e-3 of |o|.
+// the exact recurrence; the output path (Q', P, U, S in bf16) stays within ~1e-3 of |o|.
 //
 // With the q/k L2-norm fused in (lm.py:570-571), q_t = rq_t cq_t and k_t = rk_t ck_t where cq, ck are the
 // raw (exactly bf16) rows and rq, rk = rsqrt(sum c^2 + 1e-6) are fp32: every factor r is folded into the
@@ -27,8 +31,8 @@
 //
 // MFMA used: v_mfma_f32_16x16x32_bf16 (A: row lane%16, k 8*(lane/16)+0..7; B: column lane%16, same k;
 // D: row 4*(lane/16)+i, column lane%16) and v_mfma_f32_16x16x4_f32 (A[lane%16][lane/16], B[lane/16][lane%16])
-// for the fp32 block inverse. The contraction index of the [W'; Q'] S^T pass is taken in a permuted key order
-// (kappa below) so that two 16 x 16 D tiles of W'^T computed in phase 1 are directly one A fragment.
+// for the fp32 block inverse. The contraction index of the [W; Q'] S^T pass is taken in a permuted key order
+// (kappa below) so that two 16 x 16 D tiles of W^T computed in phase 1 are directly one A fragment.
 #include <type_traits>
 #include <algorithm>
 #include <atomic>
@@ -61,22 +65,25 @@ constexpr int LDF = CH + 4;  // padded LDS row (fp32) of a 64-wide matrix
 
 // Workspace of one chunk x head (bytes), every block in the register order of the phase-2 wave that reads it.
 // Token tile tb = 16 tokens, value block vb = 16 value rows, k-step kk = 32 keys; lane l:
-//   W'  [tb][kk][l] 8 bf16: W'[16 tb + l%16][kappa(kk, l, 0..7)]        (A fragments, U role)
+//   W   [tb][kk][l] 8 bf16: W[16 tb + l%16][kappa(kk, l, 0..7)]         (A fragments, U role)
 //   Q'  [tb][kk][l] 8 bf16: Q'[16 tb + l%16][kappa(kk, l, 0..7)]        (A fragments, O role)
 //   K^T [w][kk][l]  8 bf16: k[32 kk + 8 (l/16) + 0..7][16 w + l%16]     (B fragments of the state update)
-//   Ub' [vb][tb][l] 4 f32 : Ub'[16 tb + 4 (l/16) + i][16 vb + l%16]     (D tiles)
-//   Ob  [vb][tb][l] 4 bf16: Ob[16 tb + 4 (l/16) + i][16 vb + l%16]      (D tiles)
-//   G_L, then padding to a 256-byte multiple.
+//   Ub  [vb][tb][l] 4 f32 : Ub[16 tb + 4 (l/16) + i][16 vb + l%16]      (D tiles)
+//   P   [tb][kk][l] 8 bf16: P[16 tb + l%16][32 kk + 8 (l/16) + 0..7], kk < 2 (A fragments; kk = 1 of the first two
+//                           token tiles is zero and not held)
+//   Fk [64] f32: exp(G_L - G_t) rk_t;  G_L
 // kappa(kk, l, i) = 32 kk + 4 (l/16) + i for i < 4 and 32 kk + 16 + 4 (l/16) + i - 4 for i >= 4.
 // (Phase 1 keeps the k and v rows row-major in LDS and reads the K^T / V^T operands with transposing LDS
-// reads.)
+// reads.) A slot is larger than its blocks: 98,560 bytes are what zgdn_chunk_workspace_size tells callers.
 constexpr size_t WS_WP = 0;
 constexpr size_t WS_QP = WS_WP + CH * DK * 2;
 constexpr size_t WS_KT = WS_QP + CH * DK * 2;
 constexpr size_t WS_UB = WS_KT + DK * CH * 2;
-constexpr size_t WS_OB = WS_UB + CH * DV * 4;
-constexpr size_t WS_GL = WS_OB + CH * DV * 2;
-constexpr size_t WS_CHUNK = WS_GL + 256;  // 98,560 bytes
+constexpr size_t WS_P = WS_UB + CH * DV * 4;
+constexpr size_t WS_F = WS_P + CH * CH * 2;
+constexpr size_t WS_GL = WS_F + CH * 4;
+constexpr size_t WS_CHUNK = 98560;
+static_assert(WS_GL + 4 <= WS_CHUNK, "workspace slot");
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
 
@@ -127,7 +134,7 @@ __device__ __forceinline__ int tri_kend(int tb) { return tb < 2 ? 32 : 64; }
 
 // ----------------------------------------------------------------------------------------------- phase 1
 //
-// One item = one (chunk, value head): W', Q', K^T, Ub', Ob and G_L of the chunk into its workspace. Persistent
+// One item = one (chunk, value head): W, Q', K^T, Ub, P, Fk and G_L of the chunk into its workspace. Persistent
 // workgroups of 8 waves, two per CU (75,776 bytes of LDS each), loop over items. The item is laid out for few
 // VALU instructions and a short dependent chain:
 // * every LDS access is a per-lane offset formed once plus a compile-time or wave-uniform part: the XOR
@@ -137,7 +144,7 @@ __device__ __forceinline__ int tri_kend(int tb) { return tb < 2 ? 32 : 64; }
 // * a D tile is stored transposed (row n of X^T holds the tile's 4 rows of column n: one 16-byte fp32 or 8-byte
 //   bf16 write a lane), and its consumers read X's row fragments with transposing reads (ds_read_b64_tr_b16:
 //   within 16 lanes, lane s names row k0 + s/4, columns c0 + 4 (s%4) .. + 3, and lane i receives column c0 + i
-//   of the 4 rows) or take X^T's rows: A^T, P^T, T^T, (diag(Fk) T diag(Bk))^T, ((T - I) diag(beta))^T, R^T, Ub^T;
+//   of the 4 rows) or take X^T's rows: A^T, P^T, T^T, (T diag(Bk))^T, ((T - I) diag(beta))^T;
 // * the rows are read with buffer loads (a scalar base per item; rows past the chunk end fall outside the
 //   buffer range and read zero), the next item's rows in flight while the current item computes;
 // * the diagonal 16x16 blocks of T = (I + A)^-1 are inverted by one wave by right-looking substitution from rows
@@ -156,11 +163,8 @@ __device__ __forceinline__ int tri_kend(int tb) { return tb < 2 ? 32 : 64; }
 constexpr int PS_Q = 0;            // raw q rows [64][128] bf16 (256-byte rows)        } one 32 KiB region,
 constexpr int PS_AT = 0;           // A^T, then N^T in its blocks, fp32 [64][64]        } reused by phase
 constexpr int PS_TT = 16384;       // T^T fp32 (logical blocks (0, 1..3): pair products)
-constexpr int PS_TBF = 0;          // (diag(Fk) T diag(Bk))^T bf16 [64][64] (128-byte rows)
-constexpr int PS_TBT = 8192;       // (T diag(Bk))^T
+constexpr int PS_TBT = 8192;       // (T diag(Bk))^T bf16 [64][64] (128-byte rows)
 constexpr int PS_LB = 16384;       // ((T - I) diag(beta))^T
-constexpr int PS_RT = 24576;       // R^T
-constexpr int PS_UBT = 0;          // Ub^T bf16 [128][64]
 constexpr int PS_K = 32768;        // k rows [64][128] bf16
 constexpr int PS_V = 49152;        // v rows
 constexpr int PS_PT = 65536;       // P^T bf16 [64][64]; the blocks of zeros above P's diagonal blocks set once
@@ -379,12 +383,10 @@ __device__ __forceinline__ void prep_init(uint8_t* lb) {
 __device__ __forceinline__ void item_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // One phase-1 item (`it`). `R` holds the item's rows (loaded by the caller); with `has_next`, the rows of item
-// `nx` are loaded into R while this one computes. QL: the raw q of the Q' step is taken from the q rows in LDS
-// (held in registers from step 2 on; no second read of q from memory), else read again from memory before step
-// 6 (fewer registers held: the overlapped kernel's budget). W: the workgroup's waves, 8 (two workgroups a CU) or
-// 16 (one item a CU when the items are few: the phases spread over twice the waves, the item's latency
-// shorter). Ends with a workgroup barrier.
-template <typename TG, bool GATE, bool QL, int W>
+// `nx` are loaded into R while this one computes. W: the workgroup's waves, 8 (two workgroups a CU) or 16 (one
+// item a CU when the items are few: the phases spread over twice the waves, the item's latency shorter). Ends
+// with a workgroup barrier.
+template <typename TG, bool GATE, int W>
 __device__ __forceinline__ void prep_item(uint8_t* lb, const ItemAt& it, RowRegs& R, bool has_next, const ItemAt& nx,
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const TG* __restrict__ g, const TG* __restrict__ beta, const float* __restrict__ A_log,
@@ -481,18 +483,16 @@ __device__ __forceinline__ void prep_item(uint8_t* lb, const ItemAt& it, RowRegs
       F[(PSF_BK >> 2) + r] = br * __expf(gr) * rf;
     }
   }
-  // raw q of this wave's Q' jobs (step 8): token 16 tb + m, columns 32 kq + 4 gq .. + 3 and 16 further; with QL
-  // from the q rows, before A^T overwrites them (rows past the chunk end hold zeros)
+  // raw q of this wave's q fragments (token tile tb, key step kq: columns 32 kq + 4 gq .. + 3 and 16 further of token
+  // 16 tb + m), from the q rows, before A^T overwrites them (rows past the chunk end hold zeros)
   uint2 cq[NJ16][2];
-  if constexpr (QL) {
 #pragma unroll
-    for (int n = 0; n < NJ16; ++n) {
-      const int job = wave + W * n, tb = job >> 2, kq = job & 3;
-      const int tok = 16 * tb + m, cc = 4 * kq + (gq >> 1);
-      const int at = PS_Q + tok * 256 + 8 * (gq & 1);
-      cq[n][0] = lds_at<uint2>(lb, at + ((cc ^ m) << 4));
-      cq[n][1] = lds_at<uint2>(lb, at + (((cc + 2) ^ m) << 4));
-    }
+  for (int n = 0; n < NJ16; ++n) {
+    const int job = wave + W * n, tb = job >> 2, kq = job & 3;
+    const int tok = 16 * tb + m, cc = 4 * kq + (gq >> 1);
+    const int at = PS_Q + tok * 256 + 8 * (gq & 1);
+    cq[n][0] = lds_at<uint2>(lb, at + ((cc ^ m) << 4));
+    cq[n][1] = lds_at<uint2>(lb, at + (((cc + 2) ^ m) << 4));
   }
   f32x4 acc[4];
   int jrb[NJ], jcb[NJ];
@@ -533,6 +533,17 @@ __device__ __forceinline__ void prep_item(uint8_t* lb, const ItemAt& it, RowRegs
     }
   }
   item_barrier();  // A^T overwrites the q rows; the factors are visible
+  // Q' = Fq q (as A fragments)
+  {
+    uint4* gQ = reinterpret_cast<uint4*>(wsc + WS_QP);
+#pragma unroll
+    for (int n = 0; n < NJ16; ++n) {
+      const int job = wave + W * n, tb = job >> 2, kq = job & 3;
+      const float fq = F[(PSF_FQ >> 2) + 16 * tb + m];
+      auto sc = [&](uint32_t w) { return pack_bf16x2(fq * __uint_as_float(w << 16), fq * __uint_as_float(w & 0xffff0000u)); };
+      gQ[(tb * 4 + kq) * 64 + l] = make_uint4(sc(cq[n][0].x), sc(cq[n][0].y), sc(cq[n][1].x), sc(cq[n][1].y));
+    }
+  }
 
   // 3. scaled tiles -> A^T (fp32) and P^T (bf16); wave 0: the diagonal blocks, then their inverse
   // A_ij = beta_i rk_i exp(G_i - G_j) rk_j k_i.k_j (i > j), P_ij = s rq_i exp(G_i - G_j) rk_j q_i.k_j (i >= j),
@@ -620,8 +631,8 @@ __device__ __forceinline__ void prep_item(uint8_t* lb, const ItemAt& it, RowRegs
   item_barrier();
 
   // 5. bf16 forms, row by row of T^T (row j = column j of T; 8 columns i0 .. i0 + 7 a thread):
-  // TBF^T[j][i] = Fk_i T_ij... = Fk_i T[i][j] Bk_j, TBT[j][i] = T[i][j] Bk_j, LB^T[j][i] = (T - I)[i][j] beta_j;
-  // T's blocks above its diagonal blocks (pair products there) are zero
+  // TBT[j][i] = T[i][j] Bk_j, LB^T[j][i] = (T - I)[i][j] beta_j; T's blocks above its diagonal blocks (pair
+  // products there) are zero
   {
     const bool act = W == 8 || tid < 512;  // (512 threads: 8 a row of T^T)
     const int j = (tid >> 3) & 63, i0 = (tid & 7) * 8;
@@ -629,43 +640,24 @@ __device__ __forceinline__ void prep_item(uint8_t* lb, const ItemAt& it, RowRegs
     f32x4 t0 = lds_at<f32x4>(lb, rd), t1 = lds_at<f32x4>(lb, rd ^ 16);
     if ((i0 >> 4) < (j >> 4)) t0 = t1 = zero4();
     const float bkj = F[(PSF_BK >> 2) + j], bj = F[(PSF_B >> 2) + j];
-    const f32x4 fk0 = lds_at<f32x4>(lb, PS_F + PSF_FK + 4 * i0), fk1 = lds_at<f32x4>(lb, PS_F + PSF_FK + 4 * i0 + 16);
     const float tv[8] = {t0[0], t0[1], t0[2], t0[3], t1[0], t1[1], t1[2], t1[3]};
-    const float fk[8] = {fk0[0], fk0[1], fk0[2], fk0[3], fk1[0], fk1[1], fk1[2], fk1[3]};
-    uint32_t wf[4], wt[4], wl[4];
+    uint32_t wt[4], wl[4];
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
-      const float b0 = tv[2 * p] * bkj, b1 = tv[2 * p + 1] * bkj;
-      wf[p] = pack_bf16x2(fk[2 * p] * b0, fk[2 * p + 1] * b1);
-      wt[p] = pack_bf16x2(b0, b1);
+      wt[p] = pack_bf16x2(tv[2 * p] * bkj, tv[2 * p + 1] * bkj);
       wl[p] = pack_bf16x2(i0 + 2 * p == j ? 0.f : tv[2 * p] * bj, i0 + 2 * p + 1 == j ? 0.f : tv[2 * p + 1] * bj);
     }
     item_barrier();  // the forms overwrite T^T and A^T
     const int wr = j * 128 + ((((tid & 7) ^ ((j >> 1) & 7))) << 4);
     if (act) {
-      lds_put<uint4>(lb, PS_TBF + wr, make_uint4(wf[0], wf[1], wf[2], wf[3]));
       lds_put<uint4>(lb, PS_TBT + wr, make_uint4(wt[0], wt[1], wt[2], wt[3]));
       lds_put<uint4>(lb, PS_LB + wr, make_uint4(wl[0], wl[1], wl[2], wl[3]));
     }
   }
   item_barrier();
 
-  if constexpr (!QL) {
-#pragma unroll
-    for (int n = 0; n < NJ16; ++n) {
-      const int job = wave + W * n, tb = job >> 2, kq = job & 3;
-      const int tok = 16 * tb + m;
-      cq[n][0] = cq[n][1] = make_uint2(0, 0);
-      if (tok < cr.len) {
-        const uint16_t* qrow = q + (size_t)(cr.t0 + tok) * rs.q + hk * DK + 32 * kq + 4 * gq;
-        cq[n][0] = *reinterpret_cast<const uint2*>(qrow);
-        cq[n][1] = *reinterpret_cast<const uint2*>(qrow + 16);
-      }
-    }
-  }
-
-  // 6. W'^T = K^T TBF^T (A fragments to the workspace), R = P TB (as R^T; R's blocks above its diagonal
-  // blocks zero), the K^T fragments
+  // 6. to the workspace: W^T = K^T TBT^T (as A fragments), the K^T and P fragments, the factors, Ub = beta V + LB V
+  // (fp32 D tiles)
   {
     uint4* gW = reinterpret_cast<uint4*>(wsc + WS_WP);
 #pragma unroll
@@ -675,29 +667,11 @@ __device__ __forceinline__ void prep_item(uint8_t* lb, const ItemAt& it, RowRegs
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk)
         if (kk < nk) {
-          const bf16x8 bf = pfragT8(lb, PS_TBF, 16 * tb, kk, L);
+          const bf16x8 bf = pfragT8(lb, PS_TBT, 16 * tb, kk, L);
           d0 = mfma(pfragT16(lb, PS_K, 32 * kq, kk, L), bf, d0);
           d1 = mfma(pfragT16(lb, PS_K, 32 * kq + 16, kk, L), bf, d1);
         }
       gW[(tb * 4 + kq) * 64 + l] = kappa_frag(d0, d1);
-    }
-#pragma unroll
-    for (int n = 0; n < NJ16; ++n) {  // R tiles: jobs 0-9 the lower tiles, 10-15 zero tiles above
-      const int job = wave + W * n;
-      int rb, cb;
-      if (job < 10) {
-        lower_tile(job, rb, cb);
-        f32x4 r = zero4();
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk)
-          if (kk < tri_kend(rb) / 32) r = mfma(pfragT8(lb, PS_PT, 16 * rb, kk, L), pfrag8(lb, PS_TBT, 16 * cb, kk, L), r);
-        put_t16(lb, PS_RT, rb, cb, L, r);
-      } else {
-        const int t = job - 10;  // (rb, cb) with rb < cb: (0,1) (0,2) (1,2) (0,3) (1,3) (2,3)
-        cb = t < 1 ? 1 : (t < 3 ? 2 : 3);
-        rb = t - cb * (cb - 1) / 2;
-        put_t16(lb, PS_RT, rb, cb, L, zero4());
-      }
     }
     uint4* gKT = reinterpret_cast<uint4*>(wsc + WS_KT);
 #pragma unroll
@@ -705,11 +679,15 @@ __device__ __forceinline__ void prep_item(uint8_t* lb, const ItemAt& it, RowRegs
       const int f = wave + W * n;
       gKT[f * 64 + l] = __builtin_bit_cast(uint4, pfragT16(lb, PS_K, 16 * (f >> 1), f & 1, L));
     }
-  }
-  item_barrier();  // Ub^T overwrites TBF, TBT
-
-  // 7. Ub = beta V + LB V: Ub' = Fk Ub (fp32 D tiles) to the workspace, Ub^T (bf16) to LDS
-  {
+    if (wave < 6) {  // P's six fragments: (0, 0), (1, 0), (2, 0), (2, 1), (3, 0), (3, 1)
+      const int tb = wave < 2 ? wave : 2 + ((wave - 2) >> 1), kk = wave < 2 ? 0 : (wave & 1);
+      reinterpret_cast<uint4*>(wsc + WS_P)[(tb * 2 + kk) * 64 + l] =
+          __builtin_bit_cast(uint4, pfragT8(lb, PS_PT, 16 * tb, kk, L));
+    } else if (wave == 6) {
+      float* gF = reinterpret_cast<float*>(wsc + WS_F);
+      gF[l] = F[(PSF_FK >> 2) + l];
+      if (l == 0) *reinterpret_cast<float*>(wsc + WS_GL) = F[(PSF_G >> 2) + CH - 1];
+    }
     float4* gU = reinterpret_cast<float4*>(wsc + WS_UB);
     const int vb = wave & 7;
 #pragma unroll
@@ -722,56 +700,10 @@ __device__ __forceinline__ void prep_item(uint8_t* lb, const ItemAt& it, RowRegs
       const int i0 = 16 * tb + 4 * gq;
       const uint2 vv = lds_tr(lb, PS_V + 4096 * tb + (L.dv ^ (32 * vb)));
       const f32x4 bs = lds_at<f32x4>(lb, PS_F + PSF_B + 4 * i0);
-      const f32x4 fk = lds_at<f32x4>(lb, PS_F + PSF_FK + 4 * i0);
-      f32x4 ub;
-      ub[0] = fmaf(bs[0], __uint_as_float(vv.x << 16), u[0]);
-      ub[1] = fmaf(bs[1], __uint_as_float(vv.x & 0xffff0000u), u[1]);
-      ub[2] = fmaf(bs[2], __uint_as_float(vv.y << 16), u[2]);
-      ub[3] = fmaf(bs[3], __uint_as_float(vv.y & 0xffff0000u), u[3]);
-      gU[(vb * 4 + tb) * 64 + l] = make_float4(fk[0] * ub[0], fk[1] * ub[1], fk[2] * ub[2], fk[3] * ub[3]);
-      put_t16(lb, PS_UBT, tb, vb, L, ub);
+      gU[(vb * 4 + tb) * 64 + l] = make_float4(
+          fmaf(bs[0], __uint_as_float(vv.x << 16), u[0]), fmaf(bs[1], __uint_as_float(vv.x & 0xffff0000u), u[1]),
+          fmaf(bs[2], __uint_as_float(vv.y << 16), u[2]), fmaf(bs[3], __uint_as_float(vv.y & 0xffff0000u), u[3]));
     }
-  }
-  item_barrier();
-
-  // 8. Q' = Fq q - R K (as A fragments) and Ob = P Ub (bf16 D tiles); G_L
-  {
-    uint4* gQ = reinterpret_cast<uint4*>(wsc + WS_QP);
-#pragma unroll
-    for (int n = 0; n < NJ16; ++n) {
-      const int job = wave + W * n, tb = job >> 2, kq = job & 3, nk = tri_kend(tb) / 32;
-      f32x4 d0 = zero4(), d1 = zero4();
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk)
-        if (kk < nk) {
-          const bf16x8 rf = pfragT8(lb, PS_RT, 16 * tb, kk, L);
-          d0 = mfma(pfragT16(lb, PS_K, 32 * kq, kk, L), rf, d0);
-          d1 = mfma(pfragT16(lb, PS_K, 32 * kq + 16, kk, L), rf, d1);
-        }
-      const float fq = F[(PSF_FQ >> 2) + 16 * tb + m];
-      const uint2 c0 = cq[n][0], c1 = cq[n][1];
-      d0[0] = fmaf(fq, __uint_as_float(c0.x << 16), -d0[0]);
-      d0[1] = fmaf(fq, __uint_as_float(c0.x & 0xffff0000u), -d0[1]);
-      d0[2] = fmaf(fq, __uint_as_float(c0.y << 16), -d0[2]);
-      d0[3] = fmaf(fq, __uint_as_float(c0.y & 0xffff0000u), -d0[3]);
-      d1[0] = fmaf(fq, __uint_as_float(c1.x << 16), -d1[0]);
-      d1[1] = fmaf(fq, __uint_as_float(c1.x & 0xffff0000u), -d1[1]);
-      d1[2] = fmaf(fq, __uint_as_float(c1.y << 16), -d1[2]);
-      d1[3] = fmaf(fq, __uint_as_float(c1.y & 0xffff0000u), -d1[3]);
-      gQ[(tb * 4 + kq) * 64 + l] = kappa_frag(d0, d1);
-    }
-    uint2* gO = reinterpret_cast<uint2*>(wsc + WS_OB);
-    const int vb = wave & 7;
-#pragma unroll
-    for (int tt = 0; tt < TBN; ++tt) {
-      const int tb = (wave >> 3) * TBN + tt;
-      f32x4 y = zero4();
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk)
-        if (kk < tri_kend(tb) / 32) y = mfma(pfragT8(lb, PS_PT, 16 * tb, kk, L), pfrag8(lb, PS_UBT, 16 * vb, kk, L), y);
-      gO[(vb * 4 + tb) * 64 + l] = make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));
-    }
-    if (tid == 0) *reinterpret_cast<float*>(wsc + WS_GL) = F[(PSF_G >> 2) + CH - 1];
   }
   item_barrier();  // the next item's rows overwrite the LDS
 }
@@ -813,7 +745,7 @@ __global__ __launch_bounds__(64 * W, P1_WAVES_PER_SIMD) void chunk_prep_kernel(
     const bool has_next = w.item < n_items;
     ItemAt nx = cur;
     if (has_next) nx = w.at(cu, chunk_idx, n_seqs, T);
-    prep_item<TG, GATE, true, W>(lb, cur, R, has_next, nx, q, k, v, g, beta, A_log, dt_bias, Hv, scale, qk_l2norm, rs, ws, L,
+    prep_item<TG, GATE, W>(lb, cur, R, has_next, nx, q, k, v, g, beta, A_log, dt_bias, Hv, scale, qk_l2norm, rs, ws, L,
                         lr.rowoff, lr.oq, lr.ok, lr.ov);
     cur = nx;
   }
@@ -830,9 +762,10 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // Operands of one chunk held in registers (prefetched one chunk ahead), for a workgroup of NV value blocks.
 template <int NV>
 struct Pre {
-  bf16x8 A[4];   // W' (U role) or Q' (O role) fragments of this wave's 16 tokens, k-steps 0..3
+  bf16x8 A[4];   // W (U role) or Q' (O role) fragments of this wave's 16 tokens, k-steps 0..3
   bf16x8 KT[2];  // K^T fragments of this wave's 16 state columns, token steps 0, 1
-  uint4 X[NV];   // per value block, U role: Ub' (4 fp32); O role: Ob (4 bf16 in .x, .y)
+  uint4 X[NV > 2 ? NV : 2];  // U role: Ub (4 fp32) per value block; O role: the P fragments, token steps 0, 1
+  f32x4 F;       // U role: Fk of this lane's 4 tokens
   float GL;      // G at the chunk end
 };
 
@@ -840,11 +773,13 @@ struct Pre {
 // The state slice sits in 256-byte rows with 16-byte chunk c of row r at chunk c ^ r (r < 16): its fragment
 // reads (16 rows at one chunk) then meet every bank once. (With padded 272-byte rows each of those reads took
 // 8 LDS cycles, 4 of them bank conflicts, against 4 and none: measured with the hardware counters.)
-template <int NV>
+template <int NV, bool OW = false>
 struct StateSharedT {
-  uint16_t Ss[NV * VB * DK];   // state slice (bf16), key columns at positions pi(key): B operand of [W'; Q'] S^T
+  uint16_t Ss[NV * VB * DK];   // state slice (bf16), key columns at positions pi(key): B operand of [W; Q'] S^T
   uint16_t UhT[NV * VB][LDC];  // U'^T, hi part   } A operands of the state update
   uint16_t UlT[NV * VB][LDC];  // U'^T, lo part   }
+  uint16_t UT[NV * VB][LDC];   // U^T: B operand of P U
+  f32x4 OV[OW ? NV * 4 : 1][OW ? 64 : 1];  // with output waves: Q' S^T, D tiles [block][token tile]
 };
 using StateShared = StateSharedT<1>;
 __device__ __forceinline__ int ss_at(int r, int c) { return r * DK + ((((c >> 3) ^ r) & 15) << 3) + (c & 7); }
@@ -852,7 +787,7 @@ __device__ __forceinline__ int ss_at(int r, int c) { return r * DK + ((((c >> 3)
 struct StateArgs {
   const uint8_t* ws;
   int c0, bos, len, nchunks, Hv, h, vb;
-  float xs;  // 1, or 0 for a transition run (Ub' and Ob taken as zero: the pass then carries S -> S A_c)
+  float xs;  // 1, or 0 for a transition run (Ub taken as zero: the pass then carries S -> S A_c)
   // overlapped form: the ready flag of this job's chunk ci is flags[ci * flag_step], nonzero once phase 1 has
   // stored the item (flag_step 0 with flags on a word that stays zero: every wait runs out -- the host's test
   // of the error path); spin_max bounds each wait
@@ -901,15 +836,16 @@ __device__ __forceinline__ void store_o_tile(TOut* o, const StateArgs& a, int vb
   }
 }
 
-// The chunk loop of one wave. URole: waves 0-3 form U' = Ub' - W' S^T of their 16 tokens; the O role
-// (waves 4-7) forms the outputs O = Ob + Q' S^T of their 16 tokens. Both run the same barriers and each
-// wave updates 16 columns of the state slice. The slice holds NV blocks of 16 value rows (a.vb .. a.vb + NV -
-// 1): every operand fetched for a chunk but Ub' / Ob serves all of them.
-template <bool URole, typename TOut, bool Wait, int NV>
-__device__ __forceinline__ void state_loop(StateSharedT<NV>& sh, const StateArgs& a, TOut* o, f32x4 (&S)[NV]) {
+// The chunk loop of one wave. URole: waves 0-3 form U = Ub - W S^T of their 16 tokens, as bf16 for P U and
+// scaled by Fk for the state update; the O role (waves 4-7) forms the outputs O = Q' S^T + P U of their 16
+// tokens. Both run the same barriers and each wave updates 16 columns of the state slice. The slice holds NV
+// blocks of 16 value rows (a.vb .. a.vb + NV - 1): every operand fetched for a chunk but Ub serves all of them.
+// OW: four more waves (out_loop) add P U and store the outputs; the O role hands them its part through LDS.
+template <bool URole, typename TOut, bool Wait, int NV, bool OW>
+__device__ __forceinline__ void state_loop(StateSharedT<NV, OW>& sh, const StateArgs& a, TOut* o, f32x4 (&S)[NV]) {
   const int l = lane_id(), wave = threadIdx.x >> 6;
-  const int tb = wave & 3;               // this wave's token tile
-  const int j = l & 15;                  // value row within the slice (D layout column of [W'; Q'] S^T)
+  const int tb = __builtin_amdgcn_readfirstlane(wave & 3);  // this wave's token tile
+  const int j = l & 15;                  // value row within the slice (D layout column of [W; Q'] S^T)
   const int t0 = 16 * tb + 4 * (l >> 4);  // first of this lane's 4 tokens (D layout rows)
   // position of key column 16 wave + l%16 in Ss, the inverse of kappa
   const int pcol = 32 * (wave >> 1) + 8 * ((l & 15) >> 2) + 4 * (wave & 1) + (l & 3);
@@ -931,8 +867,11 @@ __device__ __forceinline__ void state_loop(StateSharedT<NV>& sh, const StateArgs
   // per-lane byte offsets inside a chunk's workspace, the same for every chunk
   const uint32_t offA = (uint32_t)(URole ? WS_WP : WS_QP) + (uint32_t)(tb * 4 * 64 + l) * 16u;
   const uint32_t offX = URole ? (uint32_t)WS_UB + (uint32_t)((a.vb * 4 + tb) * 64 + l) * 16u
-                              : (uint32_t)WS_OB + (uint32_t)((a.vb * 4 + tb) * 64 + l) * 8u;
-  constexpr uint32_t XB = URole ? 4u * 64u * 16u : 4u * 64u * 8u;  // from one value block's Ub' / Ob to the next
+                              : (uint32_t)WS_P + (uint32_t)(tb * 2 * 64 + l) * 16u;
+  constexpr int NX = URole ? NV : OW ? 0 : 2;  // X loads: NV blocks' Ub, 4 KiB apart; two P fragments (the first
+                                               // one again where the second is not held)
+  const uint32_t XB = URole ? 4u * 64u * 16u : (tb < 2 ? 0u : 1024u);
+  const uint32_t offF = (uint32_t)WS_F + 4u * (uint32_t)t0;  // (U role)
   const uint32_t offK = (uint32_t)WS_KT + (uint32_t)(wave * 2 * 64 + l) * 16u;
   auto ld16 = [](Rsrc w, uint32_t off) {
     return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(w, off, 0, 0));
@@ -947,14 +886,9 @@ __device__ __forceinline__ void state_loop(StateSharedT<NV>& sh, const StateArgs
     x.A[2] = ld16(w, offA + 2048u);
     x.A[3] = ld16(w, offA + 3072u);
 #pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      if constexpr (URole) {
-        x.X[v] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(w, offX + v * XB, 0, 0));
-      } else {
-        const uint2 ob = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(w, offX + v * XB, 0, 0));
-        x.X[v] = make_uint4(ob.x, ob.y, 0, 0);
-      }
-    }
+    for (int v = 0; v < NX; ++v)
+      x.X[v] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(w, offX + v * XB, 0, 0));
+    if constexpr (URole) x.F = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(w, offF, 0, 0));
   };
   auto fetch3 = [&](Rsrc w, Pre<NV>& x) {
     x.KT[0] = ld16(w, offK);
@@ -995,12 +929,31 @@ __device__ __forceinline__ void state_loop(StateSharedT<NV>& sh, const StateArgs
     wait_ready(ni);
     const Rsrc wn = chunk_ws(ni);
     fetch1(wn, nxt);
+    // U role: Ub and Fk Ub ahead of the barrier, so that U' = Fk Ub - Fk (W S^T) takes one step after it
+    float ub[NV][4], us[NV][4];
+    if constexpr (URole) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        const uint32_t X[4] = {cur.X[v].x, cur.X[v].y, cur.X[v].z, cur.X[v].w};
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+          ub[v][i4] = a.xs * __uint_as_float(X[i4]);
+          us[v][i4] = cur.F[i4] * ub[v][i4];
+          asm volatile("" : "+v"(us[v][i4]));
+        }
+      }
+    }
     lds_barrier();
 
     float ov[NV][4];  // O role: this wave's outputs
+    f32x4 wx[NV];     // U role: W S^T
+    auto put_u = [&](int v) {  // U = Ub - W S^T, as bf16
+      *reinterpret_cast<uint2*>(&sh.UT[v * VB + j][t0]) = make_uint2(
+          pack_bf16x2(ub[v][0] - wx[v][0], ub[v][1] - wx[v][1]), pack_bf16x2(ub[v][2] - wx[v][2], ub[v][3] - wx[v][3]));
+    };
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-      // [W'; Q'] S^T for this wave's 16 tokens, as two independent MFMA chains (half the dependent latency)
+      // [W; Q'] S^T for this wave's 16 tokens, as two independent MFMA chains (half the dependent latency)
       f32x4 x0 = zero4(), x1 = zero4();
 #pragma unroll
       for (int kk = 0; kk < 4; kk += 2) {
@@ -1008,25 +961,23 @@ __device__ __forceinline__ void state_loop(StateSharedT<NV>& sh, const StateArgs
         x1 = mfma(cur.A[kk + 1], ss_chunks[v * VB * DK / 8 + ss_r[kk + 1]], x1);
       }
       const f32x4 x = x0 + x1;
-      const uint4 X = cur.X[v];
       if constexpr (URole) {
-        // U' = Ub' - W' S^T as hi + lo bf16
-        const float ub[4] = {a.xs * __uint_as_float(X.x), a.xs * __uint_as_float(X.y), a.xs * __uint_as_float(X.z),
-                             a.xs * __uint_as_float(X.w)};
+        // U' = Fk (Ub - W S^T) as hi + lo bf16
         float u[4];
 #pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) u[i4] = ub[i4] - x[i4];
-        const uint32_t h01 = pack_bf16x2(u[0], u[1]), h23 = pack_bf16x2(u[2], u[3]);
-        const uint32_t l01 = pack_bf16x2(u[0] - __uint_as_float(h01 << 16), u[1] - __uint_as_float(h01 & 0xffff0000u));
-        const uint32_t l23 = pack_bf16x2(u[2] - __uint_as_float(h23 << 16), u[3] - __uint_as_float(h23 & 0xffff0000u));
+        for (int i4 = 0; i4 < 4; ++i4) u[i4] = fmaf(-cur.F[i4], x[i4], us[v][i4]);
+        uint32_t h01, l01, h23, l23;
+        split2(u[0], u[1], h01, l01);
+        split2(u[2], u[3], h23, l23);
         *reinterpret_cast<uint2*>(&sh.UhT[v * VB + j][t0]) = make_uint2(h01, h23);
         *reinterpret_cast<uint2*>(&sh.UlT[v * VB + j][t0]) = make_uint2(l01, l23);
+        wx[v] = x;
+        if constexpr (!OW) put_u(v);
       } else {
-        // O = Ob + Q' S^T (stored after the state update is issued)
-        const float ob[4] = {a.xs * __uint_as_float(X.x << 16), a.xs * __uint_as_float(X.x & 0xffff0000u),
-                             a.xs * __uint_as_float(X.y << 16), a.xs * __uint_as_float(X.y & 0xffff0000u)};
+        // Q' S^T (P U added, and the outputs stored, after the state update is issued)
 #pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) ov[v][i4] = ob[i4] + x[i4];
+        for (int i4 = 0; i4 < 4; ++i4) ov[v][i4] = x[i4];
+        if constexpr (OW) sh.OV[v * 4 + tb][l] = f32x4{ov[v][0], ov[v][1], ov[v][2], ov[v][3]};
       }
     }
     fetch2(wn, nxt);
@@ -1046,9 +997,19 @@ __device__ __forceinline__ void state_loop(StateSharedT<NV>& sh, const StateArgs
       acc1 = mfma(frag(&sh.UlT[v * VB][0], LDC, 0, 32), cur.KT[1], acc1);
       S[v] = acc0 + acc1;
     }
-    if constexpr (!URole) {
+    if constexpr (URole && OW) {  // for the output waves, read after the next barrier: off this chunk's path
 #pragma unroll
-      for (int v = 0; v < NV; ++v) store_o_tile(o, a, a.vb + v, ci, t0, j, ov[v]);
+      for (int v = 0; v < NV; ++v) put_u(v);
+    }
+    if constexpr (!URole && !OW) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        f32x4 y = f32x4{ov[v][0], ov[v][1], ov[v][2], ov[v][3]};
+        y = mfma(__builtin_bit_cast(bf16x8, cur.X[0]), frag(&sh.UT[v * VB][0], LDC, 0, 0), y);
+        if (tb >= 2) y = mfma(__builtin_bit_cast(bf16x8, cur.X[1]), frag(&sh.UT[v * VB][0], LDC, 0, 32), y);
+        const float yo[4] = {y[0], y[1], y[2], y[3]};
+        store_o_tile(o, a, a.vb + v, ci, t0, j, yo);
+      }
     }
   };
 
@@ -1074,20 +1035,101 @@ __device__ __forceinline__ void state_loop(StateSharedT<NV>& sh, const StateArgs
     process(ci + 1, b0, min(ci + 2, last), b1);
   }
   if (ci < a.nchunks) process(ci, b1, ci, b0);
+  if constexpr (OW) lds_barrier();  // the last chunk's U, for the output waves
 }
+
+// The chunk loop of an output wave (waves 8-11 of a workgroup that has them): O = Q' S^T + P U of token
+// tile `wave & 3`, the first part from the O role's wave. It takes that part after a chunk's second barrier and U,
+// which the U role writes there, after the next one's first, so that its products and stores run beside the next
+// chunk's, off the chain.
+template <typename TOut, int NV>
+__device__ __forceinline__ void out_loop(StateSharedT<NV, true>& sh, const StateArgs& a, TOut* o) {
+  if (a.nchunks <= 0) return;
+  const int l = lane_id(), tb = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) & 3);
+  const int j = l & 15, t0 = 16 * tb + 4 * (l >> 4);
+  const uint32_t off = (uint32_t)WS_P + (uint32_t)(tb * 2 * 64 + l) * 16u, off1 = off + (tb < 2 ? 0u : 1024u);
+  struct P2 {
+    bf16x8 f[2];
+  };
+  f32x4 ov[NV];
+  auto finish = [&](int ci, const P2& p) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      f32x4 y = mfma(p.f[0], frag(&sh.UT[v * VB][0], LDC, 0, 0), ov[v]);
+      if (tb >= 2) y = mfma(p.f[1], frag(&sh.UT[v * VB][0], LDC, 0, 32), y);
+      const float yo[4] = {y[0], y[1], y[2], y[3]};
+      store_o_tile(o, a, a.vb + v, ci, t0, j, yo);
+    }
+  };
+  auto take = [&](int ci, P2& p) {  // chunk ci's P fragments and, past its second barrier, the O role's part
+    const Rsrc w = raw_rsrc(a.ws + ((size_t)(a.c0 + ci) * a.Hv + a.h) * WS_CHUNK, WS_CHUNK);
+    p.f[0] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(w, off, 0, 0));
+    p.f[1] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(w, off1, 0, 0));
+  };
+  auto take_ov = [&]() {
+    lds_barrier();
+#pragma unroll
+    for (int v = 0; v < NV; ++v) ov[v] = sh.OV[v * 4 + tb][l];
+  };
+  P2 b0, b1;
+  take(0, b0);
+  lds_barrier();
+  take_ov();
+  int ci = 1;
+  for (; ci + 1 < a.nchunks; ci += 2) {
+    take(ci, b1);
+    lds_barrier();
+    finish(ci - 1, b0);
+    take_ov();
+    take(ci + 1, b0);
+    lds_barrier();
+    finish(ci, b1);
+    take_ov();
+  }
+  if (ci < a.nchunks) {
+    take(ci, b1);
+    lds_barrier();
+    finish(ci - 1, b0);
+    take_ov();
+    lds_barrier();
+    finish(ci, b1);
+  } else {
+    lds_barrier();
+    finish(ci - 1, b0);
+  }
+}
+
+// The chunk loop of one wave of a state workgroup by its role.
+template <typename TOut, int NV, bool OW>
+__device__ __forceinline__ void run_loop(StateSharedT<NV, OW>& sh, const StateArgs& a, TOut* o, f32x4 (&S)[NV]) {
+  const int wave = wave_id();
+  if (wave < 4)
+    state_loop<true, TOut, false, NV, OW>(sh, a, o, S);
+  else if (!OW || wave < 8)
+    state_loop<false, TOut, false, NV, OW>(sh, a, o, S);
+  else if constexpr (OW)
+    out_loop<TOut, NV>(sh, a, o);
+}
+// Waves of a state workgroup: output waves where each has a CU to itself (one block; two-block workgroups share a CU
+// in twos, and 12 waves of their registers would not). One block, T = 4096 at 16 heads: 45.2 us with them, 45.8 with
+// the O role doing P U itself, 47.3 with the U role doing it a chunk late, 49.5 with the output waves taking Q' S^T too.
+template <int NV>
+constexpr bool state_ow() { return NV == 1; }
+template <int NV>
+constexpr int state_threads() { return 64 * (state_ow<NV>() ? P2_WAVES + 4 : P2_WAVES); }
 
 // Segmented runs of phase 2 (unpacked batches whose pass would hold few CUs): each sequence is cut into G
 // segments of Cs chunks. "Local" runs carry each segment from a zero state (the first from the sequence's
 // initial state) and write its outputs and end state L_g; "transition" runs carry segments 1.. from the
-// identity with Ub' = Ob = 0, so their state is the segment's map P_c = A_1 .. A_c (S -> S A_c per chunk), their
+// identity with Ub = 0, so their state is the segment's map P_c = A_1 .. A_c (S -> S A_c per chunk), their
 // end state M_g and their outputs Q'_c P_c^T. The true state entering segment g is S_g = S_{g-1} M_{g-1} +
-// L_{g-1} (S_1 = L_0) and the true outputs are o_local + (Q' P^T) S_g^T: chunk_combine_kernel and
+// L_{g-1} (S_1 = L_0) and the true outputs are o_local + R_c S_g^T: chunk_combine_kernel and
 // chunk_correct_kernel form them. All local and transition workgroups run at once.
 struct SegRun {
   int G, Cs;               // segments per sequence, chunks per segment (G == 1: plain runs)
   float* local_final;      // L [n_seqs * G][Hv][V][K]
   float* trans_final;      // M^T [n_seqs * (G - 1)][Hv] as bf16 hi then lo, each [K][K] in mt_frag order
-  uint16_t* trans_out;     // Q' P^T [n_seqs * T][Hv][K] (bf16)
+  uint16_t* trans_out;     // R [n_seqs * T][Hv][K] (bf16)
 };
 
 // Position (in 16-bit elements) of M^T[n][k] in the transition runs' stored maps: the order in which
@@ -1102,12 +1144,13 @@ __device__ __forceinline__ size_t mt_frag(int n, int k) {
 }
 
 template <typename TOut, int NV>
-__global__ __launch_bounds__(64 * P2_WAVES) void chunk_state_kernel(
+__global__ __launch_bounds__(state_threads<NV>(), NV == 2 ? 4 : 3) void chunk_state_kernel(
     const uint8_t* ws, const float* __restrict__ s_in, float* __restrict__ s_out, TOut* __restrict__ o,
     const int32_t* __restrict__ cu, int n_seqs, int n_chunks, int T, int Hv, const SegRun seg) {
   // (ws is not __restrict__: that keeps the compiler from sinking the prefetch loads below the LDS
   // barriers, whose asm memory clobber then pins them where they are issued)
-  __shared__ StateSharedT<NV> sh;
+  constexpr bool OW = state_ow<NV>();
+  __shared__ StateSharedT<NV, OW> sh;
   constexpr int NG = DV / VB / NV;  // workgroups per (run, head): NV value blocks of 16 rows each
 
   // XCD-aware order (workgroups go round-robin over the 8 XCDs): ids are taken in groups of 8 NG = 8 pairs
@@ -1122,8 +1165,8 @@ __global__ __launch_bounds__(64 * P2_WAVES) void chunk_state_kernel(
   const int h = vp % Hv, run = vp / Hv;  // run: the (sequence, segment) index among local / transition runs
   const int seq = trans ? run / (seg.G - 1) : run / seg.G;
   const int sg = trans ? 1 + run % (seg.G - 1) : run % seg.G;
-  const int l = lane_id(), wave = threadIdx.x >> 6;
-  const int ncol = 16 * wave + (l & 15);
+  const int l = lane_id(), wave = wave_id();
+  const int ncol = 16 * (wave & 7) + (l & 15);
 
   StateArgs a;
   a.ws = ws;
@@ -1172,10 +1215,8 @@ __global__ __launch_bounds__(64 * P2_WAVES) void chunk_state_kernel(
   a.flags = nullptr;
   a.flag_step = 0;
   a.spin_max = 0;
-  if (wave < 4)
-    state_loop<true, TOut, false, NV>(sh, a, out, S);
-  else
-    state_loop<false, TOut, false, NV>(sh, a, out, S);
+  run_loop<TOut, NV, OW>(sh, a, out, S);
+  if (wave >= 8) return;  // (output waves hold no state)
 
   if (trans) {  // the segment map transposed (M^T[n][k] = M[k][n]), as bf16 hi and lo parts [K][K] each
     uint16_t* mt = reinterpret_cast<uint16_t*>(seg.trans_final + ((size_t)run * Hv + h) * hs);
@@ -1205,10 +1246,11 @@ __global__ __launch_bounds__(64 * P2_WAVES) void chunk_state_kernel(
 // (untouched when it has none; zeros for a fresh slot). The open chunk is a second, one-chunk loop, so that the
 // states between are at hand without a test in the chunk loop; otherwise chunk_state_kernel's packed form.
 template <int NV>
-__global__ __launch_bounds__(64 * P2_WAVES) void chunk_serve_state_kernel(const uint8_t* ws, const ServeRuns r,
+__global__ __launch_bounds__(state_threads<NV>(), NV == 2 ? 4 : 3) void chunk_serve_state_kernel(const uint8_t* ws, const ServeRuns r,
                                                                           float* commit, float* __restrict__ live,
                                                                           bf16* __restrict__ o, int Hv) {
-  __shared__ StateSharedT<NV> sh;
+  constexpr bool OW = state_ow<NV>();
+  __shared__ StateSharedT<NV, OW> sh;
   constexpr int NG = DV / VB / NV;
   const int id = blockIdx.x;
   const int pair = (id / (8 * NG)) * 8 + (id % 8), vb = ((id % (8 * NG)) / 8) * NV;
@@ -1216,8 +1258,8 @@ __global__ __launch_bounds__(64 * P2_WAVES) void chunk_serve_state_kernel(const 
   const int h = pair % Hv, seq = pair / Hv;
   const int slot = r.slots[seq];
   if (slot < 0 || slot >= r.n_slots) return;
-  const int l = lane_id(), wave = threadIdx.x >> 6;
-  const int ncol = 16 * wave + (l & 15);
+  const int l = lane_id(), wave = wave_id();
+  const int ncol = 16 * (wave & 7) + (l & 15);
   StateArgs a;
   a.ws = ws;
   a.Hv = Hv;
@@ -1240,17 +1282,11 @@ __global__ __launch_bounds__(64 * P2_WAVES) void chunk_serve_state_kernel(const 
 #pragma unroll
     for (int i4 = 0; i4 < 4; ++i4) S[v][i4] = fresh ? 0.f : commit[at(v, i4)];
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // settle the state loads before the pipelined loop
-  auto loop = [&]() {
-    if (wave < 4)
-      state_loop<true, bf16, false, NV>(sh, a, o, S);
-    else
-      state_loop<false, bf16, false, NV>(sh, a, o, S);
-  };
   a.bos = bos;
   a.len = whole * CH;
   a.nchunks = whole;
-  loop();
-  if (whole > 0 || fresh) {
+  run_loop<bf16, NV, OW>(sh, a, o, S);
+  if (wave < 8 && (whole > 0 || fresh)) {
 #pragma unroll
     for (int v = 0; v < NV; ++v)
 #pragma unroll
@@ -1261,8 +1297,9 @@ __global__ __launch_bounds__(64 * P2_WAVES) void chunk_serve_state_kernel(const 
     a.len = len - whole * CH;
     a.c0 += whole;
     a.nchunks = 1;
-    loop();
+    run_loop<bf16, NV, OW>(sh, a, o, S);
   }
+  if (wave >= 8) return;  // (output waves hold no state)
 #pragma unroll
   for (int v = 0; v < NV; ++v)
 #pragma unroll
@@ -1462,9 +1499,9 @@ __global__ __launch_bounds__(P1_THREADS, P1_WAVES_PER_SIMD) void chunk_fused_ker
         S[0][i4] = s_in != nullptr ? s_in[((size_t)sq * Hv + h) * hs + slice + (size_t)i4 * DK] : 0.f;
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       if (wave < 4)
-        state_loop<true, bf16, true, 1>(sm.s, a, o, S);
+        state_loop<true, bf16, true, 1, false>(sm.s, a, o, S);
       else
-        state_loop<false, bf16, true, 1>(sm.s, a, o, S);
+        state_loop<false, bf16, true, 1, false>(sm.s, a, o, S);
       if (s_out != nullptr) {
 #pragma unroll
         for (int i4 = 0; i4 < 4; ++i4) s_out[((size_t)sq * Hv + h) * hs + slice + (size_t)i4 * DK] = S[0][i4];
@@ -1516,7 +1553,7 @@ __global__ __launch_bounds__(P1_THREADS, P1_WAVES_PER_SIMD) void chunk_fused_ker
     if (cur < n_items) {
       const ItemAt ic = item_at(cur, cu, chunk_idx, n_seqs, T, Hk, Hv);
       const ItemAt in = item_at(nload >= 0 ? nload : cur, cu, chunk_idx, n_seqs, T, Hk, Hv);
-      prep_item<TG, GATE, false, P1_WAVES>(sm.p.b, ic, R, nload >= 0, in, q, k, v, g, beta, A_log, dt_bias, Hv, scale, qk_l2norm, rs,
+      prep_item<TG, GATE, P1_WAVES>(sm.p.b, ic, R, nload >= 0, in, q, k, v, g, beta, A_log, dt_bias, Hv, scale, qk_l2norm, rs,
                           ws, L, lr.rowoff, lr.oq, lr.ok, lr.ov);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's workspace stores are in the L2
       __syncthreads();
@@ -1636,9 +1673,9 @@ __global__ __launch_bounds__(256) void chunk_combine_kernel(const float* __restr
   }
 }
 
-// o[t][h][:] += (Q' P^T)[t][h][:] S_g^T for the rows of one chunk of a segment g >= 1: D = S_g . (Q'P^T)^T on
+// o[t][h][:] += R[t][h][:] S_g^T for the rows of one chunk of a segment g >= 1: D = S_g . R^T on
 // bf16 MFMA with the values as the M side (A = S_g rows, staged once in LDS for the 4 waves) and the tokens as
-// the N side (B = Q'P^T rows), so each lane's D values are 4 adjacent values of one row of o (one 8-byte
+// the N side (B = R's rows), so each lane's D values are 4 adjacent values of one row of o (one 8-byte
 // read-modify-write, its read issued first). 4 waves x 16 tokens.
 constexpr int CR_LD = DK + 8;  // bf16 row stride of the staged S_g: 272 bytes, rows 4 banks apart
 template <typename TOut>
@@ -1711,7 +1748,7 @@ __global__ __launch_bounds__(256) void chunk_correct_kernel(const uint16_t* __re
 // launches and the longer state pass). A segment count in 2 .. 8 is taken when its local and transition
 // workgroups all fit one per CU and it is the cheapest.
 // NV: value blocks of 16 rows per state-pass workgroup. Two when the plain pass's workgroups of one block
-// would outnumber the CUs (more than n_cu / 8 chains): each then reads a chunk's shared operands (W' or Q',
+// would outnumber the CUs (more than n_cu / 8 chains): each then reads a chunk's shared operands (W or Q',
 // K^T) once for 32 value rows, and the pass needs half the workgroup slots, for chunk steps about 1.4x as long
 // (measured: 32 packed sequences of 30,526 tokens at 16 heads, 4,096 one-block workgroups, 506 us with two
 // blocks against 552; one 4096-token sequence at 16 heads, 128 workgroups, 92.5 us with two against 73.6).
@@ -1738,7 +1775,7 @@ SegPlan seg_plan(int B, int T, int Hv, int n_cu) {
   return p;
 }
 
-// Bytes past the phase-1 workspace a segmented run needs: Q'P^T (bf16 [B*T][Hv][K]), L (fp32, G per
+// Bytes past the phase-1 workspace a segmented run needs: R (bf16 [B*T][Hv][K]), L (fp32, G per
 // sequence), M^T (bf16 hi and lo, G - 1 per sequence), S_g (bf16, G - 1 per sequence).
 size_t seg_bytes(int B, int T, int Hv, const SegPlan& p) {
   if (p.G <= 1) return 0;
@@ -1985,10 +2022,10 @@ int chunk_fwd_impl(const char* fn, const void* q, const void* k, const void* v, 
   // groups of 8 pairs x DV / VB / NV value-block groups
   const dim3 grid2((unsigned)(((runs + 7) / 8) * 8 * (DV / VB / plan.NV)));
   if (plan.NV == 2)
-    hipLaunchKernelGGL((chunk_state_kernel<bf16, 2>), grid2, dim3(64 * P2_WAVES), 0, s, ws, initial_state,
+    hipLaunchKernelGGL((chunk_state_kernel<bf16, 2>), grid2, dim3(state_threads<2>()), 0, s, ws, initial_state,
                        final_state, (bf16*)o, cu_seqlens, N, n_chunks, T, Hv, run);
   else
-    hipLaunchKernelGGL((chunk_state_kernel<bf16, 1>), grid2, dim3(64 * P2_WAVES), 0, s, ws, initial_state,
+    hipLaunchKernelGGL((chunk_state_kernel<bf16, 1>), grid2, dim3(state_threads<1>()), 0, s, ws, initial_state,
                        final_state, (bf16*)o, cu_seqlens, N, n_chunks, T, Hv, run);
   if (segmented) {
     hipLaunchKernelGGL(chunk_combine_kernel, dim3(N * Hv * (DV / CB_ROWS)), dim3(256), 0, s, run.local_final,
@@ -2153,10 +2190,10 @@ extern "C" int zgdn_serving_extend(const void* mixed, long mixed_ld, const void*
   const int nv = state_nv((long)n_runs * H, device_cus());
   const dim3 grid((unsigned)((((long)n_runs * H + 7) / 8) * 8 * (DV / VB / nv)));
   if (nv == 2)
-    hipLaunchKernelGGL(chunk_serve_state_kernel<2>, grid, dim3(64 * P2_WAVES), 0, s, ws, r, state_commit, state_live,
+    hipLaunchKernelGGL(chunk_serve_state_kernel<2>, grid, dim3(state_threads<2>()), 0, s, ws, r, state_commit, state_live,
                        (bf16*)o, H);
   else
-    hipLaunchKernelGGL(chunk_serve_state_kernel<1>, grid, dim3(64 * P2_WAVES), 0, s, ws, r, state_commit, state_live,
+    hipLaunchKernelGGL(chunk_serve_state_kernel<1>, grid, dim3(state_threads<1>()), 0, s, ws, r, state_commit, state_live,
                        (bf16*)o, H);
   serve_norm(r, o, m + 3 * inner, mixed_ld, norm_weight, eps, gated, x, hidden, window, win_len, H, s);
   return check_launch(fn);
