@@ -25,8 +25,9 @@
 // Matrices in LDS are fp32 row-major with the 16-byte chunk c of row r stored at chunk c ^ (r % 16): a
 // 16-byte read of 16 consecutive rows at one column (the A operands) then meets every bank once, and so
 // does a 4-byte read of 4 rows x 16 columns (the B operands read as columns).
-#include <atomic>
 #include <algorithm>
+#include <atomic>
+#include <type_traits>
 
 #include "gdn_common.h"
 
@@ -177,11 +178,18 @@ struct Rows32 {
   }
 };
 
+// The chunks of a launch's items: item i is (chunk, head) = (at(i / Hv), i % Hv); all of them, or chunks lo .. lo + n -
+// 1 of each of B sequences of nct chunks.
+struct Items32 {
+  int lo, n, nct;
+  __device__ __forceinline__ int chunk(int cc) const { return cc < n ? lo + cc : cc / n * nct + lo + cc % n; }
+};
+
 template <typename TIn, typename TG, int D>
-__device__ __forceinline__ void load_item(Rows32<TIn, TG, D>& x, int item, const TIn* q, const TIn* k, const TIn* v,
+__device__ __forceinline__ void load_item(Rows32<TIn, TG, D>& x, int item, const Items32& at, const TIn* q, const TIn* k, const TIn* v,
                                           const TG* g, const TG* beta, const int32_t* cu, const int32_t* chunk_idx,
                                           int n_seqs, int T, int Hk, int Hv, const RowStrides& rs) {
-  const int c = item / Hv, h = item % Hv, hk = h / (Hv / Hk);
+  const int c = at.chunk(item / Hv), h = item % Hv, hk = h / (Hv / Hk);
   const ChunkRange cr = chunk_range(c, cu, chunk_idx, T, n_seqs);
   constexpr uint32_t E = sizeof(TIn);
   const uint32_t r = threadIdx.x >> 4, c0 = (threadIdx.x & 15) * 4 * E;
@@ -201,32 +209,46 @@ __device__ __forceinline__ void load_item(Rows32<TIn, TG, D>& x, int item, const
   x.beta.load(raw_rsrc(beta + t, gbytes), goff);
 }
 
+// The inputs of phase 1.
+template <typename TIn, typename TG>
+struct Prep32 {
+  const TIn *q, *k, *v;
+  const TG *g, *beta;
+  const float *A_log, *dt_bias;
+  const int32_t *cu, *chunk_idx;
+  int n_seqs, n_items, T, Hk, Hv, qk_l2norm;
+  float scale;
+  RowStrides rs;
+  uint8_t* ws;
+  Items32 at;
+};
+
+// Items first, first + stride, .. by one workgroup.
 template <typename TIn, typename TG, int D, bool GATE>
-__global__ __launch_bounds__(64 * P32_WAVES) void chunk32_prep_kernel(
-    const TIn* __restrict__ q, const TIn* __restrict__ k, const TIn* __restrict__ v, const TG* __restrict__ g,
-    const TG* __restrict__ beta, const float* __restrict__ A_log, const float* __restrict__ dt_bias,
-    const int32_t* __restrict__ cu, const int32_t* __restrict__ chunk_idx, int n_seqs, int n_items, int T, int Hk,
-    int Hv, float scale, int qk_l2norm, const RowStrides rs, uint8_t* __restrict__ ws) {
+__device__ __forceinline__ void prep32(uint8_t* lb, const Prep32<TIn, TG>& p, int first, int stride) {
   using L = Lds32<D>;
   using WS = Ws32<D>;
   constexpr int RB = L::RB, NK = WS::NK;
-  extern __shared__ f32x4 lds32[];
-  uint8_t* lb = reinterpret_cast<uint8_t*>(lds32);
   const f32x4 z4 = {0.f, 0.f, 0.f, 0.f};
+  const int n_items = p.n_items, Hv = p.Hv;
   Rows32<TIn, TG, D> R;
-  if ((int)blockIdx.x >= n_items) return;
-  load_item<TIn, TG, D>(R, blockIdx.x, q, k, v, g, beta, cu, chunk_idx, n_seqs, T, Hk, Hv, rs);
+  if (first >= n_items) return;
+  auto load = [&](int item) {
+    load_item<TIn, TG, D>(R, item, p.at, p.q, p.k, p.v, p.g, p.beta, p.cu, p.chunk_idx, p.n_seqs, p.T, p.Hk, Hv, p.rs);
+  };
+  load(first);
 
-  for (int item = blockIdx.x; item < n_items; item += gridDim.x) {
+  for (int item = first; item < n_items; item += stride) {
     // the lane's and wave's indexes pass through an empty asm per item: the addresses derived from them are then
     // formed inside the item instead of being hoisted out of the loop, where they would not fit the registers
     int tid = threadIdx.x, wave = wave_id();
     asm volatile("" : "+v"(tid));
     asm volatile("" : "+s"(wave));
     const int l = tid & 63, m = l & 15, gq = l >> 4;
-    const int c = item / Hv, h = item % Hv;
-    const int len = chunk_range(c, cu, chunk_idx, T, n_seqs).len;
-    uint8_t* out = ws + (size_t)item * WS::ITEM;
+    const int c = p.at.chunk(item / Hv), h = item % Hv;
+    const int len = chunk_range(c, p.cu, p.chunk_idx, p.T, p.n_seqs).len;
+    uint8_t* out = p.ws + ((size_t)c * Hv + h) * WS::ITEM;
+    const float scale = p.scale;
 
     // ---- 1. rows of q, k (key head hk) and v (value head h) into LDS as fp32 (zeros past the chunk end), q and k
     // L2-normalised when asked: x * rsqrt(sum x^2 + 1e-6)
@@ -245,7 +267,7 @@ __global__ __launch_bounds__(64 * P32_WAVES) void chunk32_prep_kernel(
         }
       }
       float rq = 1.f, rk = 1.f;
-      if (qk_l2norm) {
+      if (p.qk_l2norm) {
         rq = 1.f / sqrtf(group_sum<16>(sq) + 1e-6f);
         rk = 1.f / sqrtf(group_sum<16>(sk) + 1e-6f);
       }
@@ -261,8 +283,8 @@ __global__ __launch_bounds__(64 * P32_WAVES) void chunk32_prep_kernel(
       float gt = 0.f, bt = 0.f;
       if (l < len) {
         const float gr = R.g.get(), br = R.beta.get();
-        gt = GATE ? -expf(A_log[h]) * softplus_exact(gr + dt_bias[h]) : gr;
-        bt = rs.beta_sigmoid ? 1.f / (1.f + expf(-br)) : br;
+        gt = GATE ? -expf(p.A_log[h]) * softplus_exact(gr + p.dt_bias[h]) : gr;
+        bt = p.rs.beta_sigmoid ? 1.f / (1.f + expf(-br)) : br;
       }
       float G = gt;
 #pragma unroll
@@ -319,8 +341,7 @@ __global__ __launch_bounds__(64 * P32_WAVES) void chunk32_prep_kernel(
     bar();
     // the next item's rows (the last item's again past it), in flight over steps 3 and 4: by now the stores of the
     // item before are through, behind which these loads would hold up the waves that issue them
-    load_item<TIn, TG, D>(R, min(item + (int)gridDim.x, n_items - 1), q, k, v, g, beta, cu, chunk_idx, n_seqs, T, Hk,
-                          Hv, rs);
+    load(min(item + stride, n_items - 1));
 
     // ---- 3. T = (I + A)^-1, the diagonal blocks: wave d < 4 by right-looking substitution on block d held as a D
     // tile (lane: rows 4 gq + i of column m). Step j subtracts column j of the block (row j of its transpose,
@@ -458,6 +479,12 @@ __global__ __launch_bounds__(64 * P32_WAVES) void chunk32_prep_kernel(
     }
     bar();  // the next item's rows overwrite the LDS
   }
+}
+
+template <typename TIn, typename TG, int D, bool GATE>
+__global__ __launch_bounds__(64 * P32_WAVES) void chunk32_prep_kernel(const Prep32<TIn, TG> p) {
+  extern __shared__ f32x4 lds32[];
+  prep32<TIn, TG, D, GATE>(reinterpret_cast<uint8_t*>(lds32), p, blockIdx.x, gridDim.x);
 }
 
 // ----------------------------------------------------------------------------------------------- phase 2
@@ -598,36 +625,66 @@ __device__ __forceinline__ void state_loop32(StateShared32<D>& sh, f32x4& st, co
   if (ci < nc) process(ci, b1, ci, b0);
 }
 
+// The inputs of the state pass: chunks lo .. lo + n - 1 of each sequence, from s_in (zeros without it) to s_out.
+template <typename TOut>
+struct State32 {
+  const uint8_t* ws;
+  const float* s_in;
+  float* s_out;
+  TOut* o;
+  const int32_t* cu;
+  int n_seqs, n_chunks, T, Hv, lo, n;
+};
+
 template <typename TOut, int D>
-__global__ __launch_bounds__(512) void chunk32_state_kernel(const uint8_t* ws, const float* __restrict__ s_in,
-                                                            float* __restrict__ s_out, TOut* __restrict__ o,
-                                                            const int32_t* __restrict__ cu, int n_seqs,
-                                                            int n_chunks, int T, int Hv) {
-  // (ws is not __restrict__: the prefetch loads stay where they are issued, ahead of the barriers)
+__device__ __forceinline__ void state32(StateShared32<D>& sh, const State32<TOut>& p, int id) {
   constexpr int NK = Ws32<D>::NK;
-  __shared__ StateShared32<D> sh;
   // the NK workgroups of one (sequence, head) share an id % 8, so they run on one XCD and share its L2 copy of
   // the chunk workspace (the grid is padded to whole groups of 8 NK)
-  const int id = blockIdx.x;
   const int pair = (id / (8 * NK)) * 8 + id % 8, vb = (id % (8 * NK)) / 8;
-  if (pair >= n_seqs * Hv) return;
-  const int seq = pair / Hv, h = pair % Hv;
+  if (pair >= p.n_seqs * p.Hv) return;
+  const int seq = pair / p.Hv, h = pair % p.Hv;
   const int wave = wave_id(), l = threadIdx.x & 63, m = l & 15, gq = l >> 4;
   int c0, bos, len;
-  seq_chunks(cu, seq, T, c0, bos, len);
+  seq_chunks(p.cu, seq, p.T, c0, bos, len);
+  c0 += p.lo;
+  bos += p.lo * CHUNK_LEN;
+  len = max(0, len - p.lo * CHUNK_LEN);
   // chunks past the workspace (a chunk table shorter than the sequences need) are not read
-  const int nc = max(0, min((len + CHUNK_LEN - 1) / CHUNK_LEN, n_chunks - c0));
+  const int nc = max(0, min(min((len + CHUNK_LEN - 1) / CHUNK_LEN, p.n), p.n_chunks - c0));
 
   const size_t at = ((size_t)pair * D + 16 * vb + m) * D + 16 * (wave & (NK - 1)) + 4 * gq;  // this lane's entries
   f32x4 st = {0.f, 0.f, 0.f, 0.f};
-  if (s_in != nullptr) st = *reinterpret_cast<const f32x4*>(s_in + at);
+  if (p.s_in != nullptr) st = *reinterpret_cast<const f32x4*>(p.s_in + at);
   if (nc > 0) {
     if (wave < 4)
-      state_loop32<true, TOut, D>(sh, st, ws, o, c0, nc, bos, len, Hv, h, vb, wave);
+      state_loop32<true, TOut, D>(sh, st, p.ws, p.o, c0, nc, bos, len, p.Hv, h, vb, wave);
     else
-      state_loop32<false, TOut, D>(sh, st, ws, o, c0, nc, bos, len, Hv, h, vb, wave);
+      state_loop32<false, TOut, D>(sh, st, p.ws, p.o, c0, nc, bos, len, p.Hv, h, vb, wave);
   }
-  if (s_out != nullptr && wave < NK) *reinterpret_cast<f32x4*>(s_out + at) = st;
+  if (p.s_out != nullptr && wave < NK) *reinterpret_cast<f32x4*>(p.s_out + at) = st;
+}
+
+template <typename TOut, int D>
+__global__ __launch_bounds__(512) void chunk32_state_kernel(const State32<TOut> p) {
+  __shared__ StateShared32<D> sh;
+  state32<TOut, D>(sh, p, blockIdx.x);
+}
+
+// Both phases side by side, on different chunks: the first n_state workgroups run the state pass over chunks that an
+// earlier launch prepared, the others prepare the chunks after them (the launches' order is all the synchronisation).
+// Each workgroup has a CU to itself (phase 1's LDS). For the batches whose state pass leaves CUs idle; see slices32.
+template <typename TIn, typename TG, int D, bool GATE>
+__global__ __launch_bounds__(64 * P32_WAVES) void chunk32_both_kernel(const Prep32<TIn, TG> p, const State32<TIn> st,
+                                                                      int n_state) {
+  extern __shared__ f32x4 lds32[];
+  static_assert(sizeof(StateShared32<D>) <= Lds32<D>::BYTES, "the state pass's LDS");
+  if ((int)blockIdx.x < n_state) {
+    if (threadIdx.x >= 512) return;  // (whole waves; the barriers count the waves that are left)
+    state32<TIn, D>(*reinterpret_cast<StateShared32<D>*>(lds32), st, blockIdx.x);
+  } else {
+    prep32<TIn, TG, D, GATE>(reinterpret_cast<uint8_t*>(lds32), p, blockIdx.x - n_state, gridDim.x - n_state);
+  }
 }
 
 // Phase 1's dynamic LDS is above the default 64 KiB at D = 128: raised once per device and kernel (the first
@@ -646,20 +703,76 @@ bool lds_ready(K kernel, int bytes, std::atomic<signed char>* state) {
   return ok;
 }
 
+// The state pass's workgroups: whole groups of 8 NK (8 chains, one on each XCD).
+template <int D>
+constexpr int state_grid(int chains) {
+  return (chains + 7) / 8 * 8 * (D / 16);
+}
+
+// Slices of a call of N sequences of nct chunks (1: phase 1, then the state pass). A state pass of few chains leaves CUs
+// idle, and phase 1 of the next slice of chunks runs on them beside it (chunk32_both_kernel). Times in us measured on
+// MI355X: a round of phase-1 items (one a CU) and a chunk of the state pass 19 and 2.0 at D = 128, 9 and 1.0 at 64; a
+// launch more costs about 2. Taken where the sum over the slices is the smallest, by 3 % or more. Measured, in two
+// launches -> sliced: D = 128, 16 heads, 2048 tokens 102 -> 92 us (2 slices), 4096 200 -> 170 (4), 8192 453 -> 331 (8:
+// a slice's workspace is read while it is still in the last-level cache); 8 heads, 4096 tokens 160 -> 147 (2); 4 heads,
+// 9580 tokens 334 -> 306 (3); D = 64, 16 heads, 4096 tokens 109 -> 104 (4).
+template <int D>
+int slices32(int N, int nct, int Hv, int n_cu) {
+  constexpr double item = D == 128 ? 19. : 9., chunk = D == 128 ? 2. : 1., launch = 2.;
+  // CUs of the state pass, on the XCDs that have most of it, and left beside it (the items spread over all XCDs)
+  const int ns = state_grid<D>(N * Hv), rest = n_cu - ns;
+  if (ns > n_cu / 2) return 1;
+  auto prep = [&](int n, int cus) { return item * ((N * n * Hv + cus - 1) / cus); };
+  const double plain = prep(nct, n_cu) + chunk * nct;
+  double best = 0.97 * plain;
+  int slices = 1;
+  for (int k = 2; k <= 8 && 4 * k <= nct; ++k) {
+    const int n = (nct + k - 1) / k;  // (the last slice may be shorter)
+    const double t = prep(n, n_cu) + (k - 1) * (std::max(chunk * n + launch, prep(n, rest)) + launch) + chunk * n;
+    if (t < best) {
+      best = t;
+      slices = k;
+    }
+  }
+  return slices;
+}
+
 template <typename TIn, typename TG, int D, bool GATE>
-int launch_prep32(const char* fn, int n_items, const void* q, const void* k, const void* v, const void* g,
-                  const void* beta, const float* A_log, const float* dt_bias, const int32_t* cu,
-                  const int32_t* chunk_idx, int n_seqs, int T, int Hk, int Hv, float scale, int qk_l2norm,
-                  const RowStrides& rs, uint8_t* ws, hipStream_t s) {
-  static std::atomic<signed char> state[C32_MAX_DEVICES];
+int launch32(const char* fn, Prep32<TIn, TG> p, State32<TIn> st, int N, int nct, hipStream_t s) {
+  static std::atomic<signed char> prep_lds[C32_MAX_DEVICES], both_lds[C32_MAX_DEVICES];
   constexpr int bytes = Lds32<D>::BYTES;
-  if (bytes > 65536 && !lds_ready(chunk32_prep_kernel<TIn, TG, D, GATE>, bytes, state))
+  if (!lds_ready(chunk32_prep_kernel<TIn, TG, D, GATE>, bytes, prep_lds))
     return fail(ZGDN_EHIP, "%s: the device refused %d bytes of LDS for the fp32 chunk kernel", fn, bytes);
-  hipLaunchKernelGGL((chunk32_prep_kernel<TIn, TG, D, GATE>), dim3(std::min(n_items, device_cus())),
-                     dim3(64 * P32_WAVES), bytes, s, (const TIn*)q, (const TIn*)k, (const TIn*)v, (const TG*)g,
-                     (const TG*)beta, A_log, dt_bias, cu, chunk_idx, n_seqs, n_items, T, Hk, Hv, scale, qk_l2norm,
-                     rs, ws);
-  return ZGDN_OK;
+  const int n_cu = device_cus(), n_state = state_grid<D>(N * p.Hv);
+  // the states between slices stay in s_out; packed sequences (of different lengths) are not sliced
+  int k = p.cu == nullptr && st.s_out != nullptr ? slices32<D>(N, nct, p.Hv, n_cu) : 1;
+  if (k > 1 && !lds_ready(chunk32_both_kernel<TIn, TG, D, GATE>, bytes, both_lds)) k = 1;
+  const int n = k > 1 ? (nct + k - 1) / k : p.at.n;
+  auto prep_of = [&](int lo) {
+    Prep32<TIn, TG> x = p;
+    if (k > 1) {
+      x.at = Items32{lo, std::min(n, nct - lo), nct};
+      x.n_items = N * x.at.n * p.Hv;
+    }
+    return x;
+  };
+  if (p.n_items > 0) {
+    const Prep32<TIn, TG> x = prep_of(0);
+    hipLaunchKernelGGL((chunk32_prep_kernel<TIn, TG, D, GATE>), dim3(std::min(x.n_items, n_cu)), dim3(64 * P32_WAVES), bytes,
+                       s, x);
+  }
+  if (k > 1) {
+    st.n = n;
+    for (; st.lo + n < nct; st.lo += n) {
+      const Prep32<TIn, TG> x = prep_of(st.lo + n);
+      const int rest = std::min(x.n_items, n_cu - n_state);
+      hipLaunchKernelGGL((chunk32_both_kernel<TIn, TG, D, GATE>), dim3(n_state + rest), dim3(64 * P32_WAVES), bytes, s, x, st,
+                         n_state);
+      st.s_in = st.s_out;
+    }
+  }
+  hipLaunchKernelGGL((chunk32_state_kernel<TIn, D>), dim3(n_state), dim3(512), 0, s, st);
+  return check_launch(fn);
 }
 
 template <typename TIn, int D>
@@ -667,27 +780,18 @@ int run32(const char* fn, int n_chunks, const void* q, const void* k, const void
           const void* beta, const float* A_log, const float* dt_bias, const int32_t* cu, const int32_t* chunk_idx,
           int N, int T, int Hk, int Hv, float scale, int qk_l2norm, const RowStrides& rs, const float* s_in,
           float* s_out, void* o, uint8_t* ws, hipStream_t s) {
-  const int n_items = n_chunks * Hv;
-  if (n_items > 0) {
-    const bool gate = A_log != nullptr;
-    int st;
-    if (gb_dtype == ZGDN_F32)
-      st = gate ? launch_prep32<TIn, float, D, true>(fn, n_items, q, k, v, g, beta, A_log, dt_bias, cu, chunk_idx, N,
-                                                     T, Hk, Hv, scale, qk_l2norm, rs, ws, s)
-                : launch_prep32<TIn, float, D, false>(fn, n_items, q, k, v, g, beta, A_log, dt_bias, cu, chunk_idx,
-                                                      N, T, Hk, Hv, scale, qk_l2norm, rs, ws, s);
-    else
-      st = gate ? launch_prep32<TIn, bf16, D, true>(fn, n_items, q, k, v, g, beta, A_log, dt_bias, cu, chunk_idx, N,
-                                                    T, Hk, Hv, scale, qk_l2norm, rs, ws, s)
-                : launch_prep32<TIn, bf16, D, false>(fn, n_items, q, k, v, g, beta, A_log, dt_bias, cu, chunk_idx, N,
-                                                     T, Hk, Hv, scale, qk_l2norm, rs, ws, s);
-    if (st != ZGDN_OK) return st;
-  }
-  constexpr int NK = D / 16;
-  const long pairs = (long)N * Hv;
-  const dim3 grid((unsigned)(((pairs + 7) / 8) * 8 * NK));
-  hipLaunchKernelGGL((chunk32_state_kernel<TIn, D>), grid, dim3(512), 0, s, ws, s_in, s_out, (TIn*)o, cu, N, n_chunks, T, Hv);
-  return check_launch(fn);
+  const int nct = (T + CHUNK_LEN - 1) / CHUNK_LEN;
+  const State32<TIn> st{ws, s_in, s_out, (TIn*)o, cu, N, n_chunks, T, Hv, 0, std::max(1, n_chunks)};
+  auto go = [&](auto* tag, auto gate) {
+    using TG = std::remove_pointer_t<decltype(tag)>;
+    const Prep32<TIn, TG> p{(const TIn*)q, (const TIn*)k, (const TIn*)v, (const TG*)g, (const TG*)beta, A_log, dt_bias, cu,
+                            chunk_idx, N, n_chunks * Hv, T, Hk, Hv, qk_l2norm, scale, rs, ws,
+                            Items32{0, std::max(1, n_chunks), 0}};
+    return launch32<TIn, TG, D, decltype(gate)::value>(fn, p, st, N, nct, s);
+  };
+  if (gb_dtype == ZGDN_F32)
+    return A_log != nullptr ? go((float*)nullptr, std::true_type{}) : go((float*)nullptr, std::false_type{});
+  return A_log != nullptr ? go((bf16*)nullptr, std::true_type{}) : go((bf16*)nullptr, std::false_type{});
 }
 
 }  // namespace
