@@ -28,3 +28,15 @@ def test_chunk_counts_and_strong_decay(gdn, cuda, lengths, H, decay):
     torch.cuda.synchronize()
     o_ref, s_ref = O.gated_delta_recurrence(d["q"], d["k"], d["v"], g, d["beta"], None, d["s0"], cu_seqlens=cu)
     assert max_abs(o, o_ref) < 2e-2 and rel_err(s, s_ref) < 1e-3, (max_abs(o, o_ref), rel_err(s, s_ref))
+
+
+@pytest.mark.parametrize("T,H", [(1665, 4), (1728, 4), (1921, 1), (2048, 4), (2433, 4), (2303, 8)])
+def test_plain_and_segmented_around_the_plan_line(gdn, cuda, T, H):
+    """Prompts around the length from which the state pass is cut into segments (27 chunks of up to 4 heads, 36 of 8),
+    partial last chunks and last segments included: whichever form the plan takes meets the bounds of the path."""
+    announce(f"chunk plan line T={T} H={H}")
+    d = O.make_inputs(1, T, H, H, 128, 128, seed=T + H, dtype=torch.bfloat16, state_std=0.02, n_states=1)
+    o, s = gdn.chunk_fwd(*(d[n].to(cuda) for n in ("q", "k", "v", "g", "beta")), initial_state=d["s0"].to(cuda))
+    torch.cuda.synchronize()
+    o_ref, s_ref = O.gated_delta_recurrence(d["q"], d["k"], d["v"], d["g"], d["beta"], None, d["s0"])
+    assert max_abs(o, o_ref) < 2e-2 and rel_err(s, s_ref) < 1e-3, (max_abs(o, o_ref), rel_err(s, s_ref))
