@@ -1746,9 +1746,10 @@ __global__ __launch_bounds__(256) void chunk_correct_kernel(const uint16_t* __re
 // MI355X, one sequence (graph replay, hundredths of a microsecond): the plain pass 66 a chunk; a segmented one 104 a
 // chunk of a segment (the correction's rows among them; segments below 10 chunks take as long as 10), 217 a combine
 // step and 270 fixed. A segment count in 2 .. 8 is taken when its local and transition workgroups all fit one per CU
-// and it is the cheapest. The call at 4 heads, plain / 4 segments, us: T = 1536 28.2 / 31.0, 1792 31.1 / 32.0, 2048
-// 33.9 / 32.6, 2304 36.8 / 32.3, 4096 53.8 / 37.2, 8192 96.4 / 54.2; 8 heads, plain / 2 segments: 2560 40.7 / 38.4,
-// 3072 46.2 / 41.4, 4096 57.5 / 48.3; 1 head, 4 / 5 segments: 2560 29.9 / 30.8. (With 64 a chunk, 80 a chunk of a
+// and it is the cheapest, for more than 32 chunks: up to there callers count on no extra workspace, and segments gain
+// 2.4 us at most. The call at 4 heads, plain / segmented, us: T = 1536 28.2 / 31.0, 1792 31.2 / 30.6, 2048 34.2 / 31.8,
+// 2304 36.7 / 33.0, 4096 53.8 / 37.2, 8192 96.4 / 54.2; 8 heads: 2304 37.9 / 37.1, 2560 40.7 / 38.4, 3072 46.2 / 41.4,
+// 4096 57.5 / 48.3; 1 head, 4 / 5 segments: 2560 29.9 / 30.8. (With 64 a chunk, 80 a chunk of a
 // segment, 207 and 985, measured on an earlier state pass, 4 heads went over from 2432 tokens and 8 heads from 3200.)
 // NV: value blocks of 16 rows per state-pass workgroup. Two when the plain pass's workgroups of one block
 // would outnumber the CUs (more than n_cu / 8 chains): each then reads a chunk's shared operands (W or Q',
@@ -1764,11 +1765,11 @@ SegPlan seg_plan(int B, int T, int Hv, int n_cu) {
   const int nct = (T + CH - 1) / CH;
   const long base = (long)B * Hv * (DV / VB);
   SegPlan p{1, nct, state_nv((long)B * Hv, n_cu)};
-  if (nct < 8 || 2 * base > n_cu) return p;  // (a segment holds at least 4 chunks)
+  if (nct <= 32 || 2 * base > n_cu) return p;  // (prompts of up to 2048 tokens need no extra workspace)
   long best = 66L * nct;
   for (int g = 2; g <= 8; ++g) {
     const int cs = (nct + g - 1) / g, gg = (nct + cs - 1) / cs;
-    if (cs < 4 || gg < 2 || base * (2 * gg - 1) > n_cu) continue;
+    if (gg < 2 || base * (2 * gg - 1) > n_cu) continue;
     const long cost = 270 + 104L * std::max(cs, 10) + 217L * (gg - 1);
     if (cost < best) {
       best = cost;
