@@ -94,3 +94,14 @@ def test_in_place_extend_equals_the_general_path(gdn, cuda, name, calls, exact):
             assert torch.equal(a._window[s, :fill], b._window[s, :fill]), (rows, s)
         others = [s for s in range(capacity) if s not in held]
         assert bool((a._live_state[others] == 0.5).all()) and bool((a._window[others] == 0.25).all())
+
+
+def test_a_call_of_no_requests_returns_no_rows(gdn, cuda):
+    serving = importlib.import_module("zonos3-mini_amd.serving")
+    announce("serving extend of no requests")
+    for layer, batch in _pair(serving, cuda, 256, 3, 5300)[0]:
+        layer._window.fill_(0.25)
+        y = layer.forward(torch.empty(0, 256, dtype=torch.bfloat16, device=cuda))
+        torch.cuda.synchronize()
+        assert y.shape == (0, 256) and y.dtype == torch.bfloat16
+        assert bool((layer._window == 0.25).all()) and not layer._win_len.any() and layer._owners == [None] * 3

@@ -193,6 +193,23 @@ def test_plan_extend_splits_each_joined_run_at_its_last_chunk(serving):
     assert open_.member_of_row == [0] * 6 + [2] * 5
 
 
+@pytest.mark.parametrize("runs", [[], [(0, 5)], [(0, 64)], [(70, 58), (0, 130), (131, 2), (64, 1)]])
+def test_run_tables_hold_five_numbers_a_run(serving, runs):
+    """The run tables of an in-place extend for (cached, new) runs: cu, slots, replayed rows, first rows in x, fresh
+    flags, then the chunk pairs -- 5 n + 1 + 2 chunks numbers, a call without requests included."""
+    reqs = [serving.Request(slot=7 - i, owner=(i, False), cached=c, new=n) for i, (c, n) in enumerate(runs)]
+    flat, rows, n_chunks = serving.run_tables(reqs)
+    joined = [c % 64 + n for c, n in runs]
+    cu, pairs = O.chunk_tables(joined)
+    assert rows == sum(joined) and n_chunks == len(pairs) and len(flat) == 5 * len(runs) + 1 + 2 * n_chunks
+    at, n = len(runs) + 1, len(runs)
+    assert flat[:at] == list(cu) and flat[at:at + n] == [7 - i for i in range(n)]
+    assert flat[at + n:at + 2 * n] == [c % 64 for c, _ in runs]
+    assert flat[at + 2 * n:at + 3 * n] == [sum(m for _, m in runs[:i]) for i in range(n)]
+    assert flat[at + 3 * n:at + 4 * n] == [int(c == 0) for c, _ in runs]
+    assert flat[at + 4 * n:] == [v for pair in pairs for v in pair]
+
+
 def test_static_prefill_bookkeeping(serving):
     """A padded static prefill (PrefillLayout of complete-chunk counts 0, 2, 1) with the packed pass replaced by
     ``_transparent_packed`` (extended with a projection stand-in, mixed = x tiled to the in_proj width):

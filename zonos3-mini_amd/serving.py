@@ -215,7 +215,7 @@ def run_tables(reqs: list[Request]) -> tuple[list[int], int, int]:
     replayed rows, first row in x, fresh flags (n each), then the (run, chunk) pairs -- with the numbers of
     packed rows and of chunks. Per request and chunk; nothing per row."""
     cu, pairs = _table_lists([r.replay + r.new for r in reqs])
-    first = list(itertools.accumulate((r.new for r in reqs[:-1]), initial=0))
+    first = list(itertools.accumulate((r.new for r in reqs), initial=0))[:-1]
     flat = cu + [r.slot for r in reqs] + [r.replay for r in reqs] + first + [int(r.cached == 0) for r in reqs] + pairs
     return flat, cu[-1], len(pairs) // 2
 
@@ -360,7 +360,8 @@ class OriginalGDN:
         if mask is not None:  # a request's adapters: the mask row of its first new row
             firsts = list(itertools.accumulate((r.new for r in reqs[:-1]), initial=0))
             mask = mask.index_select(0, device_tensor(firsts, torch.long, mask.device))
-        in_place = not batch.is_decode and mask is None and self._extends_in_place(x)
+        # (a call of no requests launches nothing: the plan's route returns its empty rows)
+        in_place = bool(reqs) and not batch.is_decode and mask is None and self._extends_in_place(x)
         fresh = [] if in_place else [r.slot for r in reqs if r.cached == 0]
         if fresh:
             self._reset_slots(device_tensor(fresh, torch.long, x.device))
