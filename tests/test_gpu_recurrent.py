@@ -75,6 +75,18 @@ def test_decode_step_in_place_chain_equals_recurrence(gdn, cuda):
     _check(torch.stack(outs, 1), state.cpu(), o_ref, s_ref, bf16=True)
 
 
+def test_decode_step_without_a_state(gdn, cuda):
+    """state=None: one step from a zero state; another object in its place gets the call's own error."""
+    announce("decode_step without a state")
+    d = O.make_inputs(3, 1, 2, 4, 128, 128, seed=1011, dtype=torch.bfloat16)
+    args = [d[n][:, 0].contiguous().to(cuda) for n in ("q", "k", "v", "g", "beta")]
+    zero = torch.zeros(3, 4, 128, 128, device=cuda)
+    assert torch.equal(gdn.decode_step(*args, None), gdn.decode_step(*args, zero))
+    assert bool(zero.any())  # a given state is updated in place
+    with pytest.raises(RuntimeError, match="initial_state: expected a tensor"):
+        gdn.decode_step(*args, [0.0])
+
+
 @pytest.mark.parametrize("hk,hv", [(1, 2), (2, 4), (8, 16)])
 def test_grouped_value_heads(gdn, cuda, hk, hv):
     announce(f"recurrent grouped heads Hk={hk} Hv={hv}")

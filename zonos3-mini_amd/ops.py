@@ -252,16 +252,16 @@ def recurrent_fwd(q, k, v, g, beta, scale=None, initial_state=None, output_final
 def decode_step(q, k, v, g, beta, state, scale=None):
     """One single-token step for B independent streams, updating ``state`` in place.
 
-    q, k [B, Hk, K]; v [B, Hv, V]; g (log decay), beta [B, Hv]; state [B, Hv, V, K] float32.
-    Returns o [B, Hv, V] in v's dtype (the recurrence of lm.py:574-583 at T = 1)."""
+    q, k [B, Hk, K]; v [B, Hv, V]; g (log decay), beta [B, Hv]; state [B, Hv, V, K] float32, or None for one step from
+    a zero state that is not kept. Returns o [B, Hv, V] in v's dtype (the recurrence of lm.py:574-583 at T = 1)."""
     if not (q.dim() == 3 and v.dim() == 3):
         raise RuntimeError("decode_step: q, k [B, Hk, K] and v [B, Hv, V] expected")
     # what recurrent_fwd checks, in one expression (this call's host time is near the step's own); a call that
     # fails it goes there for the message
     dt, gdt, idx = q.dtype, g.dtype, q.get_device()
     (B, Hk, K), (Bv, Hv, V) = q.shape, v.shape
-    if (idx >= 0 and Bv == B and Hk and Hv % Hk == 0 and dt in _CODES and gdt in _CODES and k.shape == q.shape
-            and k.dtype is dt and v.dtype is dt and beta.dtype is gdt and g.shape == beta.shape == (B, Hv)
+    if (idx >= 0 and isinstance(state, torch.Tensor) and Bv == B and Hk and Hv % Hk == 0 and dt in _CODES
+            and gdt in _CODES and k.shape == q.shape and k.dtype is dt and v.dtype is dt and beta.dtype is gdt and g.shape == beta.shape == (B, Hv)
             and state.dtype is torch.float32 and state.shape == (B, Hv, V, K)
             and k.get_device() == v.get_device() == g.get_device() == beta.get_device() == state.get_device() == idx
             and q.is_contiguous() and k.is_contiguous() and v.is_contiguous() and g.is_contiguous()
