@@ -227,13 +227,21 @@ def run_tables(reqs: list[Request]) -> tuple[list[int], int, int]:
 FEW_ROWS = 128
 
 
+def _takes_few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether F.linear(x, w) of a decode step is the split-K kernel's: up to FEW_ROWS rows of bf16 operands that it
+    reads in place (K in whole slices, 16-byte pieces from aligned bases). A weight or rows of a tensor subclass, which
+    may hold its elements in another form, and a product that autograd records stay F.linear's."""
+    plain = (torch.Tensor, torch.nn.Parameter)
+    return (x.is_cuda and x.shape[0] <= FEW_ROWS and x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2
+            and type(x) in plain and type(w) in plain and x.is_contiguous() and w.is_contiguous()
+            and x.shape[1] == w.shape[1] and w.shape[1] % 128 == 0 and w.shape[0] % 8 == 0 and w.device == x.device
+            and not (x.data_ptr() | w.data_ptr()) % 16
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
+
+
 def _few_rows(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """F.linear(x, w) for a decode step's rows."""
-    if (x.is_cuda and x.shape[0] <= FEW_ROWS and x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2
-            and w.is_contiguous() and x.shape[1] == w.shape[1] and w.shape[1] % 128 == 0 and w.shape[0] % 8 == 0
-            and w.data_ptr() % 16 == 0 and w.device == x.device):
-        return ops.gemm_rows(x, w)
-    return F.linear(x, w)
+    return ops.gemm_rows(x, w) if _takes_few_rows(x, w) else F.linear(x, w)
 
 
 class _Weight:
