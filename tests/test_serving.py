@@ -210,6 +210,15 @@ def test_run_tables_hold_five_numbers_a_run(serving, runs):
     assert flat[at + 4 * n:] == [v for pair in pairs for v in pair]
 
 
+@pytest.mark.parametrize("n_out,n_in,rows", [(2056, 256, 128), (2056, 1024, 128), (2056, 2560, 128), (2056, 2688, 64),
+                                             (2056, 4096, 64), (2056, 4224, 16), (2056, 8192, 16), (2056, 8320, 0),
+                                             (3584, 512, 128), (3592, 512, 64), (4096, 512, 64), (4104, 512, 16)])
+def test_rows_of_the_split_k_projection(serving, n_out, n_in, rows):
+    """The rows of a decode step's projection that take the split-K kernel fall as the weight widens: measured behind
+    the library's product at 96 rows from K = 2816, 32 rows at 8192, and at 112 rows of 4096 columns."""
+    assert serving._few_rows_limit(n_out, n_in) == rows
+
+
 def test_static_prefill_bookkeeping(serving):
     """A padded static prefill (PrefillLayout of complete-chunk counts 0, 2, 1) with the packed pass replaced by
     ``_transparent_packed`` (extended with a projection stand-in, mixed = x tiled to the in_proj width):

@@ -220,20 +220,28 @@ def run_tables(reqs: list[Request]) -> tuple[list[int], int, int]:
     return flat, cu[-1], len(pairs) // 2
 
 
-# The rows up to which a decode step's projections take the package's split-K kernel. Per call in a graph, us, the
-# kernel / torch's F.linear (MI355X, bf16): in_proj (1024 -> 2056) at 1 row 3.1 / 5.8, 32 rows 3.6 / 8.1, 64 rows
-# 4.4 / 8.5, 128 rows 6.3 / 9.1, 192 rows 8.2 / 8.5, 256 rows 10.1 / 8.9; wo (512 -> 1024) 2.3 / 3.6, 2.5 / 4.8,
-# 2.6 / 5.5, 3.0 / 6.5, 4.0 / 4.9, 4.3 / 6.6.
-FEW_ROWS = 128
+def _few_rows_limit(n_out: int, n_in: int) -> int:
+    """The rows up to which a decode step's projection takes the package's split-K kernel. A workgroup holds 16 rows x
+    16 columns and every 1,024 of K is a round trip of its own, so the kernel loses its lead over the library's tiles
+    as rows, columns and K grow. Per call in a graph over 16 weights in turn, us, the kernel / torch's F.linear
+    (MI355X, bf16): in_proj (hidden -> 2056) at hidden 1024, 1 row 3.1 / 5.8, 32 rows 3.6 / 8.2, 128 rows 6.4 / 9.2 (192
+    rows 8.2 / 8.5, 256 rows 10.1 / 8.9); 2560, 96 rows 8.5 / 9.6, 128 rows 10.0 / 13.6; 2816, 64 rows 7.6 / 10.6, 96
+    rows 9.1 / 8.1; 4096, 64 rows 10.4 / 13.3, 96 rows 12.4 / 11.9; 8192, 16 rows 12.2 / 13.0, 32 rows 16.6 / 15.9. wo
+    (512 -> hidden) at hidden 1024, 128 rows 2.9 / 6.5; 3584, 112 rows 6.7 / 7.0; 4096, 64 rows 4.7 / 7.1, 112 rows 7.5
+    / 7.0; 8192, 16 rows 3.6 / 7.4, 64 rows 7.8 / 7.3."""
+    if n_in <= 2560 and n_out <= 3584:
+        return 128
+    widest = max(n_in, n_out)
+    return 64 if widest <= 4096 else 16 if widest <= 8192 else 0
 
 
 def _takes_few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether F.linear(x, w) of a decode step is the split-K kernel's: up to FEW_ROWS rows of bf16 operands that it
-    reads in place (K in whole slices, 16-byte pieces from aligned bases). A weight or rows of a tensor subclass, which
-    may hold its elements in another form, and a product that autograd records stay F.linear's."""
+    """Whether F.linear(x, w) of a decode step is the split-K kernel's: few rows (``_few_rows_limit``) of bf16 operands
+    that it reads in place (K in whole slices, 16-byte pieces from aligned bases). A weight or rows of a tensor
+    subclass, which may hold its elements in another form, and a product that autograd records stay F.linear's."""
     plain = (torch.Tensor, torch.nn.Parameter)
-    return (x.is_cuda and x.shape[0] <= FEW_ROWS and x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2
-            and type(x) in plain and type(w) in plain and x.is_contiguous() and w.is_contiguous()
+    return (x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2
+            and x.shape[0] <= _few_rows_limit(*w.shape) and type(x) in plain and type(w) in plain and x.is_contiguous() and w.is_contiguous()
             and x.shape[1] == w.shape[1] and w.shape[1] % 128 == 0 and w.shape[0] % 8 == 0 and w.device == x.device
             and not (x.data_ptr() | w.data_ptr()) % 16
             and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
