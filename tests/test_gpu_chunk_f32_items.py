@@ -50,3 +50,29 @@ def test_many_items_ragged(gdn, cuda, D, Hk, Hv, gate):
     eo, es = rel_err(o, o_ref), rel_err(s, s_ref)
     print(f"fp32 items D={D}: output rel err {eo:.2e}, state rel err {es:.2e}")
     assert eo < TOL and es < TOL, (eo, es)
+
+
+@pytest.mark.parametrize("D,dtype,far_gates", [(128, torch.float32, False), (128, torch.float32, True),
+                                               (64, torch.bfloat16, True), (64, torch.float32, False)])
+def test_rows_far_apart(gdn, cuda, D, dtype, far_gates):
+    """Rows 64 MiB apart (a chunk of them is past 4 GiB) give the results of dense rows, bit for bit."""
+    announce(f"chunk f32 rows far apart D={D} {dtype} gates {far_gates}")
+    T, H = 65, 2
+    gen = torch.Generator(device=cuda).manual_seed(43 + D)
+    q, k, v = (torch.randn(1, T, H, D, generator=gen, device=cuda).to(dtype) for _ in range(3))
+    g = -torch.rand(1, T, H, generator=gen, device=cuda).to(dtype)
+    beta = torch.rand(1, T, H, generator=gen, device=cuda).to(dtype)
+    ld = 2**26 // dtype.itemsize + 64
+    buf = torch.empty(T * ld, dtype=dtype, device=cuda).view(T, ld)
+
+    def far(x, col):
+        view = buf[:, col:col + x[0, 0].numel()].view(1, *x.shape[1:])
+        view.copy_(x)
+        return view
+
+    wide = [far(x, 512 * i) for i, x in enumerate((q, k, v))]
+    gates = [far(x, 512 * i + 256 + 8) for i, x in enumerate((g, beta))] if far_gates else [g, beta]
+    o, s = gdn.chunk_fwd(*wide, *gates, use_qk_l2norm=True)
+    o_ref, s_ref = gdn.chunk_fwd(q, k, v, g, beta, use_qk_l2norm=True)
+    assert wide[0].stride(1) == ld and bool(o_ref.any())
+    assert torch.equal(o, o_ref) and torch.equal(s, s_ref)

@@ -103,8 +103,8 @@ __device__ __forceinline__ void tri_tile(int t, int& rb, int& cb) {
   cb = t - rb * (rb + 1) / 2;
 }
 
-// Four consecutive elements of a q / k / v row as loaded through a buffer resource (zeros past its range), and
-// as floats.
+// Four consecutive elements of a q / k / v row as loaded through a buffer resource (zeros past its range) or from a
+// pointer (zeros where it is null), and as floats.
 template <typename T>
 struct Row4;
 template <>
@@ -112,6 +112,9 @@ struct Row4<float> {
   f32x4 v;
   __device__ __forceinline__ void load(Rsrc r, uint32_t off) {
     v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+  }
+  __device__ __forceinline__ void load(const float* p) {
+    v = p != nullptr ? *reinterpret_cast<const f32x4*>(p) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
   __device__ __forceinline__ f32x4 get() const { return v; }
 };
@@ -121,6 +124,9 @@ struct Row4<bf16> {
   u32x2 v;
   __device__ __forceinline__ void load(Rsrc r, uint32_t off) {
     v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+  }
+  __device__ __forceinline__ void load(const bf16* p) {
+    v = p != nullptr ? *reinterpret_cast<const u32x2*>(p) : u32x2{0u, 0u};
   }
   __device__ __forceinline__ f32x4 get() const {
     return f32x4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
@@ -156,12 +162,14 @@ struct GateReg<float> {
   __device__ __forceinline__ void load(Rsrc r, uint32_t off) {
     v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
   }
+  __device__ __forceinline__ void load(const float* p) { v = p != nullptr ? *p : 0.f; }
   __device__ __forceinline__ float get() const { return v; }
 };
 template <>
 struct GateReg<bf16> {
   uint16_t v;
   __device__ __forceinline__ void load(Rsrc r, uint32_t off) { v = __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0); }
+  __device__ __forceinline__ void load(const bf16* p) { v = p != nullptr ? *reinterpret_cast<const uint16_t*>(p) : 0; }
   __device__ __forceinline__ float get() const { return bf16_to_f32(v); }
 };
 
@@ -209,6 +217,28 @@ __device__ __forceinline__ void load_item(Rows32<TIn, TG, D>& x, int item, const
   x.beta.load(raw_rsrc(beta + t, gbytes), goff);
 }
 
+// load_item for rows so far apart (64 of them 4 GiB or more) that a buffer resource, whose range and offsets are 32
+// bits, does not reach the chunk's last ones: from pointers.
+template <typename TIn, typename TG, int D>
+__device__ __forceinline__ void load_item_far(Rows32<TIn, TG, D>& x, int item, const Items32& at, const TIn* q, const TIn* k,
+                                              const TIn* v, const TG* g, const TG* beta, const int32_t* cu,
+                                              const int32_t* chunk_idx, int n_seqs, int T, int Hk, int Hv,
+                                              const RowStrides& rs) {
+  const int c = at.chunk(item / Hv), h = item % Hv, hk = h / (Hv / Hk);
+  const ChunkRange cr = chunk_range(c, cu, chunk_idx, T, n_seqs);
+  const int r = threadIdx.x >> 4, c0 = (threadIdx.x & 15) * 4, lane = threadIdx.x & 63;
+  auto rows = [&](const TIn* p, long ld, int col, Row4<TIn>* out) {
+#pragma unroll
+    for (int j = 0; j < D / 64; ++j) out[j].load(r < cr.len ? p + (size_t)(cr.t0 + r) * ld + col + c0 + 64 * j : nullptr);
+  };
+  rows(q, rs.q, hk * D, x.q);
+  rows(k, rs.k, hk * D, x.k);
+  rows(v, rs.v, h * D, x.v);
+  const size_t t = (size_t)(cr.t0 + lane) * rs.gb + h;
+  x.g.load(lane < cr.len ? g + t : nullptr);
+  x.beta.load(lane < cr.len ? beta + t : nullptr);
+}
+
 // The inputs of phase 1.
 template <typename TIn, typename TG>
 struct Prep32 {
@@ -224,7 +254,7 @@ struct Prep32 {
 };
 
 // Items first, first + stride, .. by one workgroup.
-template <typename TIn, typename TG, int D, bool GATE>
+template <typename TIn, typename TG, int D, bool GATE, bool FAR>
 __device__ __forceinline__ void prep32(uint8_t* lb, const Prep32<TIn, TG>& p, int first, int stride) {
   using L = Lds32<D>;
   using WS = Ws32<D>;
@@ -234,7 +264,10 @@ __device__ __forceinline__ void prep32(uint8_t* lb, const Prep32<TIn, TG>& p, in
   Rows32<TIn, TG, D> R;
   if (first >= n_items) return;
   auto load = [&](int item) {
-    load_item<TIn, TG, D>(R, item, p.at, p.q, p.k, p.v, p.g, p.beta, p.cu, p.chunk_idx, p.n_seqs, p.T, p.Hk, Hv, p.rs);
+    if constexpr (FAR)
+      load_item_far<TIn, TG, D>(R, item, p.at, p.q, p.k, p.v, p.g, p.beta, p.cu, p.chunk_idx, p.n_seqs, p.T, p.Hk, Hv, p.rs);
+    else
+      load_item<TIn, TG, D>(R, item, p.at, p.q, p.k, p.v, p.g, p.beta, p.cu, p.chunk_idx, p.n_seqs, p.T, p.Hk, Hv, p.rs);
   };
   load(first);
 
@@ -481,10 +514,10 @@ __device__ __forceinline__ void prep32(uint8_t* lb, const Prep32<TIn, TG>& p, in
   }
 }
 
-template <typename TIn, typename TG, int D, bool GATE>
+template <typename TIn, typename TG, int D, bool GATE, bool FAR>
 __global__ __launch_bounds__(64 * P32_WAVES) void chunk32_prep_kernel(const Prep32<TIn, TG> p) {
   extern __shared__ f32x4 lds32[];
-  prep32<TIn, TG, D, GATE>(reinterpret_cast<uint8_t*>(lds32), p, blockIdx.x, gridDim.x);
+  prep32<TIn, TG, D, GATE, FAR>(reinterpret_cast<uint8_t*>(lds32), p, blockIdx.x, gridDim.x);
 }
 
 // ----------------------------------------------------------------------------------------------- phase 2
@@ -683,7 +716,7 @@ __global__ __launch_bounds__(64 * P32_WAVES) void chunk32_both_kernel(const Prep
     if (threadIdx.x >= 512) return;  // (whole waves; the barriers count the waves that are left)
     state32<TIn, D>(*reinterpret_cast<StateShared32<D>*>(lds32), st, blockIdx.x);
   } else {
-    prep32<TIn, TG, D, GATE>(reinterpret_cast<uint8_t*>(lds32), p, blockIdx.x - n_state, gridDim.x - n_state);
+    prep32<TIn, TG, D, GATE, false>(reinterpret_cast<uint8_t*>(lds32), p, blockIdx.x - n_state, gridDim.x - n_state);
   }
 }
 
@@ -737,15 +770,21 @@ int slices32(int N, int nct, int Hv, int n_cu) {
   return slices;
 }
 
+// Whether a chunk of rows `ld` elements apart is past a buffer resource's 32-bit range.
+inline bool far_rows(long ld, size_t elem) { return (unsigned long long)ld * CHUNK_LEN * elem > UINT32_MAX; }
+
 template <typename TIn, typename TG, int D, bool GATE>
 int launch32(const char* fn, Prep32<TIn, TG> p, State32<TIn> st, int N, int nct, hipStream_t s) {
-  static std::atomic<signed char> prep_lds[C32_MAX_DEVICES], both_lds[C32_MAX_DEVICES];
+  static std::atomic<signed char> prep_lds[2][C32_MAX_DEVICES], both_lds[C32_MAX_DEVICES];
   constexpr int bytes = Lds32<D>::BYTES;
-  if (!lds_ready(chunk32_prep_kernel<TIn, TG, D, GATE>, bytes, prep_lds))
+  const bool far = far_rows(std::max({p.rs.q, p.rs.k, p.rs.v}), sizeof(TIn)) || far_rows(p.rs.gb, sizeof(TG));
+  auto prep_kernel = far ? chunk32_prep_kernel<TIn, TG, D, GATE, true> : chunk32_prep_kernel<TIn, TG, D, GATE, false>;
+  if (!lds_ready(prep_kernel, bytes, prep_lds[far]))
     return fail(ZGDN_EHIP, "%s: the device refused %d bytes of LDS for the fp32 chunk kernel", fn, bytes);
   const int n_cu = device_cus(), n_state = state_grid<D>(N * p.Hv);
-  // the states between slices stay in s_out; packed sequences (of different lengths) are not sliced
-  int k = p.cu == nullptr && st.s_out != nullptr ? slices32<D>(N, nct, p.Hv, n_cu) : 1;
+  // the states between slices stay in s_out; packed sequences (of different lengths) are not sliced, nor are rows
+  // far apart
+  int k = p.cu == nullptr && st.s_out != nullptr && !far ? slices32<D>(N, nct, p.Hv, n_cu) : 1;
   if (k > 1 && !lds_ready(chunk32_both_kernel<TIn, TG, D, GATE>, bytes, both_lds)) k = 1;
   const int n = k > 1 ? (nct + k - 1) / k : p.at.n;
   auto prep_of = [&](int lo) {
@@ -758,8 +797,7 @@ int launch32(const char* fn, Prep32<TIn, TG> p, State32<TIn> st, int N, int nct,
   };
   if (p.n_items > 0) {
     const Prep32<TIn, TG> x = prep_of(0);
-    hipLaunchKernelGGL((chunk32_prep_kernel<TIn, TG, D, GATE>), dim3(std::min(x.n_items, n_cu)), dim3(64 * P32_WAVES), bytes,
-                       s, x);
+    hipLaunchKernelGGL(prep_kernel, dim3(std::min(x.n_items, n_cu)), dim3(64 * P32_WAVES), bytes, s, x);
   }
   if (k > 1) {
     st.n = n;
