@@ -24,6 +24,32 @@ def max_abs(got, want) -> float:
     return float((got - want).abs().max()) if got.numel() else 0.0
 
 
+# Bounds on ``out_errs`` of the bf16 chunk path. An output is Q' S^T + P U: the five values rounded to bf16 on the way
+# (Q', S, P, U and the output itself, half an ulp of at most 2^-9 each, 2^-9 / sqrt(3) in the mean) make about
+# sqrt(5) 2^-9 / sqrt(3) = 2.5e-3 of its size in the mean and at most 5 x 2^-9 = 1e-2 where they all line up (a sequence
+# of a few tokens, 4.8e-3 seen); twice that for one row, whose two terms may partly cancel.
+OUT_RMS, OUT_ROW = 1e-2, 2e-2
+
+
+def out_errs(o, o_ref, cu=None) -> tuple[float, float]:
+    """Errors of outputs [B, T, H, V] (or [T, H, V]) relative to the size of the outputs they stand among: over all
+    (sequence, head) pairs, the largest 2-norm of the error over that of the outputs, and the largest 2-norm of one
+    row's error over the row's size or the rows' mean size, the larger. ``cu``: the bounds of packed sequences (B = 1)."""
+    o, o_ref = (torch.as_tensor(t).detach().cpu().double() for t in (o, o_ref))
+    if o.dim() == 3:
+        o, o_ref = o.unsqueeze(0), o_ref.unsqueeze(0)
+    runs = [(b, 0, o.shape[1]) for b in range(o.shape[0])] if cu is None else [(0, a, e) for a, e in zip(cu, cu[1:])]
+    worst = [0.0, 0.0]
+    for b, a, e in runs:
+        if e == a:
+            continue
+        err, ref = (o[b, a:e] - o_ref[b, a:e]).norm(dim=-1), o_ref[b, a:e].norm(dim=-1)  # [rows, H]
+        size = ref.square().mean(0).sqrt().clamp_min(1e-300)
+        worst[0] = max(worst[0], float((err.square().mean(0).sqrt() / size).max()))
+        worst[1] = max(worst[1], float((err / torch.maximum(ref, size)).max()))
+    return worst[0], worst[1]
+
+
 def announce(msg: str) -> None:
     """Name the case on stderr before a GPU step, flushed, so a fault can be attributed."""
     print(f"[case] {msg}", file=sys.stderr, flush=True)

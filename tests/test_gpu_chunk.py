@@ -1,7 +1,8 @@
 """Chunked prefill kernel (zgdn_chunk_fwd) against the CPU oracle on seeded inputs.
 
-Tolerances (bf16 inputs): outputs within 2e-2 max-abs, float32 final states within 1e-3 relative
-(max|err| / max|ref|).
+Tolerances (bf16 inputs): outputs within 2e-2 max-abs and, relative to the outputs they stand among, within the bounds
+of ``gdn_testing.out_errs`` (the outputs' rms is about 5e-3, so that the absolute bound alone would pass outputs without
+their carried state); float32 final states within 1e-3 relative (max|err| / max|ref|).
 """
 
 from __future__ import annotations
@@ -10,7 +11,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from gdn_testing import announce, max_abs, rel_err
+from gdn_testing import OUT_RMS, OUT_ROW, announce, max_abs, out_errs, rel_err
 from oracle import gdn_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -22,10 +23,12 @@ def _dev(d, cuda, gb_dtype=torch.float32):
     return x
 
 
-def _check(o, s, o_ref, s_ref):
+def _check(o, s, o_ref, s_ref, cu=None):
     eo, es = max_abs(o, o_ref), rel_err(s, s_ref)
-    print(f"[errors] output max-abs {eo:.3e}, state rel {es:.3e}")
+    rms, row = out_errs(o, o_ref, cu)
+    print(f"[errors] output max-abs {eo:.3e}, rms {rms:.3e}, row {row:.3e}, state rel {es:.3e}")
     assert eo < 2e-2 and es < 1e-3, (eo, es)
+    assert rms < OUT_RMS and row < OUT_ROW, (rms, row)
     return eo, es
 
 
@@ -90,7 +93,7 @@ def test_packed_sequences(gdn, cuda):
     o, s = gdn.chunk_fwd(x["q"], x["k"], x["v"], x["g"], x["beta"], initial_state=x["s0"], cu_seqlens=cu_t)
     torch.cuda.synchronize()
     o_ref, s_ref = O.gated_delta_recurrence(d["q"], d["k"], d["v"], d["g"], d["beta"], None, d["s0"], cu_seqlens=cu)
-    _check(o.cpu(), s.cpu(), o_ref, s_ref)
+    _check(o.cpu(), s.cpu(), o_ref, s_ref, cu)
     assert torch.equal(s[3].cpu(), d["s0"][3])  # the empty sequence keeps its state
 
 
@@ -111,7 +114,7 @@ def test_many_short_packed_sequences(gdn, cuda):
     o, s = gdn.chunk_fwd(x["q"], x["k"], x["v"], x["g"], x["beta"], initial_state=x["s0"], cu_seqlens=cu_t)
     torch.cuda.synchronize()
     o_ref, s_ref = O.gated_delta_recurrence(d["q"], d["k"], d["v"], d["g"], d["beta"], None, d["s0"], cu_seqlens=cu)
-    _check(o.cpu(), s.cpu(), o_ref, s_ref)
+    _check(o.cpu(), s.cpu(), o_ref, s_ref, cu)
     for i, n in enumerate(lengths):
         if n == 0:
             assert torch.equal(s[i].cpu(), d["s0"][i])
@@ -298,7 +301,7 @@ def test_overlapped_launch_packed(gdn, cuda, lengths, Hk, Hv):
     assert torch.equal(o1, o0) and torch.equal(s1, s0_)
     assert torch.equal(o2, o0) and torch.equal(s2, s0_)
     o_ref, s_ref = O.gated_delta_recurrence(d["q"], d["k"], d["v"], d["g"], d["beta"], None, d["s0"], cu_seqlens=cu)
-    _check(o1.cpu(), s1.cpu(), o_ref, s_ref)
+    _check(o1.cpu(), s1.cpu(), o_ref, s_ref, cu)
     for i, n in enumerate(lengths):
         if n == 0:
             assert torch.equal(s1[i].cpu(), d["s0"][i])
@@ -372,4 +375,4 @@ def test_random_packed_batches(gdn, cuda, case):
     assert torch.equal(o1, o0) and torch.equal(s1, s0_)
     o_ref, s_ref = O.gated_delta_recurrence(q_ref, k_ref, d["v"].float(), g_log, beta_ref, None,
                                             d["s0"] if c["state"] else None, cu_seqlens=cu)
-    _check(o1.cpu(), s1.cpu(), o_ref, s_ref)
+    _check(o1.cpu(), s1.cpu(), o_ref, s_ref, cu)

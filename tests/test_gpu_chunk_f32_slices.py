@@ -18,11 +18,13 @@ pytestmark = pytest.mark.gpu
 TOL = 2e-5
 
 
-@pytest.mark.parametrize("D,B,T,Hk,Hv", [(128, 1, 4096, 16, 16), (128, 1, 4033, 8, 8), (128, 2, 2999, 4, 8),
-                                         (128, 1, 9580, 2, 4), (128, 1, 3301, 12, 12), (128, 1, 8192, 16, 16),
-                                         (64, 1, 4096, 16, 16), (64, 1, 4095, 4, 8)])
-def test_slices_equal_two_launches(gdn, cuda, D, B, T, Hk, Hv):
+@pytest.mark.parametrize("D,B,T,Hk,Hv,slices", [(128, 1, 4096, 16, 16, 4), (128, 1, 4033, 8, 8, 2),
+                                                (128, 2, 2999, 4, 8, 3), (128, 1, 9580, 2, 4, 3),
+                                                (128, 1, 3301, 12, 12, 3), (128, 1, 8192, 16, 16, 8),
+                                                (64, 1, 4096, 16, 16, 4), (64, 1, 4095, 4, 8, 2)])
+def test_slices_equal_two_launches(gdn, cuda, D, B, T, Hk, Hv, slices):
     announce(f"chunk f32 slices D={D} B={B} T={T} Hv={Hv}")
+    assert gdn._native.lib().zgdn_chunk32_slices(D, B, T, Hv) == slices  # (the call is sliced, as often as listed)
     gen = torch.Generator().manual_seed(5 + T)
     q, k = (O.l2norm(torch.randn(B, T, Hk, D, generator=gen)) for _ in range(2))
     v = torch.randn(B, T, Hv, D, generator=gen)

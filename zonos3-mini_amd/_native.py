@@ -87,6 +87,7 @@ SIGNATURES: dict[str, tuple] = {
 
 # Entry points of this package's own host layer, outside the published header: name -> (restype, argtypes).
 INTERNAL: dict[str, tuple] = {
+    "zgdn_chunk32_slices": (c_int, [c_int, c_int, c_int, c_int]),
     "zgdn_gemm_rows": (c_int, [_P, c_long, _P, _P, c_long, c_int, c_int, c_int, c_int, _P]),
     "zgdn_serving_gather": (
         c_int, [_P, _P, c_int, c_int, _P, c_int, c_int, c_int, c_int, c_int, _P, _P]),

@@ -720,7 +720,7 @@ __global__ __launch_bounds__(64 * P32_WAVES) void chunk32_both_kernel(const Prep
   }
 }
 
-// Phase 1's dynamic LDS is above the default 64 KiB at D = 128: raised once per device and kernel (the first
+// Phase 1's dynamic LDS is above the default 64 KiB (148,736 bytes at D = 128, 99,584 at 64): raised once per device and kernel (the first
 // call on that device); false when the device refuses.
 constexpr int C32_MAX_DEVICES = 64;
 template <typename K>
@@ -853,3 +853,10 @@ int chunk32_fwd(const char* fn, const void* q, const void* k, const void* v, int
 }
 
 }  // namespace zgdn
+
+// Slices that an unpacked call of B sequences with a final state takes on the current device (for tests).
+extern "C" int zgdn_chunk32_slices(int D, int B, int T, int Hv) {
+  using namespace zgdn;
+  const int nct = (T + CHUNK_LEN - 1) / CHUNK_LEN;
+  return D == 64 ? slices32<64>(B, nct, Hv, device_cus()) : slices32<128>(B, nct, Hv, device_cus());
+}
