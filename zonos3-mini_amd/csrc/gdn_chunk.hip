@@ -885,6 +885,8 @@ __device__ __forceinline__ void state_loop(StateSharedT<NV, OW>& sh, const State
   auto fetch2 = [&](Rsrc w, Pre<NV>& x) {
     x.A[2] = ld16(w, offA + 2048u);
     x.A[3] = ld16(w, offA + 3072u);
+  };
+  auto fetch2x = [&](Rsrc w, Pre<NV>& x) {
 #pragma unroll
     for (int v = 0; v < NX; ++v)
       x.X[v] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(w, offX + v * XB, 0, 0));
@@ -921,7 +923,28 @@ __device__ __forceinline__ void state_loop(StateSharedT<NV, OW>& sh, const State
     }
   };
 
-  auto process = [&](int ci, const Pre<NV>& cur, int ni, Pre<NV>& nxt) {
+  // O role, without output waves: the outputs of chunk ci run a chunk late. add_pu (P's fragments in p) stands between
+  // the next chunk's barriers, where the U role has the longer part, put_o behind its state update's products. (P U
+  // and the stores behind the chunk's own update, with U stored ahead of the second barrier, stood in every chunk's
+  // chain: 20 packed sequences of 1 .. 2,000 tokens at 4 heads 65.9 us, 60.9 so, 62.7 with the stores right behind
+  // add_pu; 12 of 16 .. 4,096 104.4, 95.1 and 98.3; 32 of 64 .. 2,048 at 16 heads 486, 485 and 490; the overlapped
+  // launch of T = 4096 at 16 heads 83.8, 79.1 and 78.8.)
+  f32x4 ov[NV], yv[NV];  // Q' S^T of the current chunk; the outputs of the one before
+  auto add_pu = [&](const Pre<NV>& p) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      yv[v] = mfma(__builtin_bit_cast(bf16x8, p.X[0]), frag(&sh.UT[v * VB][0], LDC, 0, 0), ov[v]);
+      if (tb >= 2) yv[v] = mfma(__builtin_bit_cast(bf16x8, p.X[1]), frag(&sh.UT[v * VB][0], LDC, 0, 32), yv[v]);
+    }
+  };
+  auto put_o = [&](int ci) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const float yo[4] = {yv[v][0], yv[v][1], yv[v][2], yv[v][3]};
+      store_o_tile(o, a, a.vb + v, ci, t0, j, yo);
+    }
+  };
+  auto process = [&](int ci, const Pre<NV>& cur, int ni, Pre<NV>& nxt, auto first) {
 #pragma unroll
     for (int v = 0; v < NV; ++v)
 #pragma unroll
@@ -945,8 +968,7 @@ __device__ __forceinline__ void state_loop(StateSharedT<NV, OW>& sh, const State
     }
     lds_barrier();
 
-    float ov[NV][4];  // O role: this wave's outputs
-    f32x4 wx[NV];     // U role: W S^T
+    f32x4 wx[NV];  // U role: W S^T; O role: Q' S^T
     auto put_u = [&](int v) {  // U = Ub - W S^T, as bf16
       *reinterpret_cast<uint2*>(&sh.UT[v * VB + j][t0]) = make_uint2(
           pack_bf16x2(ub[v][0] - wx[v][0], ub[v][1] - wx[v][1]), pack_bf16x2(ub[v][2] - wx[v][2], ub[v][3] - wx[v][3]));
@@ -971,16 +993,18 @@ __device__ __forceinline__ void state_loop(StateSharedT<NV, OW>& sh, const State
         split2(u[2], u[3], h23, l23);
         *reinterpret_cast<uint2*>(&sh.UhT[v * VB + j][t0]) = make_uint2(h01, h23);
         *reinterpret_cast<uint2*>(&sh.UlT[v * VB + j][t0]) = make_uint2(l01, l23);
-        wx[v] = x;
-        if constexpr (!OW) put_u(v);
-      } else {
-        // Q' S^T (P U added, and the outputs stored, after the state update is issued)
-#pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) ov[v][i4] = x[i4];
-        if constexpr (OW) sh.OV[v * 4 + tb][l] = f32x4{ov[v][0], ov[v][1], ov[v][2], ov[v][3]};
+      } else if constexpr (OW) {
+        sh.OV[v * 4 + tb][l] = x;
       }
+      wx[v] = x;
     }
     fetch2(wn, nxt);
+    if constexpr (!URole && !OW) {
+      if constexpr (!decltype(first)::value) add_pu(nxt);  // (nxt.X: the chunk before's P until fetch2x)
+#pragma unroll
+      for (int v = 0; v < NV; ++v) ov[v] = wx[v];
+    }
+    fetch2x(wn, nxt);
     lds_barrier();
     // (the next chunk's K^T fragments are not needed before the next update: issued past the barrier, so that
     // their issue is off the barrier's path; 71.8-71.9 against 73.7-73.9 us at T = 4096, 16 heads)
@@ -997,19 +1021,10 @@ __device__ __forceinline__ void state_loop(StateSharedT<NV, OW>& sh, const State
       acc1 = mfma(frag(&sh.UlT[v * VB][0], LDC, 0, 32), cur.KT[1], acc1);
       S[v] = acc0 + acc1;
     }
-    if constexpr (URole && OW) {  // for the output waves, read after the next barrier: off this chunk's path
+    if constexpr (!URole && !OW && !decltype(first)::value) put_o(ci - 1);
+    if constexpr (URole) {  // for P U, read after the next barrier: off this chunk's path
 #pragma unroll
       for (int v = 0; v < NV; ++v) put_u(v);
-    }
-    if constexpr (!URole && !OW) {
-#pragma unroll
-      for (int v = 0; v < NV; ++v) {
-        f32x4 y = f32x4{ov[v][0], ov[v][1], ov[v][2], ov[v][3]};
-        y = mfma(__builtin_bit_cast(bf16x8, cur.X[0]), frag(&sh.UT[v * VB][0], LDC, 0, 0), y);
-        if (tb >= 2) y = mfma(__builtin_bit_cast(bf16x8, cur.X[1]), frag(&sh.UT[v * VB][0], LDC, 0, 32), y);
-        const float yo[4] = {y[0], y[1], y[2], y[3]};
-        store_o_tile(o, a, a.vb + v, ci, t0, j, yo);
-      }
     }
   };
 
@@ -1026,16 +1041,21 @@ __device__ __forceinline__ void state_loop(StateSharedT<NV, OW>& sh, const State
     const Rsrc w0 = chunk_ws(0);
     fetch1(w0, b0);
     fetch2(w0, b0);
+    fetch2x(w0, b0);
     fetch3(w0, b0);
   }
-  process(0, b0, min(1, last), b1);
+  process(0, b0, min(1, last), b1, std::true_type{});
   int ci = 1;
   for (; ci + 1 < a.nchunks; ci += 2) {
-    process(ci, b1, ci + 1, b0);
-    process(ci + 1, b0, min(ci + 2, last), b1);
+    process(ci, b1, ci + 1, b0, std::false_type{});
+    process(ci + 1, b0, min(ci + 2, last), b1, std::false_type{});
   }
-  if (ci < a.nchunks) process(ci, b1, ci, b0);
-  if constexpr (OW) lds_barrier();  // the last chunk's U, for the output waves
+  if (ci < a.nchunks) process(ci, b1, ci, b0, std::false_type{});
+  lds_barrier();  // the last chunk's U
+  if constexpr (!URole && !OW) {
+    add_pu(b0);  // (either buffer holds the last chunk's P by now)
+    put_o(last);
+  }
 }
 
 // The chunk loop of an output wave (waves 8-11 of a workgroup that has them): O = Q' S^T + P U of token
@@ -1112,7 +1132,8 @@ __device__ __forceinline__ void run_loop(StateSharedT<NV, OW>& sh, const StateAr
 }
 // Waves of a state workgroup: output waves where each has a CU to itself (one block; two-block workgroups share a CU
 // in twos, and 12 waves of their registers would not). One block, T = 4096 at 16 heads: 45.2 us with them, 45.8 with
-// the O role doing P U itself, 47.3 with the U role doing it a chunk late, 49.5 with the output waves taking Q' S^T too.
+// the O role doing P U itself behind its update, 47.3 with the U role doing it a chunk late, 49.5 with the output waves
+// taking Q' S^T too; with the O role doing it a chunk late, as two-block workgroups do, the call 73.9 against 73.1.
 template <int NV>
 constexpr bool state_ow() { return NV == 1; }
 template <int NV>
@@ -1802,16 +1823,14 @@ std::atomic<int> g_launch_form{launch_form_from_env()};
 std::atomic<int> g_spin_max{SPIN_MAX};
 std::atomic<int> g_never_ready{0};
 
-// Whether an eligible batch takes the overlapped launch: only when the launch form asks for it. With the
-// phase-1 item of this file the two launches measured faster on every shape tried (MI355X, bf16,
-// dk = dv = 128, HIP graph replay, us two launches / overlapped, both forms forced in one process):
-// 1 x 4096 at 16 heads 81.3 / 86.4, at 8 heads 57.3 / 57.7; 2 x 4096 139.6 / 168.0; 1 x 2048 47.2 / 56.3;
-// 4 x 1024 63.9 / 81.7; packed 32 x 512, 16 x 1024, 8 x 2048 310.2 / 347.3, 303.6 / 312.7, 302.6 / 311.8;
-// 32 packed sequences of 64 .. 2048 tokens 730.0 / 747.7. (The overlapped launch won where phase 1 was slower:
-// with an item of 10-11k VALU instructions it took the 4096-token, 16-head prefill in 78-81 us against 83 us,
-// and the 32-sequence packed batch in 548-559 against 624-634 us.) The overlapped state jobs share their CUs
-// with phase-1 workgroups, which slows their chunk steps by a third, and the faster phase 1 leaves less of its
-// time to hide.
+// Whether an eligible batch takes the overlapped launch: only when the launch form asks for it. The two launches are
+// faster on every shape tried (MI355X, bf16, dk = dv = 128, 16 heads, HIP graph replay, us two launches / overlapped,
+// both forms in one process): 1 x 2048 42.8 / 52.8, 1 x 4096 72.9 / 79.3, 1 x 8192 147.0 / 149.1; 2 x 2048 54.8 /
+// 73.5, 2 x 4096 109.7 / 143.8; 4 x 1024 50.6 / 74.1, 8 x 1024 97.8 / 138.3; packed 32 x 512, 16 x 1024, 8 x 2048
+// 229.9 / 324.1, 228.2 / 299.5, 227.1 / 303.2; 32 packed sequences of 64 .. 2048 tokens 441 / 569. The overlapped
+// state jobs share their CUs with phase-1 workgroups, which slows their chunk steps by a third, and phase 1 is too
+// short for what hiding it gains. (With an item of 10-11k VALU instructions the overlapped launch took the 4096-token,
+// 16-head prefill in 78-81 us against 83 us, and a 32-sequence packed batch in 548-559 against 624-634 us.)
 bool overlap_wanted() { return g_launch_form.load(std::memory_order_relaxed) == 1; }
 
 // Queues of the overlapped launch: one per XCD (their L2s are not coherent with each other), or 0 when the
