@@ -4,6 +4,7 @@ arguments with a status and a message before touching the device."""
 from __future__ import annotations
 
 import ctypes
+import importlib
 import re
 from pathlib import Path
 
@@ -242,3 +243,38 @@ def test_launch_form_reads_the_environment_once_at_load():
                          timeout=300)
     assert out.returncode == 0, out.stderr
     assert out.stdout.split() == ["0", "0"]
+
+
+def test_internal_entry_points_refuse_bad_arguments(gdn):
+    """The entry points of the serving layer's own calls refuse what their kernels do not take before any launch."""
+    native = importlib.import_module("zonos3-mini_amd._native")
+    p = ctypes.c_void_p(1 << 20)  # never read: every call below is refused
+    odd = ctypes.c_void_p((1 << 20) + 8)
+
+    def refused(name, args, match, **over):
+        with pytest.raises(RuntimeError, match=match):
+            native.call(name, *{**args, **over}.values())
+
+    rows = dict(x=p, x_ld=256, w=p, y=p, y_ld=64, M=4, N=64, K=256, dtype=native.BF16, stream=None)
+    for over, match in ((dict(dtype=native.F32), "bf16 only"), (dict(K=192), "K=192"), (dict(N=60), "N=60"),
+                        (dict(M=-1), "bad sizes"), (dict(x=None), "null pointer"), (dict(w=odd), "16-byte"),
+                        (dict(x_ld=128), "row strides"), (dict(y_ld=56), "row strides"), (dict(M=2**23, x_ld=2**10), "4 GiB")):
+        refused("zgdn_gemm_rows", rows, match, **over)
+    gather = dict(x=p, window=p, hidden=256, dtype=native.BF16, tables=p, n_runs=2, n_chunks=3, rows=100, new_rows=60,
+                  n_slots=4, out=p, stream=None)
+    for over, match in ((dict(tables=None), "null pointer"), (dict(n_runs=0), "bad sizes"), (dict(new_rows=101), "bad sizes"),
+                        (dict(new_rows=0), "bad sizes"), (dict(window=None), "null pointer"), (dict(hidden=252), "multiple of 8"),
+                        (dict(dtype=native.F32), "bf16 rows"), (dict(out=odd), "16-byte")):
+        refused("zgdn_serving_gather", gather, match, **over)
+    size = native.lib().zgdn_serving_extend_workspace
+    assert size(0, 10, 4) == size(2, 0, 4) == size(2, 10, 0) == 0 < size(3, 100, 4) < size(3, 100, 8)
+    extend = dict(mixed=p, mixed_ld=2056, x=p, hidden=256, dtype=native.BF16, tables=p, n_runs=2, n_chunks=3, rows=100,
+                  new_rows=60, n_slots=4, H=4, conv_weight=p, A_log=p, dt_bias=p, norm_weight=p, conv_commit=p,
+                  conv_live=p, state_commit=p, state_live=p, window=p, win_len=p, gated=p, eps=1e-5, scale=1.0,
+                  workspace=p, bytes=size(3, 100, 4), stream=None)
+    for over, match in ((dict(n_chunks=0), "bad sizes"), (dict(n_slots=0), "bad sizes"), (dict(win_len=None), "null pointer"),
+                        (dict(H=3), "1, 2, 4, 8 or 16 heads"), (dict(H=32), "1, 2, 4, 8 or 16 heads"),
+                        (dict(hidden=12), "multiple of 8"), (dict(dtype=native.F32), "bf16"),
+                        (dict(mixed_ld=2048), "in_proj rows"), (dict(mixed_ld=2060), "in_proj rows"),
+                        (dict(conv_live=odd), "16-byte"), (dict(bytes=size(3, 100, 4) - 1), "workspace")):
+        refused("zgdn_serving_extend", extend, match, **over)

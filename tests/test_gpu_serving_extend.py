@@ -105,3 +105,64 @@ def test_a_call_of_no_requests_returns_no_rows(gdn, cuda):
         torch.cuda.synchronize()
         assert y.shape == (0, 256) and y.dtype == torch.bfloat16
         assert bool((layer._window == 0.25).all()) and not layer._win_len.any() and layer._owners == [None] * 3
+
+
+@pytest.mark.parametrize("H", [1, 2, 8, 16])
+def test_head_counts_of_the_entry(gdn, cuda, H):
+    """``ops.serving_extend`` at the head counts that the four-head layer does not pass: fresh runs, runs behind
+    replayed rows and a run of complete chunks alone, against the package's own operators run by run, to the bit."""
+    ops, serving = gdn.ops, importlib.import_module("zonos3-mini_amd.serving")
+    announce(f"serving_extend at {H} heads")
+    gen = torch.Generator().manual_seed(5500 + H)
+    bf, hidden, cap, inner = torch.bfloat16, 128, 6, 128 * H
+    C, width = 3 * inner, (514 * H + 7) // 8 * 8  # q|k|v, z, a, b and columns up to whole 16-byte pieces
+    r = lambda *s, std=1.0: (std * torch.randn(*s, generator=gen)).to(cuda)
+    in_proj, conv_w, norm_w = r(width, hidden, std=0.05).to(bf), r(C, 4, std=0.2).to(bf), (1 + r(128, std=0.1)).to(bf)
+    A_log, dt_bias = r(H, std=0.2), r(H, std=0.2)
+    conv_c, state_c, window = r(cap, C, 4).to(bf), r(cap, H, 128, 128, std=0.02), r(cap, 64, hidden).to(bf)
+    conv_l, state_l, win_len = torch.zeros_like(conv_c), torch.zeros_like(state_c), torch.full((cap,), 9, dtype=torch.int32, device=cuda)
+    reqs = [serving.Request(slot=s, owner=(s, False), cached=c, new=n)
+            for s, c, n in ((3, 0, 70), (0, 74, 60), (5, 64, 128), (1, 5, 2))]
+    new = sum(q.new for q in reqs)
+    x = r(new, hidden).to(bf)
+    flat, rows, n_chunks = serving.run_tables(reqs)
+    # the operators, run by run, from the same rows through the same projection
+    parts, at = [], 0
+    for q in reqs:
+        parts += [window[q.slot, :q.replay], x[at:at + q.new]]
+        at += q.new
+    mixed = torch.nn.functional.linear(torch.cat(parts), in_proj)
+
+    def run(lo, n, slot, fresh):
+        m = mixed[lo:lo + n].unsqueeze(0)
+        h0, s0 = (torch.zeros_like(t[slot:slot + 1]) if fresh else t[slot:slot + 1].clone() for t in (conv_c, state_c))
+        cu = torch.tensor([0, n], dtype=torch.int32, device=cuda)
+        y, h = ops.causal_conv1d(m[..., :C], conv_w, initial_state=h0, activation="silu", cu_seqlens=cu, state_width=4)
+        q, k, v = (t.unflatten(-1, (H, 128)) for t in y.split(inner, dim=-1))
+        o, s = ops.chunk_fwd(ops.l2norm(q[0])[0].unsqueeze(0), ops.l2norm(k[0])[0].unsqueeze(0), v,
+                             m[..., 4 * inner:4 * inner + H], m[..., 4 * inner + H:4 * inner + 2 * H], beta_is_logit=True,
+                             scale=128**-0.5, initial_state=s0, cu_seqlens=cu, A_log=A_log, dt_bias=dt_bias)
+        z = m[0, :, C:C + inner].unflatten(-1, (H, 128))
+        return ops.gated_rmsnorm(o[0], z, norm_w, eps=1e-5)[0].reshape(n, inner), h[0], s[0]
+
+    want = dict(conv_c=conv_c.clone(), state_c=state_c.clone(), conv_l=conv_l.clone(), state_l=state_l.clone(),
+                window=window.clone(), win_len=win_len.clone())
+    outs, lo, at = [], 0, 0
+    for q in reqs:
+        n, fresh = q.replay + q.new, q.cached == 0
+        whole = n - n % 64
+        y, want["conv_l"][q.slot], want["state_l"][q.slot] = run(lo, n, q.slot, fresh)
+        outs.append(y[q.replay:])
+        if whole:
+            _, want["conv_c"][q.slot], want["state_c"][q.slot] = run(lo, whole, q.slot, fresh)
+        joined = torch.cat((window[q.slot, :q.replay], x[at:at + q.new]))
+        want["window"][q.slot, :n - whole] = joined[whole:]
+        want["win_len"][q.slot] = n - whole
+        lo, at = lo + n, at + q.new
+    gated = ops.serving_extend(x, in_proj, conv_w, A_log, dt_bias, norm_w, conv_c, conv_l, state_c, state_l, window,
+                               win_len, torch.tensor(flat, dtype=torch.int32, device=cuda), len(reqs), n_chunks, rows, H,
+                               1e-5, 128**-0.5)
+    torch.cuda.synchronize()
+    assert torch.equal(gated, torch.cat(outs))
+    for name, t in dict(conv_c=conv_c, state_c=state_c, conv_l=conv_l, state_l=state_l, window=window, win_len=win_len).items():
+        assert torch.equal(t, want[name]), name
