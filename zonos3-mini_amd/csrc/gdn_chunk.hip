@@ -61,7 +61,6 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t&
 }
 
 constexpr int LDC = CH + 8;  // padded LDS row (bf16) of a 64-wide matrix
-constexpr int LDF = CH + 4;  // padded LDS row (fp32) of a 64-wide matrix
 
 // Workspace of one chunk x head (bytes), every block in the register order of the phase-2 wave that reads it.
 // Token tile tb = 16 tokens, value block vb = 16 value rows, k-step kk = 32 keys; lane l:
@@ -192,9 +191,8 @@ __device__ __forceinline__ uint2 lds_tr(const uint8_t* base, int off) {
 // Per-lane LDS offsets, formed once per workgroup (lane l, m = l % 16, g = l / 16).
 struct PrepLane {
   int f16[4];    // row fragment (rows r0 + m, k = 32 kk + 8 g ..) of a 256-byte-row matrix: + 256 r0
-  int f8[2];     // the same for 128-byte rows: + 128 r0
   int t16, t16h;  // transposing-read fragment of a 256-byte-row matrix: (t ^ 2 r0) + 8192 kk
-  int t8, t8h;   // the same for 128-byte rows: (t ^ 2 r0) + 4096 kk
+  int t8, t8h;   // the same of a 128-byte-row matrix: (t ^ 2 r0) + 4096 kk
   int w32;       // transposed D-tile store, fp32 256-byte rows: (w32 ^ 64 ri) + 4096 rj
   int w16;       // transposed D-tile store, bf16 128-byte rows: (w16 ^ 32 ri) + 2048 rj
   int rA, rB;    // fp32 block operands of the 16x16x4 products (see mm_t)
@@ -203,8 +201,6 @@ struct PrepLane {
     const int m = l & 15, g = l >> 4, s = m;
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) f16[kk] = m * 256 + (((4 * kk + g) ^ m) << 4);
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) f8[kk] = m * 128 + (((4 * kk + g) ^ (m >> 1)) << 4);
     const int y16 = 8 * (g & 1) + (s >> 2);
     t16 = (8 * g + (s >> 2)) * 256 + ((((s & 3) >> 1) ^ y16) << 4) + 8 * (s & 1);
     t16h = (t16 + 1024) ^ 64;
@@ -222,9 +218,6 @@ struct PrepLane {
 // Row fragment (rows r0 + lane%16, k-step kk) of a row-major swizzled matrix at byte `mat`.
 __device__ __forceinline__ bf16x8 pfrag16(const uint8_t* lb, int mat, int r0, int kk, const PrepLane& L) {
   return lds_at<bf16x8>(lb, mat + 256 * r0 + L.f16[kk]);
-}
-__device__ __forceinline__ bf16x8 pfrag8(const uint8_t* lb, int mat, int r0, int kk, const PrepLane& L) {
-  return lds_at<bf16x8>(lb, mat + 128 * r0 + L.f8[kk]);
 }
 // Row fragment of M (rows r0 + lane%16 of M, k-step kk) read from M^T stored row-major (transposing reads):
 // 256-byte rows of M^T (M^T has 64 rows: k up to 64, columns up to 128) and 128-byte rows (64 columns).
@@ -398,7 +391,7 @@ __device__ __forceinline__ void prep_item(uint8_t* lb, const ItemAt& it, RowRegs
   PrepLane L = L0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(L.f16[i]));
-  asm volatile("" : "+v"(L.f8[0]), "+v"(L.f8[1]), "+v"(L.t16), "+v"(L.t16h), "+v"(L.t8), "+v"(L.t8h));
+  asm volatile("" : "+v"(L.t16), "+v"(L.t16h), "+v"(L.t8), "+v"(L.t8h));
   asm volatile("" : "+v"(L.w32), "+v"(L.w16), "+v"(L.rA), "+v"(L.rB), "+v"(L.dv), "+v"(rowoff));
   int tid = threadIdx.x;  // (opaque per item as well, for the values derived from it)
   asm volatile("" : "+v"(tid));
@@ -1767,8 +1760,9 @@ __global__ __launch_bounds__(256) void chunk_correct_kernel(const uint16_t* __re
 // MI355X, one sequence (graph replay, hundredths of a microsecond): the plain pass 66 a chunk; a segmented one 104 a
 // chunk of a segment (the correction's rows among them; segments below 10 chunks take as long as 10), 217 a combine
 // step and 270 fixed. A segment count in 2 .. 8 is taken when its local and transition workgroups all fit one per CU
-// and it is the cheapest, for more than 32 chunks: up to there callers count on no extra workspace, and segments gain
-// 2.4 us at most. The call at 4 heads, plain / segmented, us: T = 1536 28.2 / 31.0, 1792 31.2 / 30.6, 2048 34.2 / 31.8,
+// and it is the cheapest, for more than 32 chunks: calls of up to 2048 tokens keep the plain pass and its workspace,
+// though the longest of them would gain (2048 tokens: 1 head 32.8 / 28.9, 4 heads 34.2 / 31.8). The call at 4 heads,
+// plain / segmented, us: T = 1536 28.2 / 31.0, 1792 31.2 / 30.6, 2048 34.2 / 31.8,
 // 2304 36.7 / 33.0, 4096 53.8 / 37.2, 8192 96.4 / 54.2; 8 heads: 2304 37.9 / 37.1, 2560 40.7 / 38.4, 3072 46.2 / 41.4,
 // 4096 57.5 / 48.3; 1 head, 4 / 5 segments: 2560 29.9 / 30.8. (With 64 a chunk, 80 a chunk of a
 // segment, 207 and 985, measured on an earlier state pass, 4 heads went over from 2432 tokens and 8 heads from 3200.)
