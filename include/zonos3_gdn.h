@@ -125,7 +125,8 @@ int zgdn_chunk_set_wait_limit(int spins, int never_ready);
  * Extra workspace bytes (after zgdn_chunk_workspace_size's) with which zgdn_chunk_fwd runs an unpacked batch of
  * B sequences of T tokens as segments, 0 when it would not. When the sequential state pass would hold at most
  * half the current device's CUs (few sequences and heads) and the sequences are long enough for it to pay
- * (about 48 chunks at one sequence of 4 heads), each sequence is cut into 2 .. 8 segments run at once -- from
+ * (more than 32 chunks: from 33 at one sequence of up to 4 heads, 36 at 8 heads; prompts of up to 2048 tokens need
+ * no extra workspace), each sequence is cut into 2 .. 8 segments run at once -- from
  * zero states, and from the identity to obtain each segment's state map -- and their outputs and states are
  * combined (the same results up to rounding). A smaller workspace runs the plain pass.
  */

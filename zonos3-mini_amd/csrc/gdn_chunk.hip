@@ -15,8 +15,8 @@
 // registers: one MFMA pass over [W; Q'] gives U and the outputs' state part, a second the state update and P U.
 // (With the outputs' parts that need no state formed ahead, P Ub and P W: 112 more products and two more phases an
 // item, 10 KiB more written and read, for 2 products a chunk less in the state pass. T = 4096 at 16 heads: phase 1
-// 29.7 us against 25.7, the state pass 41.8 against 43.9; 32 packed sequences of 30,526 tokens at 16 heads 217 and 263
-// us against 200 and 254.) Only the state pass is sequential, so the workspace is
+// 29.4 us against 25.7, the state pass 41.4 against 43.7; 32 packed sequences of 30,526 tokens at 16 heads 220 and 258
+// us against 203 and 259.) Only the state pass is sequential, so the workspace is
 // stored in MFMA fragment order: every phase-2 operand load is one contiguous 1 KiB per wave (rows read
 // straight from row-major matrices cost about 2.3x as much per byte on CDNA), and the next chunk's loads are
 // issued in three groups spread over the current chunk so they overlap its MFMA and LDS work.
@@ -1124,9 +1124,9 @@ __device__ __forceinline__ void run_loop(StateSharedT<NV, OW>& sh, const StateAr
     out_loop<TOut, NV>(sh, a, o);
 }
 // Waves of a state workgroup: output waves where each has a CU to itself (one block; two-block workgroups share a CU
-// in twos, and 12 waves of their registers would not). One block, T = 4096 at 16 heads: 45.2 us with them, 45.8 with
-// the O role doing P U itself behind its update, 47.3 with the U role doing it a chunk late, 49.5 with the output waves
-// taking Q' S^T too; with the O role doing it a chunk late, as two-block workgroups do, the call 73.9 against 73.1.
+// in twos, and 12 waves of their registers would not). One block, T = 4096 at 16 heads, the kernel trace of 200 calls,
+// two runs each: 44.0 and 44.7 us with them, 45.1 and 45.4 with the O role doing P U itself behind its update, 44.8 and
+// 45.4 with the O role doing it a chunk late, as two-block workgroups do.
 template <int NV>
 constexpr bool state_ow() { return NV == 1; }
 template <int NV>

@@ -419,7 +419,7 @@ __global__ __launch_bounds__(256) void gated_rmsnorm_kernel(const T* __restrict_
 // request's joined run -- its slot's unfinished chunk, then its new rows -- as one packed sequence, reading and
 // writing the slots' caches in place. The kernels below are its row-local parts; each workgroup finds its rows
 // from the run tables (a few dozen integers), so the host lists no rows. Six requests, 1,067 new rows, hidden 1024:
-// 107 us a call, 65 us of it kernels (two GEMMs 25, phase 1 12, state pass 8, conv 6, norm and gather 4.6 each);
+// 102 us a call, 61 us of it kernels (two GEMMs 26.0, phase 1 10.6, state pass 9.5, conv 6.3, gather 4.5, norm 4.1);
 // through index lists of every row, two passes and some 45 launches of index_select / index_copy / index_fill and
 // the operators 1,074-1,127 us, nearly all of it the host.
 

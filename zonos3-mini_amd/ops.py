@@ -261,7 +261,8 @@ def decode_step(q, k, v, g, beta, state, scale=None):
     dt, gdt, idx = q.dtype, g.dtype, q.get_device()
     (B, Hk, K), (Bv, Hv, V) = q.shape, v.shape
     if (idx >= 0 and isinstance(state, torch.Tensor) and Bv == B and Hk and Hv % Hk == 0 and dt in _CODES
-            and gdt in _CODES and k.shape == q.shape and k.dtype is dt and v.dtype is dt and beta.dtype is gdt and g.shape == beta.shape == (B, Hv)
+            and gdt in _CODES and k.shape == q.shape and k.dtype is dt and v.dtype is dt and beta.dtype is gdt
+            and g.shape == beta.shape == (B, Hv)
             and state.dtype is torch.float32 and state.shape == (B, Hv, V, K)
             and k.get_device() == v.get_device() == g.get_device() == beta.get_device() == state.get_device() == idx
             and q.is_contiguous() and k.is_contiguous() and v.is_contiguous() and g.is_contiguous()

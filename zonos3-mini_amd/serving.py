@@ -14,11 +14,11 @@ Design of this module.
 - Eager prefills and extends of a bf16 layer on this package's own operators run each request's joined run (its
   unfinished chunk, then its new rows) as one packed sequence, the kernels reading and writing the slots' caches in
   place from a few numbers a request (``_extend_in_place``).
-- Other eager calls (accent adapters, rebound operators, fp32) are planned on the host first (``plan_extend``): every request's replayed window rows and
-  new rows form one joined run, cut after its last complete chunk; the complete part goes to a committed
-  pass, the rest to an open pass. The plan is a set of index lists (source rows, output rows, window rows)
-  uploaded in one pinned copy; the device work is then one gather per pass, the packed pass itself and one
-  scatter of the outputs, whatever the number of requests.
+- Other eager calls (accent adapters, rebound operators, fp32) are planned on the host first (``plan_extend``): every
+  request's replayed window rows and new rows form one joined run, cut after its last complete chunk; the
+  complete part goes to a committed pass, the rest to an open pass. The plan is a set of index lists (source
+  rows, output rows, window rows) uploaded in one pinned copy; the device work is then one gather per pass, the
+  packed pass itself and one scatter of the outputs, whatever the number of requests.
 - ``_pass`` is the one place a packed pass touches the caches: it runs ``_run_packed`` from the slots'
   committed states and stores the final states as live (and as committed for a committed pass). The eager
   and static prefill paths both use it.
@@ -241,8 +241,9 @@ def _takes_few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
     subclass, which may hold its elements in another form, and a product that autograd records stay F.linear's."""
     plain = (torch.Tensor, torch.nn.Parameter)
     return (x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2
-            and x.shape[0] <= _few_rows_limit(*w.shape) and type(x) in plain and type(w) in plain and x.is_contiguous() and w.is_contiguous()
-            and x.shape[1] == w.shape[1] and w.shape[1] % 128 == 0 and w.shape[0] % 8 == 0 and w.device == x.device
+            and x.shape[0] <= _few_rows_limit(*w.shape) and type(x) in plain and type(w) in plain
+            and x.is_contiguous() and w.is_contiguous() and x.shape[1] == w.shape[1] and w.shape[1] % 128 == 0
+            and w.shape[0] % 8 == 0 and w.device == x.device
             and not (x.data_ptr() | w.data_ptr()) % 16
             and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
 
