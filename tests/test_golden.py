@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 import torch
 
-from gdn_testing import announce, max_abs, rel_err
+from gdn_testing import OUT_RMS, OUT_ROW, announce, max_abs, out_errs, rel_err
 from oracle import gdn_oracle as O
 
 GOLDEN = Path(__file__).resolve().parent / "golden"
@@ -74,6 +74,8 @@ def test_kernels_reproduce_fixtures(gdn, cuda):
     o, s = gdn.chunk_fwd(d["q"].to(bf), d["k"].to(bf), d["v"].to(bf), d["g"], d["beta"], initial_state=d["s0"],
                          cu_seqlens=d["cu"], chunk_indices=d["chunks"])
     assert max_abs(o.cpu(), f["o"]) < 2e-2 and rel_err(s.cpu(), f["s"]) < 1e-3
+    rms, row = out_errs(o, f["o"], f["cu"].tolist())
+    assert rms < OUT_RMS and row < OUT_ROW, (rms, row)
     f = _load("conv_varlen_D16")
     d = {k: v.to(cuda) for k, v in f.items()}
     st = d["s0"].clone()
